@@ -1,0 +1,46 @@
+"""The routes a team stage picks by size and alignment, each at the sizes
+where it can go wrong (edges of tiles, remainders, planes that start inside a
+line), against the oracle or against an independent computation."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _unit(tmp_path, kernels, mode="float64"):
+    import hawk_amd as hawk
+    hawk.build(kernels, tmp_path, mode=mode)
+    return [hawk.load(tmp_path, k.name) for k in kernels]
+
+
+def _plane(a, gpu, shift=0):
+    """``a`` on the device, its first element ``shift`` elements past an allocation's start."""
+    import torch
+    flat = torch.from_numpy(np.ascontiguousarray(a)).reshape(-1)
+    held = torch.empty(flat.numel() + shift, dtype=flat.dtype, device=gpu)
+    held[shift:] = flat.to(gpu)
+    return held[shift:].view(a.shape)
+
+
+@pytest.mark.parametrize("mode", ["float32", "float64"])
+@pytest.mark.parametrize("n, shift", [(32, 0), (64, 0), (64, 1), (4128, 0), (4128, 3), (4127, 0), (100, 0)])
+def test_mm16_streamed_and_cached(tmp_path, gpu, mode, n, shift):
+    """Whole-line planes stream, others (a row that is no multiple of 128
+    bytes, a plane starting inside a line) go through the cache.  On small
+    integers every partial sum is exact, so both give the exact product."""
+    from hawk_amd import examples as E
+    import hawk_amd as hawk
+    dt = np.float32 if mode == "float32" else np.float64
+    g = np.random.default_rng(n + shift)
+    A, B, C = (g.integers(-8, 9, size=(16, 16, n)).astype(dt) for _ in range(3))
+    fwd, vjp = _unit(tmp_path, [E.mm16, E.mm16_vjp], mode)
+    zero = np.zeros((16, 16, n), dt)
+    got, bar_A, bar_B = (_plane(zero, gpu, shift) for _ in range(3))
+    a, b, c = (_plane(x, gpu, shift) for x in (A, B, C))
+    hawk.run(fwd, A=a, B=b, C=got, layout="samples_last")
+    hawk.run(vjp, A=a, B=b, bar_C=c, bar_A=bar_A, bar_B=bar_B, layout="samples_last")
+    for x, (X, Y) in ((got, (A, B)), (bar_A, (C, B.transpose(1, 0, 2))), (bar_B, (A.transpose(1, 0, 2), C))):
+        assert np.array_equal(x.cpu().numpy(), np.einsum("ikn,kjn->ijn", X, Y))
