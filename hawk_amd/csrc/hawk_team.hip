@@ -862,31 +862,16 @@ __global__ __launch_bounds__(256) void hawk_keyed_small(const T* __restrict__ u,
 //
 // parts[b][k] is the in-lane-order sum (from +0.0) of chunk b's values with
 // key k; cell k then adds parts[0][k], parts[1][k], ... in chunk order from
-// +0.0 and adds that onto target[k].  Up to 65536 cells the split walk below
-// makes those additions.  Past that, one 1024-thread workgroup walks one chunk
-// in tiles of 4096 lanes: each tile is sorted stably by key in LDS (LSD radix,
-// 8-bit digits), so every key's lanes form one run in lane order, and the
-// run's owner thread adds them one by one onto the key's accumulator — the
-// additions the serial walk makes, in its order.  Accumulators of keys below
-// kAccKeys live in LDS, the others in the zero-filled parts[b] (only this
-// workgroup touches that row).
+// +0.0 and adds that onto target[k].  Two walks make those additions, the
+// split walk (a workgroup a chunk) and the wide walk (a workgroup a chunk and
+// key range, for few chunks or many cells); in both every accumulator is in
+// LDS while its chunk is walked.
 // ---------------------------------------------------------------------------
 constexpr int kScatterChunks = 256;    // reference hawk/_lane_bind.py:108
 constexpr int kWalkThreads = 1024;
 constexpr int kWalkWaves = kWalkThreads / 64;
 constexpr int kWalkItems = 4;                      // lanes per thread per tile
 constexpr int kTile = kWalkThreads * kWalkItems;   // 4096 lanes per tile
-constexpr int kPosBits = 12;                       // 2^12 == kTile
-constexpr unsigned kPosMask = (1u << kPosBits) - 1u;
-constexpr unsigned kInvalid = 0x80000000u;         // a skipped (-1), bad or padding lane
-constexpr int kMaxKeyBits = 31 - kPosBits;         // key field: bits 12..30
-constexpr int kDigitBits = 8;
-constexpr int kDigits = 1 << kDigitBits;
-constexpr int kHistRow = kWalkWaves + 1;          // one digit's per-wave counts, padded: rows in different banks
-constexpr int kAccKeys = 4096;                     // keys whose accumulators live in LDS
-constexpr int kFoldUnroll = 8;
-
-static_assert(kTile == 1 << kPosBits, "tile positions fill the position field");
 
 // Inclusive scan over the 64 lanes of a wave in DPP moves, no LDS: within
 // each row of 16 lanes by row shifts 1, 2, 4, 8 (a lane past the row's start
@@ -900,90 +885,6 @@ __device__ __forceinline__ unsigned wave_inclusive_scan(unsigned x) {
     x += __builtin_amdgcn_update_dpp(0u, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1, 3
     x += __builtin_amdgcn_update_dpp(0u, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2, 3
     return x;
-}
-
-template <class T>
-struct WalkShared {
-    T vals[kTile];                               // 32 KiB: the tile's values, lane order
-    unsigned ent[2][kTile];                           // 32 KiB: (key << 12) | position | invalid
-    unsigned hist[kDigits][kHistRow];                 // 17 KiB: [digit][wave] counts, then offsets
-    union {
-        unsigned long long peer[kWalkWaves][kDigits]; // 32 KiB: per-wave lane masks of one digit (sort)
-        T sv[kTile];                             //         the tile's values in sorted order (fold)
-    };
-    T acc[kAccKeys];                             // 32 KiB: accumulators of keys < kAccKeys
-    unsigned long long starts[kTile / 64];            // run heads of the sorted tile
-    unsigned wsum[kWalkWaves];
-};
-
-// Stable LSD radix sort of the tile's entries by the key field (bits
-// 12..12+key_bits), 8 bits a pass, ping-ponging ent[0] <-> ent[1]; returns the
-// buffer holding the result.  Wave w ranks its 256 entries w*256 + j*64 + lane
-// window by window (j = 0..3, in order): the lanes of a window holding digit d
-// find each other through one LDS OR into peer[w][d]; the lowest of them adds
-// the group's size onto hist[d][w] after all of them read it.  The exclusive
-// scan of hist in (digit, wave) order then places every wave's group after
-// the earlier waves' groups of the same digit, so each pass keeps input order
-// within a digit.
-template <class T>
-__device__ int walk_sort(WalkShared<T>& sh, int key_bits) {
-    const int t = threadIdx.x;
-    const int wave = t >> 6;
-    const int lane = t & 63;
-    const unsigned long long me = 1ull << lane;
-    int src = 0;
-    for (int lo = 0; lo < key_bits; lo += kDigitBits) {
-        const int width = key_bits - lo < kDigitBits ? key_bits - lo : kDigitBits;
-        const unsigned dmask = (1u << width) - 1u;
-        const int shift = kPosBits + lo;
-        const unsigned* in = sh.ent[src];
-        unsigned* out = sh.ent[src ^ 1];
-        for (int d = lane; d < kDigits; d += 64) sh.hist[d][wave] = 0u;
-        __builtin_amdgcn_wave_barrier();
-        unsigned item[kWalkItems], digit[kWalkItems], rank[kWalkItems];
-#pragma unroll
-        for (int j = 0; j < kWalkItems; ++j) item[j] = in[wave * (kWalkItems * 64) + j * 64 + lane];
-#pragma unroll
-        for (int j = 0; j < kWalkItems; ++j) {
-            digit[j] = (item[j] >> shift) & dmask;
-            atomicOr(&sh.peer[wave][digit[j]], me);
-            __builtin_amdgcn_wave_barrier();
-            const unsigned long long peers = sh.peer[wave][digit[j]];
-            const unsigned below = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(peers >> 32),
-                                                             __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(peers), 0u));
-            const unsigned old = sh.hist[digit[j]][wave];
-            rank[j] = old + below;
-            __builtin_amdgcn_wave_barrier();
-            if (below == 0u) {
-                sh.hist[digit[j]][wave] = old + static_cast<unsigned>(__popcll(peers));
-                sh.peer[wave][digit[j]] = 0ull;
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-        __syncthreads();
-        // Exclusive scan over f = digit*16 + wave: thread t owns f = 4t .. 4t+3.
-        const int d = t >> 2;
-        const int w0 = (t & 3) * 4;
-        const unsigned c0 = sh.hist[d][w0], c1 = sh.hist[d][w0 + 1];
-        const unsigned c2 = sh.hist[d][w0 + 2], c3 = sh.hist[d][w0 + 3];
-        const unsigned mine = c0 + c1 + c2 + c3;
-        const unsigned incl = wave_inclusive_scan(mine);
-        if (lane == 63) sh.wsum[wave] = incl;
-        __syncthreads();
-        unsigned before = 0u;
-        for (int w = 0; w < wave; ++w) before += sh.wsum[w];
-        const unsigned base = incl - mine + before;
-        sh.hist[d][w0] = base;
-        sh.hist[d][w0 + 1] = base + c0;
-        sh.hist[d][w0 + 2] = base + c0 + c1;
-        sh.hist[d][w0 + 3] = base + c0 + c1 + c2;
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < kWalkItems; ++j) out[sh.hist[digit[j]][wave] + rank[j]] = item[j];
-        __syncthreads();
-        src ^= 1;
-    }
-    return src;
 }
 
 // Lane base + wave*256 + j*64 + lane goes to thread slot j: every load
@@ -1003,195 +904,12 @@ __device__ __forceinline__ void walk_load(const int* __restrict__ key, const T* 
     }
 }
 
-// The first run head after position i of the sorted tile (kTile if none).
-template <class T>
-__device__ __forceinline__ int next_head(const WalkShared<T>& sh, int i) {
-    int wi = i >> 6;
-    const int bit = i & 63;
-    unsigned long long m = bit == 63 ? 0ull : (sh.starts[wi] & (~0ull << (bit + 1)));
-    while (m == 0ull && ++wi < kTile / 64) m = sh.starts[wi];
-    return m ? (wi << 6) + __builtin_ctzll(m) : kTile;
-}
-
-// a + x[s] + x[s+1] + ... + x[e-1], one addition at a time in that order; the
-// next eight values are in flight while the current eight are added.
-template <class T>
-__device__ __forceinline__ T fold_run(const T* x, int s, int e, T a) {
-    int m = s;
-    if (e - m >= 2 * kFoldUnroll) {
-        T cur[kFoldUnroll];
-#pragma unroll
-        for (int q = 0; q < kFoldUnroll; ++q) cur[q] = x[m + q];
-        m += kFoldUnroll;
-        for (; m + kFoldUnroll <= e; m += kFoldUnroll) {
-            T nxt[kFoldUnroll];
-#pragma unroll
-            for (int q = 0; q < kFoldUnroll; ++q) nxt[q] = x[m + q];
-#pragma unroll
-            for (int q = 0; q < kFoldUnroll; ++q) a = a + cur[q];
-#pragma unroll
-            for (int q = 0; q < kFoldUnroll; ++q) cur[q] = nxt[q];
-        }
-#pragma unroll
-        for (int q = 0; q < kFoldUnroll; ++q) a = a + cur[q];
-    }
-    for (; m < e; ++m) a = a + x[m];
-    return a;
-}
-
-// Accumulators outside LDS are read and written at agent scope, so a value
-// one thread stores in a tile is what another thread of the workgroup loads
-// after the tile's closing barrier.
-template <class T>
-__device__ __forceinline__ T acc_load(const T* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <class T>
-__device__ __forceinline__ void acc_store(T* p, T x) {
-    __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// One workgroup per chunk b: lanes [b*span, min((b+1)*span, n)); parts
-// arrives zero-filled.
-template <class T>
-__global__ __launch_bounds__(kWalkThreads) void hawk_scatter_walk(
-        const int* __restrict__ key, const T* __restrict__ v, long long n, long long cells, long long span,
-        int key_bits, T* __restrict__ parts, int* __restrict__ status) {
-    __shared__ WalkShared<T> sh;
-    const int t = threadIdx.x;
-    const int wave = t >> 6;
-    const int lane = t & 63;
-    const int b = blockIdx.x;
-    const long long lo = static_cast<long long>(b) * span;
-    const long long hi = lo + span < n ? lo + span : n;
-    const int acc_n = cells < kAccKeys ? static_cast<int>(cells) : kAccKeys;
-    const unsigned kmask = (1u << key_bits) - 1u;
-    const unsigned sentinel = kmask;          // the key field of an invalid lane
-    T* row = parts + static_cast<long long>(b) * cells;
-
-    for (int k = t; k < acc_n; k += kWalkThreads) sh.acc[k] = T(0);
-    bool bad = false;
-    int nk[kWalkItems];
-    T nv[kWalkItems];
-    if (lo < hi) walk_load(key, v, lo, hi, nk, nv);
-    __syncthreads();
-    for (long long base = lo; base < hi; base += kTile) {
-        int kk[kWalkItems];
-        T vv[kWalkItems];
-#pragma unroll
-        for (int j = 0; j < kWalkItems; ++j) { kk[j] = nk[j]; vv[j] = nv[j]; }
-        if (base + kTile < hi) walk_load(key, v, base + kTile, hi, nk, nv);
-#pragma unroll
-        for (int j = 0; j < kWalkItems; ++j) {
-            const unsigned p = static_cast<unsigned>(wave * (kWalkItems * 64) + j * 64 + lane);
-            const bool valid = kk[j] >= 0 && kk[j] < cells;
-            bad = bad || (kk[j] != -1 && !valid);
-            const unsigned field = valid ? static_cast<unsigned>(kk[j]) : sentinel;
-            sh.ent[0][p] = (field << kPosBits) | p | (valid ? 0u : kInvalid);
-            sh.vals[p] = vv[j];
-            // the previous tile's sorted values share LDS with the sort's peer
-            // masks, which must start at zero
-            (&sh.peer[0][0])[p] = 0ull;
-        }
-        __syncthreads();
-        const unsigned* sorted = sh.ent[walk_sort(sh, key_bits)];
-        // The values in sorted order (an invalid lane's as +0.0) and the run
-        // heads, one ballot per 64 entries.
-        bool head[kWalkItems];
-#pragma unroll
-        for (int j = 0; j < kWalkItems; ++j) {
-            const int i = j * kWalkThreads + t;
-            const unsigned e = sorted[i];
-            sh.sv[i] = (e & kInvalid) ? T(0) : sh.vals[e & kPosMask];
-            const unsigned k = (e >> kPosBits) & kmask;
-            head[j] = i == 0 || k != ((sorted[i - (i > 0)] >> kPosBits) & kmask);
-            const unsigned long long m = __ballot(head[j]);
-            if (lane == 0) sh.starts[(j * kWalkThreads + wave * 64) >> 6] = m;
-        }
-        __syncthreads();
-        // Every run's owner: its accumulator first (the loads of all its runs
-        // in flight together), then its lanes in order, then the store.
-        int rs[kWalkItems], re[kWalkItems];
-        unsigned rk[kWalkItems];
-        bool load[kWalkItems];
-#pragma unroll
-        for (int j = 0; j < kWalkItems; ++j) {
-            rs[j] = j * kWalkThreads + t;
-            rk[j] = (sorted[rs[j]] >> kPosBits) & kmask;
-            re[j] = 0;
-            load[j] = false;
-            if (!head[j] || rk[j] >= cells) continue;
-            re[j] = next_head(sh, rs[j]);
-            const unsigned k = rk[j];
-            load[j] = k >= static_cast<unsigned>(acc_n);
-        }
-        T ra[kWalkItems];
-#pragma unroll
-        for (int j = 0; j < kWalkItems; ++j) {
-            const unsigned k = rk[j] < static_cast<unsigned>(acc_n) ? rk[j] : 0u;
-            ra[j] = load[j] ? acc_load(row + rk[j])
-                            : (re[j] != 0 && rk[j] < static_cast<unsigned>(acc_n) ? sh.acc[k] : T(0));
-        }
-#pragma unroll 1
-        for (int j = 0; j < kWalkItems; ++j) {
-            if (re[j] == 0) continue;
-            const unsigned k = rk[j];
-            T a = ra[j];
-            bool any = true;
-            if (k == sentinel) {
-                // The one run that can hold invalid lanes: skip them.
-                any = false;
-                for (int m = rs[j]; m < re[j]; ++m) {
-                    if (sorted[m] & kInvalid) continue;
-                    a = a + sh.sv[m];
-                    any = true;
-                }
-            } else {
-                a = fold_run(sh.sv, rs[j], re[j], a);
-            }
-            if (!any) continue;
-            if (k < static_cast<unsigned>(acc_n)) sh.acc[k] = a;
-            else acc_store(row + k, a);
-        }
-        __syncthreads();
-    }
-    for (int k = t; k < acc_n; k += kWalkThreads) row[k] = sh.acc[k];
-    if (bad) status[1 + b] = 1;
-}
-
-// More keys than the sort's key field holds: one thread per chunk walks its
-// lanes in order onto the zero-filled parts[b] (the reference's serial walk).
-template <class T>
-__global__ __launch_bounds__(64) void hawk_scatter_serial(const int* __restrict__ key, const T* __restrict__ v,
-                                                          long long n, long long cells, long long span,
-                                                          T* __restrict__ parts, int* __restrict__ status) {
-    if (threadIdx.x != 0) return;
-    const int b = blockIdx.x;
-    const long long lo = static_cast<long long>(b) * span;
-    const long long hi = lo + span < n ? lo + span : n;
-    T* row = parts + static_cast<long long>(b) * cells;
-    bool bad = false;
-    for (long long i = lo; i < hi; ++i) {
-        const int k = key[i];
-        if (k == -1) continue;
-        if (k < 0 || k >= cells) { bad = true; continue; }
-        row[k] = row[k] + v[i];
-    }
-    if (bad) status[1 + b] = 1;
-}
-
-template <class T>
-__global__ __launch_bounds__(256) void hawk_fill_zero(T* __restrict__ p, long long count) {
-    for (long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; i < count;
-         i += static_cast<long long>(gridDim.x) * 256)
-        p[i] = T(0);
-}
-
 // Cell c adds its chunk partials in chunk order from +0.0, then onto the
 // target: target[c] += sum (reference hawk/emit/team.py:437-460).  Two blocks
 // of kAhead chunks are in flight while a third is added: 64 loads a thread,
 // since a grid of one thread per cell (65536 at the split walk's largest)
-// holds only a wave or two per SIMD to cover HBM's latency.
+// holds only a wave or two per SIMD to cover HBM's latency.  A short block
+// reads only the groups of 8 chunks it holds.
 template <class T>
 __global__ __launch_bounds__(256) void hawk_scatter_cells(const T* __restrict__ parts, long long cells,
                                                           int chunks, T* __restrict__ target) {
@@ -1200,12 +918,18 @@ __global__ __launch_bounds__(256) void hawk_scatter_cells(const T* __restrict__ 
     constexpr int kAhead = 32;
     auto fetch = [&](int b, T (&x)[kAhead]) {
 #pragma unroll
-        for (int q = 0; q < kAhead; ++q) {
-            // past the last chunk a partial reads as +0.0, which adds nothing
-            // to a sum that is never -0.0
-            const int bq = b + q < chunks ? b + q : chunks - 1;
-            const T p = parts[static_cast<long long>(bq) * cells + c];
-            x[q] = b + q < chunks ? p : T(0);
+        for (int q = 0; q < kAhead; ++q) x[q] = T(0);
+#pragma unroll
+        for (int q8 = 0; q8 < kAhead; q8 += 8) {
+            if (b + q8 >= chunks) break;                      // the whole grid
+#pragma unroll
+            for (int q = q8; q < q8 + 8; ++q) {
+                // past the last chunk a partial reads as +0.0, which adds
+                // nothing to a sum that is never -0.0
+                const int bq = b + q < chunks ? b + q : chunks - 1;
+                const T p = parts[static_cast<long long>(bq) * cells + c];
+                x[q] = b + q < chunks ? p : T(0);
+            }
         }
     };
     T x0[kAhead], x1[kAhead];
@@ -1226,16 +950,8 @@ __global__ __launch_bounds__(256) void hawk_scatter_cells(const T* __restrict__ 
     target[c] = target[c] + s;
 }
 
-__global__ void hawk_scatter_status(int* status, long long cells) {
-    const int t = threadIdx.x;
-    if (t == 0) status[0] = static_cast<int>(cells);
-    if (t < kScatterChunks) status[1 + t] = 0;
-}
-
 // ---- the split walk: the ordered scatter into at most 65536 cells ----------
-// The same additions as hawk_scatter_walk (each (chunk, key) sum in lane order
-// from +0.0), with every accumulator in LDS, so no partial is read back from
-// memory while a chunk is walked:
+// Each (chunk, key) sum in lane order from +0.0, every accumulator in LDS:
 //
 // * hawk_split_hot: one workgroup per chunk, keys [0, kSplitHot) in LDS.  Each
 //   tile of 4096 lanes is split stably into buckets in one pass: window keys
@@ -1267,30 +983,31 @@ constexpr int kHotStride = kSplitTailBase + kSplitMaxRanges + 3;   // 60: a wave
 constexpr int kTailClassBits = 3;                // hawk_split_tail's classes: key & 7
 constexpr int kTailClasses = 1 << kTailClassBits;
 constexpr int kTailStride = kSplitClassBase + kTailClasses + 8;   // 48
-constexpr int kTailKeys = kTailRange >> kTailClassBits;   // 768 keys a class
 constexpr int kTailWaves = kTailClasses;         // a wave per class
 constexpr int kTailThreads = 64 * kTailWaves;
 constexpr int kTailBatch = kTailThreads * kWalkItems;   // 2048 entries a batch
 
 static_assert(kSplitHot - kSplitHeads < (1 << 15), "hot_class_index is exact below 2^15");
-static_assert((kSplitHot - kSplitHeads) / 15 < 1024 && (kTailRange >> kTailClassBits) <= 1024,
-              "class matching covers a class index of ten bits");
+static_assert((kSplitHot - kSplitHeads) / 15 < 1024, "fold_class matches ten bits of hawk_split_hot's class index");
 static_assert(kHotStride >= kSplitTailBase + kSplitMaxRanges + 1, "bucket starts need one past the last bucket");
 static_assert(kTailStride >= kSplitClassBase + kTailClasses + 1, "bucket starts need one past the last bucket");
 static_assert(kSplitNone >= kHotStride && kSplitNone >= kTailStride, "the no-bucket code is outside the count rows");
 static_assert(kTailRange < (1 << 16), "bins hold window-local keys as u16");
 
 constexpr int kSplitPad = 72;                    // entries read (and ignored) past a run's end
-constexpr unsigned kPeerSlots = 128;             // a class fold's match slots: class-index bits 0..6
+constexpr unsigned kPeerSlots = 128;             // hawk_split_hot's match slots a wave: class-index bits 0..6
 constexpr int kHeadBlock = 8;                    // a head chain's reads in flight: four blocks of kHeadBlock
 static_assert(4 * kHeadBlock <= kSplitPad, "a head chain reads at most kSplitPad entries past its run");
 
 // A split walk workgroup's LDS: Waves waves, Window accumulators, count rows
-// of Stride buckets, and the split tile (Waves * 256 entries).
-template <class T, int Waves, int Window, int Stride>
+// of Stride buckets, and the split tile (Waves * 256 entries); Peers match
+// slots a wave for the folds.
+template <class T, int Waves, int Window, int Stride, unsigned Peers = kPeerSlots>
 struct SplitShared {
     static constexpr int kWaves = Waves;
     static constexpr int kStride = Stride;
+    static constexpr int kWindow = Window;
+    static constexpr unsigned kPeers = Peers;
     static constexpr int kSpan = Waves * 64 * kWalkItems;
     T acc[Window];                              // the window's accumulators
     T val[kSpan + kSplitPad];                   // the tile's values, bucket order
@@ -1298,7 +1015,7 @@ struct SplitShared {
     union {                                     // one phase at a time:
         unsigned long long win[Waves][Stride];                 // split: a match table per wave
         struct {
-            unsigned long long peer[Waves][kPeerSlots];        // fold: per-wave match masks
+            unsigned long long peer[Waves][Peers];             // fold: per-wave match masks
         } f;
     };
     unsigned cnt[Waves][Stride];                // bucket counts, a row per wave (lane b reads word b)
@@ -1306,9 +1023,9 @@ struct SplitShared {
 };
 template <class T>
 using HotShared = SplitShared<T, kWalkWaves, kSplitHot, kHotStride>;      // 157 KiB (float64)
-template <class T>
-using TailShared = SplitShared<T, kTailWaves, kTailRange, kTailStride>;   // 78 KiB (float64): two a CU
-static_assert(sizeof(TailShared<double>) <= 80 * 1024, "two tail workgroups share a CU's 160 KiB");
+template <class T, int Window>
+using TailShared = SplitShared<T, kTailWaves, Window, kTailStride, 64>;
+static_assert(sizeof(TailShared<double, kTailRange>) <= 80 * 1024, "two tail workgroups share a CU's 160 KiB");
 
 // The bucket of window-local key kl (0 <= kl < window) in hawk_split_hot:
 // keys 0..31 a head bucket each; keys from 32 up one of fifteen classes by
@@ -1317,14 +1034,17 @@ __device__ __forceinline__ unsigned hot_class_index(unsigned kl) {   // (kl - 32
     return ((kl - static_cast<unsigned>(kSplitHeads)) * 34953u) >> 19;
 }
 // hawk_split_tail keeps a class's accumulators together (class c = kl & 7 at
-// [768c, 768c + 768), key index m = kl >> 3), so a class wave's reads and
-// writes of distinct keys spread over the LDS banks; in key order all of a
-// class's keys sit 64 bytes apart, on four bank positions.  m is XORed with
-// 8c, which keeps it below 768 and turns the final store's reads (eight
-// classes a wave) from eight-way bank conflicts into two-way ones.
+// [K c, K c + K), K = Window / 8, key index m = kl >> 3), so a class wave's
+// reads and writes of distinct keys spread over the LDS banks; in key order all
+// of a class's keys sit 64 bytes apart, on four bank positions.  m is XORed
+// with 8c, which keeps it below K (a multiple of 64) and turns the final
+// store's reads (eight classes a wave) from eight-way bank conflicts into
+// two-way ones.
+template <int Window>
 __device__ __forceinline__ unsigned tail_slot(unsigned kl) {
+    static_assert(Window % (64 * kTailClasses) == 0, "the XOR stays inside a class");
     const unsigned c = kl & (kTailClasses - 1u);
-    return c * static_cast<unsigned>(kTailKeys) + ((kl >> kTailClassBits) ^ (c << 3));
+    return c * static_cast<unsigned>(Window / kTailClasses) + ((kl >> kTailClassBits) ^ (c << 3));
 }
 __device__ __forceinline__ int split_bucket(unsigned kl) {
     const unsigned u = kl - static_cast<unsigned>(kSplitHeads);
@@ -1525,6 +1245,11 @@ __device__ void fold_class(Sh& sh, int c) {
     const int s = static_cast<int>(sh.bstart[kSplitClassBase + c]);
     const int e = static_cast<int>(sh.bstart[kSplitClassBase + c + 1]);
     if (s >= e) return;
+    // bits below kLow pick the match slot, bits kLow .. kBits - 1 are balloted
+    constexpr int kKeys = Hot ? 1024 : Sh::kWindow / kTailClasses;
+    constexpr int kLow = Sh::kPeers == 64 ? 6 : 7;
+    constexpr int kBits = kKeys > 512 ? 10 : kKeys > 256 ? 9 : kKeys > 128 ? 8 : 7;
+    static_assert(Sh::kPeers == (1u << kLow) && kKeys <= (1 << kBits), "class matching covers every key");
     unsigned long long* peer = sh.f.peer[wave];
     unsigned k = sh.key[s + lane];
     T x = sh.val[s + lane];
@@ -1538,16 +1263,16 @@ __device__ void fold_class(Sh& sh, int c) {
         }
         const unsigned kv = valid ? k : 0u;
         const unsigned m = Hot ? hot_class_index(kv) : (kv >> kTailClassBits);
-        const unsigned h = m & (kPeerSlots - 1u);
+        const unsigned h = m & (Sh::kPeers - 1u);
         if (valid) atomicOr(&peer[h], me);
         __builtin_amdgcn_wave_barrier();
         unsigned long long pm = valid ? peer[h] : 0ull;
-        const unsigned ai = Hot ? kv : tail_slot(kv);
+        const unsigned ai = Hot ? kv : tail_slot<Sh::kWindow>(kv);
         const T a0 = valid ? sh.acc[ai] : T(0);
         __builtin_amdgcn_wave_barrier();
         if (valid) peer[h] = 0ull;
 #pragma unroll
-        for (int bit = 7; bit < 10; ++bit) {
+        for (int bit = kLow; bit < kBits; ++bit) {
             const bool one = (m >> bit) & 1u;
             const unsigned long long ones = __ballot(valid && one);
             pm &= one ? ones : ~ones;
@@ -1597,14 +1322,14 @@ __device__ void split_fold(HotShared<T>& sh) {
 }
 
 // hawk_split_tail's folds: wave w folds class w (keys with kl & 7 == w).
-template <class T>
-__device__ void split_fold_tail(TailShared<T>& sh) {
+template <class T, int Window>
+__device__ void split_fold_tail(TailShared<T, Window>& sh) {
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (unsigned i = 0; i < kPeerSlots; i += 64) sh.f.peer[wave][i + lane] = 0ull;
+    for (unsigned i = 0; i < TailShared<T, Window>::kPeers; i += 64) sh.f.peer[wave][i + lane] = 0ull;
     __builtin_amdgcn_wave_barrier();
-    fold_class<T, TailShared<T>, false>(sh, wave);
+    fold_class<T, TailShared<T, Window>, false>(sh, wave);
 }
 
 // The window's partials of chunk b, every key [klo, klo+window): a key no
@@ -1684,8 +1409,7 @@ __global__ __launch_bounds__(kWalkThreads) void hawk_split_hot(
         for (int i = t; i < (tiles - tile) * (ranges + 1); i += kWalkThreads)
             bin_off[(b * tiles + tile) * (ranges + 1) + i] = 0u;
     split_store<T>(sh, b, cells, 0, window, parts);
-    // the status plane (hawk_scatter_status's values, written here in the
-    // split walk): chunk b's flag, and from chunk 0 the cell count and the
+    // the status plane: chunk b's flag, and from chunk 0 the cell count and the
     // flags of the chunks past the last
     const int any = __syncthreads_or(bad ? 1 : 0);
     if (t == 0) status[1 + b] = any ? 1 : 0;
@@ -1725,7 +1449,7 @@ __device__ __forceinline__ int tail_reg(const int (&x)[kTailGroup / 64], int m) 
 // Group [g0, g0 + gn) of chunk b's slots, range r: every wave reads the
 // group's bounds (hawk_split_hot wrote 0 <= o[r] <= o[r+1] <= 4096; the
 // clamps keep every read inside its slot whatever the plane holds).
-__device__ __forceinline__ TailSegs tail_segs(const unsigned* __restrict__ bin_off, long long b, int tiles, int ranges,
+__device__ __forceinline__ TailSegs tail_segs(const unsigned* __restrict__ bin_off, long long b, int tiles, int row,
                                               int r, int g0, int gn) {
     const int lane = threadIdx.x & 63;
     TailSegs S;
@@ -1735,7 +1459,7 @@ __device__ __forceinline__ TailSegs tail_segs(const unsigned* __restrict__ bin_o
         const int g = k * 64 + lane;
         unsigned lo = 0u, hi = 0u;
         if (g < gn) {
-            const unsigned* o = bin_off + (b * tiles + g0 + g) * (ranges + 1);
+            const unsigned* o = bin_off + (b * tiles + g0 + g) * row;
             const unsigned a = o[r], z = o[r + 1];
             lo = a < static_cast<unsigned>(kTile) ? a : static_cast<unsigned>(kTile);
             hi = z < lo ? lo : (z < static_cast<unsigned>(kTile) ? z : static_cast<unsigned>(kTile));
@@ -1755,19 +1479,19 @@ __device__ __forceinline__ TailSegs tail_segs(const unsigned* __restrict__ bin_o
     return S;
 }
 
-// The batch at stream position qb: thread slot j of wave w takes position
-// qb + w*256 + j*64 + lane (positions past the group's end read as nothing).
+// A wave's entries from stream position q0 (wave-uniform): slot j takes
+// position q0 + j*64 + lane (positions past the group's end read as nothing).
 // Each window of 64 positions finds the segment of its first position with
-// two ballots, then steps over the segments that start inside it.
-template <class T>
+// two ballots, then steps over the segments that start inside it.  Keys: read
+// the entries' keys too.
+template <class T, bool Keys = true>
 __device__ __forceinline__ void tail_load(const TailSegs& S, const unsigned short* __restrict__ bin_key,
-                                          const T* __restrict__ bin_val, unsigned qb, unsigned (&kk)[kWalkItems],
+                                          const T* __restrict__ bin_val, unsigned q0, unsigned (&kk)[kWalkItems],
                                           T (&vv)[kWalkItems]) {
-    const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int j = 0; j < kWalkItems; ++j) {
-        const unsigned qw = qb + static_cast<unsigned>(wave * (kWalkItems * 64) + j * 64);
+        const unsigned qw = q0 + static_cast<unsigned>(j * 64);
         const unsigned q = qw + static_cast<unsigned>(lane);
         kk[j] = 0u;
         vv[j] = T(0);
@@ -1786,53 +1510,282 @@ __device__ __forceinline__ void tail_load(const TailSegs& S, const unsigned shor
         }
         if (q < S.count) {
             const long long at = S.base + a + static_cast<long long>(q);
-            kk[j] = bin_key[at];
+            if constexpr (Keys) kk[j] = bin_key[at];
             vv[j] = bin_val[at];
         }
     }
 }
 
-// (chunk b, tail range r) = (blockIdx.x / ranges, blockIdx.x % ranges): keys
-// [kSplitHot + kTailRange*r, +kTailRange) of chunk b, read as a stream from the
-// bin's slots in tile order, kTailBatch entries a batch, the next batch's reads
-// in flight while a batch is split and folded.
+// The key ranges a walk's bins hold.  The split walk: `ranges` ranges of
+// `width` keys from `first` up (singles 0, octaves 0).  The wide walk: keys
+// 0..7 a range each (singles 8), then octaves [8, 16), [16, 32), ... up to
+// `first` = 8 * 2^octaves, then ranges of `width` keys.
+struct TailRanges {
+    long long cells, first;      // keys 0 .. cells - 1 of this pass, its cell 0 at parts[0]
+    long long stride;            // cells of a chunk's row of parts
+    int ranges, singles, octaves, width;
+    int row;                     // words a tile's row of bin_off has
+};
+constexpr int kWideSingles = kTailWaves;         // 8: a wave each
+constexpr int kWideOctaves = 7;                  // [8, 16) .. [512, 1024)
+
+// a + x0 + x1 + ... + x15, one addition at a time, x_q the value lane q of
+// each row of 16 lanes holds: every row adds its own lanes' values, each
+// handed to the whole row by the add itself (DPP row_newbcast), so a value
+// costs one instruction and no LDS read: 4.9 cycles an add on MI355X (5.6
+// in float32), where a chain fed from LDS takes 11 to 25 and one fed by
+// readlane 13.5.  The fp64 add is the fused x * 1 + a, which rounds x + a once.
+// The leading s_nop covers a DPP read's wait on the lane's last write of x.
+__device__ __forceinline__ double row_chain(double a, double x) {
+    const double one = 1.0;
+#define HK_STEP(q) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #q " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" HK_STEP(0) HK_STEP(1) HK_STEP(2) HK_STEP(3) HK_STEP(4) HK_STEP(5) HK_STEP(6) HK_STEP(7)
+        HK_STEP(8) HK_STEP(9) HK_STEP(10) HK_STEP(11) HK_STEP(12) HK_STEP(13) HK_STEP(14) HK_STEP(15)
+        : "+v"(a) : "v"(x), "v"(one));
+#undef HK_STEP
+    return a;
+}
+__device__ __forceinline__ float row_chain(float a, float x) {
+#define HK_STEP(q) "v_add_f32_dpp %0, %1, %0 row_newbcast:" #q " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" HK_STEP(0) HK_STEP(1) HK_STEP(2) HK_STEP(3) HK_STEP(4) HK_STEP(5) HK_STEP(6) HK_STEP(7)
+        HK_STEP(8) HK_STEP(9) HK_STEP(10) HK_STEP(11) HK_STEP(12) HK_STEP(13) HK_STEP(14) HK_STEP(15)
+        : "+v"(a) : "v"(x));
+#undef HK_STEP
+    return a;
+}
+
+// Chunk b's chain of single key k, by one wave: the key's segment of every
+// tile slot in tile order, 256 values a step through the wave's LDS (so each
+// row of lanes holds the same 16 values at a time), the next two steps' reads
+// in flight while a step is added.  Positions past the end read as +0.0, which
+// adds nothing to a sum that is never -0.0.
 template <class T>
-__global__ __launch_bounds__(kTailThreads, 2) void hawk_split_tail(
-        long long cells, int tiles, int ranges, const unsigned short* __restrict__ bin_key,
-        const T* __restrict__ bin_val, const unsigned* __restrict__ bin_off, T* __restrict__ parts) {
-    __shared__ TailShared<T> sh;
-    const long long b = blockIdx.x / ranges;
-    const int r = static_cast<int>(blockIdx.x % ranges);
-    const long long klo = kSplitHot + static_cast<long long>(kTailRange) * r;
-    const int window = cells - klo < kTailRange ? static_cast<int>(cells - klo) : kTailRange;
-    split_clear<T>(sh, kTailRange);
+__device__ __forceinline__ T wide_chain(const T* __restrict__ bin_val, const unsigned* __restrict__ bin_off,
+                                        long long b, int tiles, int row, int k, T* buf) {
+    const int lane = threadIdx.x & 63;
+    constexpr unsigned kStep = 64 * kWalkItems;
+    T a = T(0);
     for (int g0 = 0; g0 < tiles; g0 += kTailGroup) {
         const int gn = tiles - g0 < kTailGroup ? tiles - g0 : kTailGroup;
-        const TailSegs S = tail_segs(bin_off, b, tiles, ranges, r, g0, gn);
+        const TailSegs S = tail_segs(bin_off, b, tiles, row, k, g0, gn);
+        unsigned none[kWalkItems];
+        auto load = [&](unsigned q, T (&v)[kWalkItems]) {
+            if (q < S.count) tail_load<T, false>(S, nullptr, bin_val, q, none, v);
+        };
+        auto step = [&](unsigned q, T (&v)[kWalkItems]) {
+            if (q >= S.count) return;
+#pragma unroll
+            for (int j = 0; j < kWalkItems; ++j) buf[j * 64 + lane] = v[j];
+            __builtin_amdgcn_wave_barrier();
+            load(q + 2 * kStep, v);
+            const int left = static_cast<int>(S.count - q < kStep ? S.count - q : kStep);
+            for (int m = 0; m < left; m += 64) {
+                T x[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = buf[m + 16 * e + (lane & 15)];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a = row_chain(a, x[e]);
+            }
+            __builtin_amdgcn_wave_barrier();
+        };
+        T v0[kWalkItems], v1[kWalkItems];
+        load(0u, v0);
+        load(kStep, v1);
+        for (unsigned q = 0; q < S.count; q += 2 * kStep) {
+            step(q, v0);
+            step(q + kStep, v1);
+        }
+    }
+    return a;
+}
+
+// The chains of a split tile's buckets c, c + step, ... below `keys` (each the
+// run of one key, lane order), by one wave, 64 values a round.
+template <class T, class Sh>
+__device__ __forceinline__ void fold_rows(Sh& sh, int c, int step, int keys) {
+    const int lane = threadIdx.x & 63;
+    for (; c < keys; c += step) {
+        const int s = static_cast<int>(sh.bstart[c]), e = static_cast<int>(sh.bstart[c + 1]);
+        if (s >= e) continue;
+        T a = sh.acc[c];
+        for (int m = s; m < e; m += 64) {
+            T x[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int at = m + 16 * q + (lane & 15);
+                const T v = sh.val[at];                      // up to 63 entries past the run (the padding)
+                x[q] = at < e ? v : T(0);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (m + 16 * q < e) a = row_chain(a, x[q]);
+        }
+        if (lane == 0) sh.acc[c] = a;
+    }
+}
+
+// Range r of chunk b, read as a stream from the bin's slots in tile order,
+// kTailBatch entries a batch, the next batch's reads in flight while a batch
+// is split and folded: in eight classes, or, for a range of at most 32 keys,
+// in a bucket a key (a chain a key: few keys share many lanes).  Workgroups
+// chunk by chunk, range after range; with
+// single keys (the wide walk) the first `chunks` workgroups are the chunks'
+// chains, a wave a key, and with a status plane they also gather the chunk's
+// bad-key flags, which hawk_wide_bin left behind each tile's
+// offsets.  Windows up to 3072 keys leave three workgroups a CU, larger two.
+template <class T, int Window>
+__global__ __launch_bounds__(kTailThreads, Window <= 3072 ? 6 : 4) void hawk_split_tail(
+        TailRanges R, int chunks, int tiles, const unsigned short* __restrict__ bin_key,
+        const T* __restrict__ bin_val, const unsigned* __restrict__ bin_off, T* __restrict__ parts,
+        int* __restrict__ status) {
+    __shared__ __align__(16) TailShared<T, Window> sh;
+    const int t = threadIdx.x;
+    const int i = static_cast<int>(blockIdx.x);
+    const long long b = i % chunks;
+    if (R.singles > 0 && i < chunks) {
+        const int k = t >> 6;
+        const T a = wide_chain<T>(bin_val, bin_off, b, tiles, R.row, k, sh.val + k * (64 * kWalkItems));
+        if ((t & 63) == 0 && k < R.cells) parts[b * R.stride + k] = a;
+        if (status == nullptr) return;
+        unsigned bad = 0u;
+        for (int g = t; g < tiles; g += kTailThreads) bad |= bin_off[(b * tiles + g) * R.row + R.row - 1];
+        const int any = __syncthreads_or(bad ? 1 : 0);
+        if (t == 0) status[1 + b] = any;
+        if (b == 0)
+            for (int c = chunks + t; c < kScatterChunks; c += kTailThreads) status[1 + c] = 0;
+        if (i == 0 && t == 0) status[0] = static_cast<int>(R.stride);
+        return;
+    }
+    const int r = R.singles + i / chunks - (R.singles > 0 ? 1 : 0);
+    const int u = r - R.singles - R.octaves;
+    const long long klo = u < 0 ? static_cast<long long>(kWideSingles) << (r - R.singles)
+                                : R.first + static_cast<long long>(R.width) * u;
+    const long long size = u < 0 ? klo : R.width;
+    // past the last pass's cells a range holds no key (and its window none)
+    const int window = static_cast<int>(klo + size < R.cells ? size : R.cells - klo);
+    const bool few = size <= kSplitHeads;
+    split_clear<T>(sh, Window);
+    for (int g0 = 0; g0 < tiles; g0 += kTailGroup) {
+        const int gn = tiles - g0 < kTailGroup ? tiles - g0 : kTailGroup;
+        const TailSegs S = tail_segs(bin_off, b, tiles, R.row, r, g0, gn);
+        const unsigned w0 = static_cast<unsigned>((t >> 6) * (kWalkItems * 64));
         unsigned nk[kWalkItems];
         T nv[kWalkItems];
-        if (S.count > 0u) tail_load(S, bin_key, bin_val, 0u, nk, nv);
+        if (S.count > 0u) tail_load(S, bin_key, bin_val, w0, nk, nv);
         for (unsigned qb = 0; qb < S.count; qb += kTailBatch) {
             unsigned kl[kWalkItems];
             int d[kWalkItems];
             T vv[kWalkItems];
 #pragma unroll
             for (int j = 0; j < kWalkItems; ++j) {
-                const unsigned q = qb + static_cast<unsigned>((threadIdx.x >> 6) * (kWalkItems * 64) + j * 64 +
-                                                              (threadIdx.x & 63));
+                const unsigned q = qb + w0 + static_cast<unsigned>(j * 64 + (t & 63));
                 kl[j] = nk[j];
                 vv[j] = nv[j];
-                d[j] = q < S.count ? kSplitClassBase + static_cast<int>(kl[j] & (kTailClasses - 1u)) : kSplitNone;
+                const unsigned in = few ? kl[j] & (kSplitHeads - 1u) : kSplitClassBase + (kl[j] & (kTailClasses - 1u));
+                d[j] = q < S.count ? static_cast<int>(in) : kSplitNone;
             }
-            if (qb + kTailBatch < S.count) tail_load(S, bin_key, bin_val, qb + kTailBatch, nk, nv);
-            split_tile<T, TailShared<T>, false>(sh, kl, d, vv, kSplitClassBase + kTailClasses, TailSink<T>());
-            split_fold_tail(sh);
+            if (qb + kTailBatch < S.count) tail_load(S, bin_key, bin_val, qb + kTailBatch + w0, nk, nv);
+            split_tile<T, TailShared<T, Window>, false>(sh, kl, d, vv, kSplitClassBase + kTailClasses, TailSink<T>());
+            if (few) fold_rows<T>(sh, t >> 6, kTailWaves, static_cast<int>(size));
+            else split_fold_tail<T, Window>(sh);
             __syncthreads();
         }
     }
     __syncthreads();
-    T* row = parts + b * cells + klo;
-    for (int k = threadIdx.x; k < window; k += kTailThreads) row[k] = sh.acc[tail_slot(static_cast<unsigned>(k))];
+    T* row = parts + b * R.stride + klo;
+    for (int k = t; k < window; k += kTailThreads) row[k] = sh.acc[few ? static_cast<unsigned>(k) : tail_slot<Window>(static_cast<unsigned>(k))];
+}
+
+// ---- the wide walk ----------------------------------------------------------
+// hawk_split_hot walks a chunk in one workgroup, so a scatter of few chunks
+// (n / cells of them, at most 256) leaves most of the chip idle, and its
+// window and buckets end at 65536 cells.  The wide walk splits first and walks
+// after: hawk_wide_bin splits every tile of every chunk on its own (a workgroup
+// a tile, no order between them) into the key ranges' bins, and
+// hawk_split_tail folds every (chunk, range) in lane order, a workgroup each:
+// the same additions.  A skewed histogram's head keys 0..7 are chains of their
+// own, a wave each, and the ranges above them grow by octaves, so a Zipf
+// histogram's ranges hold about equal shares of its other lanes.  More than
+// kWideCells cells take a pass (both launches) per kWideCells of them.
+constexpr int kWideBuckets = 62;                 // ranges a tile splits into (bucket 63 is a lane that adds nothing)
+constexpr int kWideStride = 63;
+constexpr long long kWideCells = (static_cast<long long>(kWideSingles) << kWideOctaves) +
+                                 static_cast<long long>(kWideBuckets - kWideSingles - kWideOctaves) * kTailRange;
+constexpr int kWideGroups = 2048;                // workgroups hawk_split_tail gets where the cells allow it
+
+// Which walk: the wide one where the split walk cannot go (more than 65536
+// cells) and where its workgroup a chunk leaves the chip idle for longer than
+// a second pass over the lanes takes.  Measured (fp64, split / wide, us, at
+// uniform keys; the same lines hold at Zipf keys): 65536 cells in 16 chunks
+// 113 / 31, in 64 135 / 72, in 128 164 / 129, in 183 195 / 175, in 256
+// 225 / 238; 20000 cells in 104 chunks 73 / 51, in 209 83 / 87.  Up to 12288
+// cells (no tail ranges) a chunk is at most three tiles: 10000 cells in 20
+// chunks 29 / 23, in 50 31 / 34; 4000 cells in 16 chunks 16 / 18.  Past 65536
+// cells, against the sorted walk this replaced: 2^18 cells, 2^22 lanes 1470 us
+// uniform and 1395 us Zipf -> 74 and 166 us.
+bool wide_walk(int64_t cells, int chunks) {
+    return cells > kSplitCells || chunks < (cells > kSplitHot ? 192 : cells > 2 * kTile ? 32 : 0);
+}
+
+template <class T>
+using WideShared = SplitShared<T, kWalkWaves, 1, kWideStride, 1>;        // 54 KiB (float64): two a CU
+static_assert(kWideBuckets < kWideStride && kSplitNone >= kWideStride, "bucket starts need one past the last bucket");
+
+// Tile g of chunk b (blockIdx.x = b * tiles + g): its entries in range order
+// into the tile's slot of the bins, the ranges' offsets and a flag for a key
+// that is neither a cell nor -1 into the tile's row of bin_off.  The pass takes
+// keys [key0, key0 + R.cells).  magic is floor(2^32 / width): the quotient it
+// gives is exact or one short.
+template <class T>
+__global__ __launch_bounds__(kWalkThreads) void hawk_wide_bin(
+        const int* __restrict__ key, const T* __restrict__ v, long long n, long long span, int tiles, TailRanges R,
+        unsigned key0, unsigned magic, unsigned short* __restrict__ bin_key, T* __restrict__ bin_val,
+        unsigned* __restrict__ bin_off) {
+    __shared__ WideShared<T> sh;
+    const int t = threadIdx.x;
+    const long long b = blockIdx.x / static_cast<unsigned>(tiles);
+    const long long g = blockIdx.x % static_cast<unsigned>(tiles);
+    const long long lo = b * span + g * kTile;
+    const long long end = (b + 1) * span < n ? (b + 1) * span : n;
+    const long long hi = lo + kTile < end ? lo + kTile : end;
+    int kk[kWalkItems];
+    T vv[kWalkItems];
+    walk_load(key, v, lo, hi, kk, vv);
+    unsigned kl[kWalkItems];
+    int d[kWalkItems];
+    bool bad = false;
+    const unsigned first = static_cast<unsigned>(R.first), width = static_cast<unsigned>(R.width);
+#pragma unroll
+    for (int j = 0; j < kWalkItems; ++j) {
+        bad = bad | ((kk[j] != -1) & !(static_cast<unsigned>(kk[j]) < static_cast<unsigned>(R.stride)));
+        // a key below key0 wraps past the pass's cells
+        const unsigned u = static_cast<unsigned>(kk[j]) - key0;
+        const bool mine = (kk[j] >= 0) & (u < static_cast<unsigned>(R.cells));
+        const unsigned w = u - first;
+        unsigned q = __umulhi(w, magic);
+        unsigned rem = w - q * width;
+        if (rem >= width) {
+            q += 1u;
+            rem -= width;
+        }
+        const int o = 31 - __builtin_clz(u | 1u);            // key u's octave, 2^o <= u
+        const bool single = u < static_cast<unsigned>(kWideSingles);
+        const int low = single ? static_cast<int>(u) : kWideSingles + o - 3;
+        d[j] = !mine ? kSplitNone : u < first ? low : kWideSingles + R.octaves + static_cast<int>(q);
+        kl[j] = u < first ? (single ? 0u : u - (1u << o)) : rem;
+    }
+    static_assert(kWideSingles == 8, "the first octave is [8, 16)");
+    split_tile<T, WideShared<T>, false>(sh, kl, d, vv, R.ranges, TailSink<T>());
+    const long long slot = b * tiles + g;
+    const unsigned count = sh.bstart[R.ranges];
+    for (unsigned i = t; i < count; i += kWalkThreads) {
+        bin_key[slot * kTile + i] = sh.key[i];
+        bin_val[slot * kTile + i] = sh.val[i];
+    }
+    unsigned* row = bin_off + slot * R.row;
+    if (t <= R.ranges) row[t] = sh.bstart[t];
+    const int any = __syncthreads_or(bad ? 1 : 0);
+    if (t == 0) row[R.row - 1] = static_cast<unsigned>(any);
 }
 
 // The ordered scatter's scratch, in this order (each part 256-byte aligned):
@@ -1842,9 +1795,11 @@ __global__ __launch_bounds__(kTailThreads, 2) void hawk_split_tail(
 struct ScatterLayout {
     int chunks = 1;
     long long span = 0;
-    bool split = false;
+    bool wide = false;             // the wide walk, else the split walk
     int tiles = 0;
-    int ranges = 0;
+    int ranges = 0;                // key ranges the bins hold
+    int octaves = 0, width = 0;    // the wide walk's octaves, and keys a range past them
+    int row = 0;                   // words a tile's row of bin_off has
     size_t parts = 0, bin_off = 0, bin_key = 0, bin_val = 0, bytes = 0;
 };
 
@@ -1854,24 +1809,43 @@ ScatterLayout scatter_layout(int64_t n, int64_t cells, int chunks) {
     ScatterLayout L;
     L.chunks = chunks;
     L.span = (n + chunks - 1) / chunks;
-    L.split = cells <= kSplitCells;
+    L.wide = wide_walk(cells, chunks);
     const size_t c = static_cast<size_t>(chunks);
     size_t at = 0;
     L.parts = at;
     at += align256(sizeof(double) * c * static_cast<size_t>(cells));
-    if (L.split) {
-        const long long tiles = (L.span + kTile - 1) / kTile;
-        L.tiles = static_cast<int>(tiles < 1 ? 1 : tiles);
-        L.ranges = cells > kSplitHot ? static_cast<int>((cells - kSplitHot + kTailRange - 1) / kTailRange) : 0;
-        if (L.ranges > 0) {
-            const size_t slots = c * static_cast<size_t>(L.tiles);
-            L.bin_off = at;
-            at += align256(sizeof(unsigned) * slots * static_cast<size_t>(L.ranges + 1));
-            L.bin_key = at;
-            at += align256(sizeof(unsigned short) * slots * kTile);
-            L.bin_val = at;
-            at += align256(sizeof(double) * slots * kTile);
+    const long long tiles = (L.span + kTile - 1) / kTile;
+    L.tiles = static_cast<int>(tiles < 1 ? 1 : tiles);
+    if (L.wide) {
+        // octaves up to the pass's cells; past them enough ranges for
+        // kWideGroups workgroups of hawk_split_tail, no more than the buckets,
+        // none narrower than 64 keys
+        const long long pass = cells < kWideCells ? cells : kWideCells;
+        while (L.octaves < kWideOctaves && (static_cast<long long>(kWideSingles) << L.octaves) < pass) ++L.octaves;
+        const long long rest = pass - (static_cast<long long>(kWideSingles) << L.octaves);
+        if (rest > 0) {
+            long long want = kWideGroups / chunks;
+            const long long most = kWideBuckets - kWideSingles - L.octaves;
+            const long long least = (rest + kTailRange - 1) / kTailRange;
+            if (want > (rest + 63) / 64) want = (rest + 63) / 64;
+            if (want < least) want = least;
+            if (want > most) want = most;
+            L.width = static_cast<int>((rest + want - 1) / want);
+            L.ranges = static_cast<int>((rest + L.width - 1) / L.width);
         }
+        L.ranges += kWideSingles + L.octaves;
+    } else {
+        L.ranges = cells > kSplitHot ? static_cast<int>((cells - kSplitHot + kTailRange - 1) / kTailRange) : 0;
+    }
+    L.row = L.ranges + (L.wide ? 2 : 1);
+    if (L.ranges > 0) {
+        const size_t slots = c * static_cast<size_t>(L.tiles);
+        L.bin_off = at;
+        at += align256(sizeof(unsigned) * slots * static_cast<size_t>(L.row));
+        L.bin_key = at;
+        at += align256(sizeof(unsigned short) * slots * kTile);
+        L.bin_val = at;
+        at += align256(sizeof(double) * slots * kTile);
     }
     L.bytes = at;
     return L;
@@ -1980,12 +1954,6 @@ int launch_error(const char* what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hawk_internal::set_hip_error(what, e);
     return HK_OK;
-}
-
-int bits_for(long long max_value) {
-    int b = 1;
-    while ((1LL << b) <= max_value) ++b;
-    return b;
 }
 
 }  // namespace
@@ -2207,6 +2175,16 @@ int keyed_log_fold(const T* values, int64_t stride, const int32_t* cells_log, in
     return launch_error("hawk_log_fold_waves launch");
 }
 
+template <class T, int Window>
+int split_tail(const TailRanges& R, int chunks, int tiles, const unsigned short* bin_key, const T* bin_val,
+               const unsigned* bin_off, T* parts, int32_t* status, hipStream_t s) {
+    // the wide walk's single keys share a workgroup a chunk
+    const int groups = R.singles > 0 ? R.ranges - R.singles + 1 : R.ranges;
+    hipLaunchKernelGGL((hawk_split_tail<T, Window>), dim3(static_cast<unsigned>(chunks * groups)),
+                       dim3(kTailThreads), 0, s, R, chunks, tiles, bin_key, bin_val, bin_off, parts, status);
+    return launch_error("hawk_split_tail launch");
+}
+
 // The ordered scatter in T (hk_ordered_scatter_f64 / _f32).
 template <class T>
 int ordered_scatter(const int32_t* key, const T* v, int64_t n, T* target, int64_t cells, void* scratch,
@@ -2225,50 +2203,45 @@ int ordered_scatter(const int32_t* key, const T* v, int64_t n, T* target, int64_
     const ScatterLayout L = scatter_layout(n, cells, chunks);
     unsigned char* base = static_cast<unsigned char*>(scratch);
     auto* parts = reinterpret_cast<T*>(base + L.parts);     // a float scatter uses the front of each region
+    auto* bin_off = reinterpret_cast<unsigned*>(base + L.bin_off);
+    auto* bin_key = reinterpret_cast<unsigned short*>(base + L.bin_key);
+    auto* bin_val = reinterpret_cast<T*>(base + L.bin_val);
     int rc = HK_OK;
-    if (!L.split) {
-        hipLaunchKernelGGL(hawk_scatter_status, dim3(1), dim3(kScatterChunks + 64), 0, s, status,
-                           static_cast<long long>(cells));
-        rc = launch_error("hawk_scatter_status launch");
-        if (rc != HK_OK) return rc;
-    }
-    if (L.split) {
-        auto* bin_off = reinterpret_cast<unsigned*>(base + L.bin_off);
-        auto* bin_key = reinterpret_cast<unsigned short*>(base + L.bin_key);
-        auto* bin_val = reinterpret_cast<T*>(base + L.bin_val);
+    if (L.wide) {
+        const long long slots = static_cast<long long>(chunks) * L.tiles;
+        if (slots > 0x7fffffffLL) return hawk_internal::set_error(HK_EVALUE, who + ": too many samples");
+        // with no width every key is below `first`
+        const unsigned magic = L.width > 1 ? static_cast<unsigned>((1ull << 32) / static_cast<unsigned>(L.width))
+                                           : 0xffffffffu;
+        for (long long key0 = 0; key0 < cells; key0 += kWideCells) {
+            const TailRanges R{cells - key0 < kWideCells ? cells - key0 : kWideCells,
+                               static_cast<long long>(kWideSingles) << L.octaves, static_cast<long long>(cells),
+                               L.ranges, kWideSingles, L.octaves, L.width, L.row};
+            hipLaunchKernelGGL(hawk_wide_bin<T>, dim3(static_cast<unsigned>(slots)), dim3(kWalkThreads), 0, s, key, v,
+                               static_cast<long long>(n), L.span, L.tiles, R, static_cast<unsigned>(key0), magic,
+                               bin_key, bin_val, bin_off);
+            rc = launch_error("hawk_wide_bin launch");
+            if (rc != HK_OK) return rc;
+            T* row = parts + key0;
+            int32_t* flags = key0 == 0 ? status : nullptr;
+            rc = L.width <= 1024   ? split_tail<T, 1024>(R, chunks, L.tiles, bin_key, bin_val, bin_off, row, flags, s)
+                 : L.width <= 3072 ? split_tail<T, 3072>(R, chunks, L.tiles, bin_key, bin_val, bin_off, row, flags, s)
+                                   : split_tail<T, kTailRange>(R, chunks, L.tiles, bin_key, bin_val, bin_off, row,
+                                                               flags, s);
+            if (rc != HK_OK) return rc;
+        }
+    } else {
         hipLaunchKernelGGL(hawk_split_hot<T>, dim3(static_cast<unsigned>(chunks)), dim3(kWalkThreads), 0, s, key, v,
                            static_cast<long long>(n), static_cast<long long>(cells), L.span, L.tiles, L.ranges,
                            bin_key, bin_val, bin_off, parts, status);
         rc = launch_error("hawk_split_hot launch");
         if (rc != HK_OK) return rc;
         if (L.ranges > 0) {
-            hipLaunchKernelGGL(hawk_split_tail<T>, dim3(static_cast<unsigned>(chunks * L.ranges)), dim3(kTailThreads),
-                               0, s, static_cast<long long>(cells), L.tiles, L.ranges, bin_key, bin_val, bin_off,
-                               parts);
-            rc = launch_error("hawk_split_tail launch");
+            const TailRanges R{static_cast<long long>(cells), kSplitHot, static_cast<long long>(cells), L.ranges, 0, 0,
+                               kTailRange, L.row};
+            rc = split_tail<T, kTailRange>(R, chunks, L.tiles, bin_key, bin_val, bin_off, parts, nullptr, s);
             if (rc != HK_OK) return rc;
         }
-    } else {
-        // more cells than the split walk's windows cover: parts arrives
-        // zero-filled and the sorted walk (or, past its key field, the serial
-        // walk) adds onto it
-        const long long count = static_cast<long long>(chunks) * cells;
-        const long long blocks = (count + 255) / 256 < 4096 ? (count + 255) / 256 : 4096;
-        hipLaunchKernelGGL(hawk_fill_zero<T>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, parts, count);
-        rc = launch_error("hawk_fill_zero launch");
-        if (rc != HK_OK) return rc;
-        const int key_bits = bits_for(cells - 1);
-        if (key_bits <= kMaxKeyBits) {
-            hipLaunchKernelGGL(hawk_scatter_walk<T>, dim3(static_cast<unsigned>(chunks)), dim3(kWalkThreads), 0, s,
-                               key, v, static_cast<long long>(n), static_cast<long long>(cells), L.span, key_bits,
-                               parts, status);
-            rc = launch_error("hawk_scatter_walk launch");
-        } else {
-            hipLaunchKernelGGL(hawk_scatter_serial<T>, dim3(static_cast<unsigned>(chunks)), dim3(64), 0, s, key, v,
-                               static_cast<long long>(n), static_cast<long long>(cells), L.span, parts, status);
-            rc = launch_error("hawk_scatter_serial launch");
-        }
-        if (rc != HK_OK) return rc;
     }
     const long long grid = (cells + 255) / 256;
     hipLaunchKernelGGL(hawk_scatter_cells<T>, dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, parts,

@@ -44,3 +44,44 @@ def test_mm16_streamed_and_cached(tmp_path, gpu, mode, n, shift):
     hawk.run(vjp, A=a, B=b, bar_C=c, bar_A=bar_A, bar_B=bar_B, layout="samples_last")
     for x, (X, Y) in ((got, (A, B)), (bar_A, (C, B.transpose(1, 0, 2))), (bar_B, (A.transpose(1, 0, 2), C))):
         assert np.array_equal(x.cpu().numpy(), np.einsum("ikn,kjn->ijn", X, Y))
+
+
+@pytest.mark.parametrize("mode", ["float64", "float32"])
+@pytest.mark.parametrize("cells, n, keys", [
+    (8192, 60_000, "zipf"), (8193, 60_000, "zipf"), (9000, 9000 * 31, "one"), (9000, 9000 * 32, "one"),
+    (12_289, 100, "uniform"), (20_000, 20_000 * 191, "zipf"), (20_000, 20_000 * 192, "sorted"),
+    (65_537, 65_537, "uniform"), (65_537, 400_003, "sorted"), (65_600, 700_001, "zipf"), (65_600, 300_000, "one"),
+    (289_792, 600_001, "zipf"), (289_793, 600_001, "zipf"), (1 << 20, 5_000, "uniform"), (70_000, 0, "uniform")])
+def test_ordered_scatter_walks(tmp_path, gpu, mode, cells, n, keys):
+    """Few chunks, many cells and their neighbours on the other walk: the
+    serial walk's bits, skip keys and infinities among the lanes, and the bad
+    keys reported with every other lane added."""
+    import hawk_amd as hawk
+    import oracle_lib as O
+    import torch
+    from hawk_amd import HawkError
+    from hawk_amd import examples as E
+    dt = np.float32 if mode == "float32" else np.float64
+    g = np.random.default_rng(cells + n)
+    key = {"uniform": lambda: g.integers(0, cells, n), "sorted": lambda: np.sort(g.integers(0, cells, n)),
+           "zipf": lambda: (g.zipf(1.1, n) - 1) % cells, "one": lambda: np.full(n, cells - 3)}[keys]().astype(np.int32)
+    key[::11] = -1
+    x = (g.normal(size=n) * np.exp(g.normal(size=n))).astype(dt)
+    x[5::1001] = np.inf
+    acc0 = np.linspace(1.0, 2.0, cells).astype(dt)
+    (k,) = _unit(tmp_path, [E.ordered_add], mode)
+    planes = {"x": torch.from_numpy(x).to(gpu)}
+    for bad in (False, True):
+        if bad and n:
+            key[n // 2], key[n - 1] = cells, -2
+        acc = torch.from_numpy(acc0).to(gpu)
+        print(f"scatter cells={cells} n={n} {keys} {mode} bad={bad}", flush=True)
+        call = dict(key=torch.from_numpy(key).to(gpu), acc=acc, **planes)
+        if bad and n:
+            with pytest.raises(HawkError, match="outside"):
+                hawk.run(k, **call)
+        else:
+            hawk.run(k, **call)
+        want, status = O.ordered_scatter(key, x, acc0)
+        assert bool(status[1:].any()) == (bad and n > 0)
+        assert acc.cpu().numpy().tobytes() == want.tobytes()
