@@ -85,3 +85,39 @@ def test_ordered_scatter_walks(tmp_path, gpu, mode, cells, n, keys):
         want, status = O.ordered_scatter(key, x, acc0)
         assert bool(status[1:].any()) == (bad and n > 0)
         assert acc.cpu().numpy().tobytes() == want.tobytes()
+
+
+def _per_key(group, policy):
+    import hawk_amd as hawk
+    from hawk_amd import Grid, Kernel, Scalar
+
+    @hawk.kernel
+    def key_total(lane: Grid["key", "sample":group], x: Scalar) -> Scalar:
+        return hawk.sum(x, over="sample", policy=policy)
+    return Kernel("key_total", key_total.program)
+
+
+@pytest.mark.parametrize("mode", ["float64", "float32"])
+@pytest.mark.parametrize("keys, group", [
+    (9, 1), (7, 31), (8, 32), (5, 33), (3, 64), (5, 65), (6, 128), (5, 129), (3, 256), (5, 257), (5, 512), (4, 513),
+    (5, 1024), (5, 1025), (3, 2048), (511, 2049), (512, 2049), (2, 256 * 32 + 1), (2, 131_072), (2, 131_073),
+    (600, 8193)])
+def test_keyed_default_sum_routes(tmp_path, gpu, mode, keys, group):
+    """Rows of eight lanes, every number of rows a step and a key can hold: the
+    oracle's bits, with infinities, NaN and signed zeros among the values."""
+    import hawk_amd as hawk
+    import oracle_lib as O
+    import torch
+    dt = np.float32 if mode == "float32" else np.float64
+    g = np.random.default_rng(keys * 7 + group)
+    x = (g.normal(size=keys * group) * 2.0 ** g.integers(-20, 20, keys * group)).astype(dt)
+    x[g.random(x.size) < 0.1] = -0.0
+    if keys > 2:
+        x[group // 2], x[2 * group - 1] = np.inf, np.nan
+    (k,) = _unit(tmp_path, [_per_key(group, "auto")], mode)
+    out = torch.full((keys,), 7.0, dtype=torch.float32 if mode == "float32" else torch.float64, device=gpu)
+    hawk.run(k, x=torch.from_numpy(x).to(gpu), out=out)
+    want = O.keyed_sample_sum(x, group)
+    got = out.cpu().numpy()
+    nan = np.isnan(want)
+    assert (np.isnan(got) == nan).all() and got[~nan].tobytes() == want[~nan].tobytes()
