@@ -548,7 +548,7 @@ STAGE_KERNELS = {"ordered_sum": ("hawk_sum_lanes", "hawk_sum_fold"),
                  "band_ordered_sum": ("hawk_band_sum_lanes", "hawk_band_sum_fold"),
                  "ordered_scatter": ("hawk_split_hot", "hawk_wide_bin", "hawk_split_tail", "hawk_scatter_cells"),
                  "mm16": ("hawk_mm16_f32", "hawk_mm16_f64"),
-                 "keyed_sum": ("hawk_keyed_rows",),      # keys of at most 65536 samples (config 5k: 4096)
+                 "keyed_sum": ("hawk_keyed_rows",),      # keys of 1025 to 65536 samples (config 5k: 4096)
                  "mm16#2": ("hawk_mm16_f32_shared", "hawk_mm16_f64_shared"),
                  "ordered_fold": ("hawk_log_fold_lanes", "hawk_log_fold_waves")}
 COPY_PROBE_BYTES = 1 << 30

@@ -27,6 +27,7 @@ constexpr int kFoldLanes = 1024;
 constexpr int kGroups = 64;            // reference hawk/ir/team.py:649 GROUPS
 constexpr int kLaneBlock = 256;
 constexpr int kSumUnroll = 32;
+constexpr int kSumTail = 8;
 
 // Scratch layout (bytes): lanes[65536] f64 | gp[64] f64 | ticket u32 (+pad).
 constexpr size_t kLanesBytes = sizeof(double) * kVirtualLanes;
@@ -55,7 +56,16 @@ __global__ __launch_bounds__(kLaneBlock) void hawk_sum_lanes(const T* __restrict
 #pragma unroll
         for (int k = 0; k < kSumUnroll; ++k) s += a[k];
     }
-    for (; r < n; r += kStep) s += u[r];
+    // the rows left, eight loads in flight; a row past the end adds +0.0, which
+    // leaves a sum that is never -0.0 as it is.  One load at a time they took
+    // 14 of the kernel's 23 us at n = 10^7 (24 rows past four full blocks).
+    for (; r < n; r += kSumTail * kStep) {
+        T a[kSumTail];
+#pragma unroll
+        for (int k = 0; k < kSumTail; ++k) a[k] = r + k * kStep < n ? __builtin_nontemporal_load(u + r + k * kStep) : T(0);
+#pragma unroll
+        for (int k = 0; k < kSumTail; ++k) s += a[k];
+    }
     lanes[l] = s;
 }
 
@@ -608,15 +618,21 @@ __global__ __launch_bounds__(256) void hawk_keyed_comp_wave(const T* __restrict_
     const long long k = Steps > 1 ? wave : wave * (8 / G) + g / G;
     const int row = Steps > 1 ? g : g & (G - 1);
     const T* __restrict__ mine = u + (k < keys ? k : 0) * group;
-    const long long len = k < keys ? group : 0;
+    const int len = k < keys ? static_cast<int>(group) : 0;
+    const T* __restrict__ from = mine + row * 32 + j;
     T x[Steps][4];
 #pragma unroll
-    for (int s = 0; s < Steps; ++s)
+    for (int s = 0; s < Steps; ++s) {
+        if (Steps > 1 && (s + 1) * 256 <= len) {            // eight whole rows of the wave's key
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const long long at = (s * 8 + row) * 32 + j + 8 * v;
-            x[s][v] = at < len ? __builtin_nontemporal_load(mine + at) : T(0);
+            for (int v = 0; v < 4; ++v) x[s][v] = __builtin_nontemporal_load(from + s * 256 + 8 * v);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                x[s][v] = s * 256 + row * 32 + j + 8 * v < len ? __builtin_nontemporal_load(from + s * 256 + 8 * v)
+                                                               : T(0);
         }
+    }
     T h[Steps], c[Steps];
 #pragma unroll
     for (int s = 0; s < Steps; ++s) row_of_eight<T>(x[s], h[s], c[s]);
@@ -656,14 +672,23 @@ __global__ __launch_bounds__(64 * Waves) void hawk_keyed_comp(const T* __restric
         for (int i = 0; i < kOwn; ++i) h[i] = c[i] = T(0);
         for (int r0 = 0; r0 < cnt; r0 += kRowSlots) {
             T x[kOwn][4];
+            const long long base = (first + r0) * 32;
+            const T* __restrict__ from = mine + base + mine8 * 32 + j;
+            if (base + kRowSlots * 32 <= group) {               // whole rows, a row a slot
 #pragma unroll
-            for (int i = 0; i < kOwn; ++i)
+                for (int i = 0; i < kOwn; ++i)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const long long at = (first + r0 + mine8 + kGroups8 * i) * 32 + j + 8 * v;
-                    const bool in = r0 + mine8 + kGroups8 * i < cnt && at < group;
-                    x[i][v] = in ? __builtin_nontemporal_load(mine + at) : T(0);
-                }
+                    for (int v = 0; v < 4; ++v)
+                        x[i][v] = __builtin_nontemporal_load(from + kGroups8 * i * 32 + 8 * v);
+            } else {
+                const int left = static_cast<int>(group - base) - mine8 * 32 - j;
+#pragma unroll
+                for (int i = 0; i < kOwn; ++i)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        x[i][v] = kGroups8 * i * 32 + 8 * v < left
+                                      ? __builtin_nontemporal_load(from + kGroups8 * i * 32 + 8 * v) : T(0);
+            }
 #pragma unroll
             for (int i = 0; i < kOwn; ++i) {
                 if (r0 + wave8 + kGroups8 * i >= cnt) break;             // no rows for the whole wave
@@ -726,160 +751,165 @@ __global__ __launch_bounds__(64 * Waves) void hawk_keyed_comp(const T* __restric
 // others are +0.0, and so are the groups past ceil(lv / 1024).  No lane value
 // or tree sum is ever -0.0 (each starts at +0.0; a round-to-nearest sum is
 // -0.0 only from two -0.0 operands), so adding +0.0 is the identity and the
-// trees need only their first P = min(1024, 2^ceil(log2 lv)) lanes and first
-// Q = 2^ceil(log2 groups) group values: the bits of the full trees.
+// trees need only the lanes and group values that hold rows, the others +0.0:
+// the bits of the full trees.
 // ---------------------------------------------------------------------------
-template <class T>
-__global__ __launch_bounds__(256) void hawk_keyed_lanes(const T* __restrict__ u, long long group, long long lv,
-                                                        long long total, T* __restrict__ lanes) {
-    for (long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; i < total;
-         i += static_cast<long long>(gridDim.x) * 256) {
-        const long long k = i / lv, l = i - k * lv;
-        const T* row = u + k * group;
-        T part = T(0);
-        for (long long r = l; r < group; r += kVirtualLanes) part = part + __builtin_nontemporal_load(row + r);
-        lanes[i] = part;
-    }
-}
-
 __host__ __device__ __forceinline__ int pow2_at_least(long long x) {
     int p = 1;
     while (p < x) p <<= 1;
     return p;
 }
 
-// The halving tree s[i] += s[i + w], w = P/2 .. 1, of P <= 1024 values (a
-// power of 2; zeros past the data) held by a 256-thread workgroup as
-// s[t + 256j] = v[j]: the levels w = 512 and 256 pair values of one thread,
-// w = 128 and 64 go through LDS, w = 32 .. 1 through the first wave's
-// shuffles (lane i reads lane i + w; only lanes below w carry on).  The
-// same pairs, in the same order, as the tree over LDS.  Thread 0 returns s[0].
+// The halving tree over a wave's lanes, lane i adding lane i + w's value for
+// w = P/2 .. 1 (P a power of 2; only lanes below w carry on): lane 0 of each
+// P lanes ends with their tree's sum.  Rows of 16 lanes shift by DPP.
 template <class T>
-__device__ __forceinline__ T block_tree(T (&v)[4], int P, T* sh) {
-    const int t = threadIdx.x;
-    if (P > 512) { v[0] = v[0] + v[2]; v[1] = v[1] + v[3]; }
-    if (P > 256) v[0] = v[0] + v[1];
-    T x = v[0];
-    if (P > 64) {
-        sh[t] = x;
-        __syncthreads();
-        if (P > 128 && t < 128) sh[t] = sh[t] + sh[t + 128];
-        __syncthreads();
-        if (t < 64) x = sh[t] + sh[t + 64];
-    }
-    if (t < 64) {
-#pragma unroll
-        for (int w = 32; w >= 1; w >>= 1) {
-            const T y = __shfl_down(x, w, 64);
-            if (P > w) x = x + y;
-        }
-    }
-    __syncthreads();                      // sh is free for the next tree
+__device__ __forceinline__ T wave_tree(T x, int P) {
+    if (P > 32) x = x + __shfl_down(x, 32, 64);
+    if (P > 16) x = x + __shfl_down(x, 16, 64);
+    if (P > 8) x = x + dpp_move<T, 0x108>(x);            // row_shl:8
+    if (P > 4) x = x + dpp_move<T, 0x104>(x);
+    if (P > 2) x = x + dpp_move<T, 0x102>(x);
+    if (P > 1) x = x + dpp_move<T, 0x101>(x);
     return x;
 }
 
-// The 64 group values' tree over Q = 2^ceil(log2 used) of them, in the first wave.
-template <class T>
-__device__ __forceinline__ T group_tree(const T* gp, int used) {
-    const int t = threadIdx.x;
-    const int q = pow2_at_least(used);
-    T x = t < used ? gp[t] : T(0);
+// 64 J consecutive values from u, `left` of them live: lane l's x[j] is value
+// l + 64 j, or +0.0 past the live ones.  A whole run loads without a test a
+// value: testing each took 16384 keys of 4096 rows from 75 to 110 us.
+template <class T, int J>
+__device__ __forceinline__ void wave_rows(T (&x)[J], const T* __restrict__ u, long long left) {
+    const int lane = threadIdx.x & 63;
+    if (left >= 64 * J) {
 #pragma unroll
-    for (int w = 32; w >= 1; w >>= 1) {
-        const T y = __shfl_down(x, w, 64);
-        if (q > w) x = x + y;
+        for (int j = 0; j < J; ++j) x[j] = __builtin_nontemporal_load(u + lane + 64 * j);
+        return;
     }
-    return x;
+    const int most = static_cast<int>(left);
+#pragma unroll
+    for (int j = 0; j < J; ++j) x[j] = lane + 64 * j < most ? __builtin_nontemporal_load(u + lane + 64 * j) : T(0);
 }
 
-// One workgroup per key whose lanes are already folded into `lanes` (groups
-// of more than 65536 rows): the used groups' trees, then the group values'.
-template <class T>
-__global__ __launch_bounds__(256) void hawk_keyed_fold(const T* __restrict__ lanes, long long lv,
-                                                       T* __restrict__ out) {
-    __shared__ T sh[256];
-    __shared__ T gp[kGroups];
-    const long long k = blockIdx.x;
-    const int t = threadIdx.x;
-    const int used = static_cast<int>((lv + kFoldLanes - 1) / kFoldLanes);     // <= 64
-    const int width = lv >= kFoldLanes ? kFoldLanes : pow2_at_least(lv);
-    const T* mine = lanes + k * lv;
-    for (int g = 0; g < used; ++g) {
-        T v[4];
+// The halving tree over 64 J values held as wave_rows holds them: the levels
+// from 32 J down to 64 join registers and the rest are wave_tree's, with no LDS
+// and no barrier.  Lane 0 returns the sum.
+template <class T, int J>
+__device__ __forceinline__ T rows_tree(T (&v)[J]) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const long long at = static_cast<long long>(g) * kFoldLanes + t + 256 * j;
-            v[j] = at < lv ? mine[at] : T(0);
-        }
-        const T s = block_tree<T>(v, width, sh);
-        if (t == 0) gp[g] = s;
-    }
-    __syncthreads();
-    const T total = t < 64 ? group_tree<T>(gp, used) : T(0);
-    if (t == 0) out[k] = total;
+    for (int off = J / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int j = 0; j < off; ++j) v[j] = v[j] + v[j + off];
+    return wave_tree(v[0], 64);
 }
 
-// One workgroup per key of at most 65536 rows: virtual lane l holds row l
-// alone (0.0 + u[l], the add from +0.0), so the trees read u directly.
-template <class T>
-__global__ __launch_bounds__(256) void hawk_keyed_rows(const T* __restrict__ u, long long group,
+// Keys of 65 to 1024 rows (64 J or fewer): a wave a key.  A workgroup a key
+// with the tree through LDS took 103 us where this takes 23 (100000 keys of 100
+// rows, fp64) and 25 where it takes 11.5 (20000 of 500: 7.0 TB/s).
+template <class T, int J>
+__global__ __launch_bounds__(256) void hawk_keyed_wave(const T* __restrict__ u, long long group, long long keys,
                                                        T* __restrict__ out) {
-    __shared__ T sh[256];
+    const long long k = static_cast<long long>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (k >= keys) return;                               // the whole wave
+    T v[J];
+    wave_rows<T, J>(v, u + k * group, group);
+#pragma unroll
+    for (int j = 0; j < J; ++j) v[j] = T(0) + v[j];
+    const T s = rows_tree<T, J>(v);
+    if ((threadIdx.x & 63) == 0) out[k] = s;
+}
+
+// Keys of at most 65536 rows: a workgroup a key, its waves the key's groups of
+// 1024 lanes in turn (the next group's rows in flight during a group's tree),
+// then the group values' tree in the first wave.  Four waves where the keys
+// fill the chip; sixteen for few keys of at most 16 groups, and for the plain
+// ordered sum of at most 16384 rows.
+template <class T, int Waves>
+__global__ __launch_bounds__(64 * Waves) void hawk_keyed_rows(const T* __restrict__ u, long long group,
+                                                              T* __restrict__ out) {
     __shared__ T gp[kGroups];
-    const long long k = blockIdx.x;
     const int t = threadIdx.x;
     const int used = static_cast<int>((group + kFoldLanes - 1) / kFoldLanes);
-    const int width = group >= kFoldLanes ? kFoldLanes : pow2_at_least(group);
-    const T* mine = u + k * group;
-    T nxt[4];                        // the next group's rows, loaded during this group's tree
+    const T* mine = u + static_cast<long long>(blockIdx.x) * group;
+    T x[16];
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    if (w < used) wave_rows<T, 16>(x, mine + w * kFoldLanes, group - w * kFoldLanes);
+    for (int g = w; g < used; g += Waves) {
+        T v[16];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const long long at = t + 256 * j;
-        nxt[j] = at < group ? __builtin_nontemporal_load(mine + at) : T(0);
-    }
-    for (int g = 0; g < used; ++g) {
-        T v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const long long at = static_cast<long long>(g) * kFoldLanes + t + 256 * j;
-            v[j] = at < group ? T(0) + nxt[j] : T(0);
-        }
-        if (g + 1 < used) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const long long at = static_cast<long long>(g + 1) * kFoldLanes + t + 256 * j;
-                nxt[j] = at < group ? __builtin_nontemporal_load(mine + at) : T(0);
-            }
-        }
-        const T s = block_tree<T>(v, width, sh);
-        if (t == 0) gp[g] = s;
+        for (int j = 0; j < 16; ++j) v[j] = T(0) + x[j];
+        if (g + Waves < used) wave_rows<T, 16>(x, mine + (g + Waves) * kFoldLanes, group - (g + Waves) * kFoldLanes);
+        const T s = rows_tree<T, 16>(v);
+        if ((t & 63) == 0) gp[g] = s;
     }
     __syncthreads();
-    const T total = t < 64 ? group_tree<T>(gp, used) : T(0);
-    if (t == 0) out[k] = total;
+    if (t < 64) {
+        const T total = wave_tree(t < used ? gp[t] : T(0), kGroups);
+        if (t == 0) out[blockIdx.x] = total;
+    }
+}
+
+// Longer keys, and few keys of more than 16 groups: a wave a (key, group),
+// virtual lane m adding rows m, m + 65536, ... (the next ones in flight), each
+// group's sum into gp[key][group]; then a wave a key for the group values'
+// tree.
+template <class T>
+__global__ __launch_bounds__(256) void hawk_keyed_groups(const T* __restrict__ u, long long group, int used,
+                                                         long long keys, T* __restrict__ gp) {
+    const long long i = static_cast<long long>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    const long long k = i / used, g = i % used;
+    if (k >= keys) return;                               // the whole wave
+    const T* mine = u + k * group + g * kFoldLanes;
+    const long long rows = group - g * kFoldLanes;
+    T x[16], v[16];
+    wave_rows<T, 16>(x, mine, rows);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = T(0);
+    for (long long r = 0; r < rows; r += kVirtualLanes) {
+        T a[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) a[j] = x[j];
+        if (r + kVirtualLanes < rows) wave_rows<T, 16>(x, mine + r + kVirtualLanes, rows - r - kVirtualLanes);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = v[j] + a[j];
+    }
+    const T s = rows_tree<T, 16>(v);
+    if ((threadIdx.x & 63) == 0) gp[k * kGroups + g] = s;
+}
+template <class T>
+__global__ __launch_bounds__(256) void hawk_keyed_top(const T* __restrict__ gp, int used, long long keys,
+                                                      T* __restrict__ out) {
+    const long long k = static_cast<long long>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (k >= keys) return;                               // the whole wave
+    const int lane = threadIdx.x & 63;
+    const T s = wave_tree(lane < used ? gp[k * kGroups + lane] : T(0), kGroups);
+    if (lane == 0) out[k] = s;
 }
 
 // Keys of at most 64 rows: a wave holds 64 / P keys, P = 2^ceil(log2 group),
 // in segments of P lanes (lane j of a segment holds row j, 0.0 + u, or +0.0
-// past the key's rows), and each segment runs the halving tree by shuffles
-// (lane j adds lane j + w for w = P/2 .. 1; only lanes below w carry on): the
-// pairs of the tree over P values.  The group tree has one value, which it
-// returns unchanged.
+// past the key's rows), and each segment runs the halving tree.  The group
+// tree has one value, which it returns unchanged.  A wave takes four such sets,
+// their loads in flight together.
+constexpr int kSmallSets = 4;
 template <class T>
 __global__ __launch_bounds__(256) void hawk_keyed_small(const T* __restrict__ u, long long group, int P,
                                                         long long keys, T* __restrict__ out) {
     const int lane = threadIdx.x & 63;
-    const long long per_wave = 64 / P;
-    const long long k = (static_cast<long long>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * per_wave + lane / P;
+    const int per_wave = 64 / P;
     const int j = lane & (P - 1);
-    T x = T(0);
-    if (k < keys && j < group) x = T(0) + __builtin_nontemporal_load(u + k * group + j);
+    const long long k0 = (static_cast<long long>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * (kSmallSets * per_wave) +
+                         lane / P;
+    T x[kSmallSets];
 #pragma unroll
-    for (int w = 32; w >= 1; w >>= 1) {
-        const T y = __shfl_down(x, w, 64);
-        if (P > w) x = x + y;
+    for (int q = 0; q < kSmallSets; ++q) {
+        const long long k = k0 + q * per_wave;
+        x[q] = k < keys && j < group ? T(0) + __builtin_nontemporal_load(u + k * group + j) : T(0);
     }
-    if (j == 0 && k < keys) out[k] = x;
+#pragma unroll
+    for (int q = 0; q < kSmallSets; ++q) x[q] = wave_tree(x[q], P);
+#pragma unroll
+    for (int q = 0; q < kSmallSets; ++q)
+        if (j == 0 && k0 + q * per_wave < keys) out[k0 + q * per_wave] = x[q];
 }
 
 // ---------------------------------------------------------------------------
@@ -2027,7 +2057,17 @@ int scratch_of(hipStream_t stream, void** out) {
     return HK_OK;
 }
 
-// The ordered sum in T (hk_ordered_sum_f64 / _f32): the lanes, then the fold.
+// Fewer keys than this leave CUs idle at four waves a key; below a quarter of
+// it long keys go group by group (10 keys of 60000 rows: 40 us a workgroup a
+// key, 7.4 group by group; 400 of 20000: 12 a workgroup a key).
+constexpr long long kFewKeys = 512;
+// The rows a sixteen-wave workgroup sums in one launch: a group of 1024 a wave
+// (1000 rows: 7.1 us as lanes and fold, 4.6 in one launch; 60000 rows, four
+// groups a wave: 7.1 and 9.8).
+constexpr long long kOneLaunchRows = 16 * kFoldLanes;
+
+// The ordered sum in T (hk_ordered_sum_f64 / _f32): the lanes, then the fold;
+// up to kOneLaunchRows rows one launch of the keyed sum's kernel.
 // A float sum keeps the double layout's offsets, its data in the front of
 // each region.
 template <class T>
@@ -2040,6 +2080,10 @@ int ordered_sum(const T* u, int64_t n, T* out, void* scratch, void* stream, cons
     auto* gp = reinterpret_cast<T*>(base + kLanesBytes);
     auto* ticket = reinterpret_cast<unsigned*>(base + kLanesBytes + kGpBytes);
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (n <= kOneLaunchRows) {
+        hipLaunchKernelGGL((hawk_keyed_rows<T, 16>), dim3(1), dim3(1024), 0, s, u, static_cast<long long>(n), out);
+        return launch_error("hawk_keyed_rows launch");
+    }
     hipLaunchKernelGGL(hawk_sum_lanes<T>, dim3(kVirtualLanes / kLaneBlock), dim3(kLaneBlock), 0, s, u,
                        static_cast<long long>(n), lanes, ticket);
     int rc = launch_error("hawk_sum_lanes launch");
@@ -2062,29 +2106,40 @@ int keyed_ordered_sum(const T* u, int64_t n, int64_t group, T* out, void* scratc
     const long long keys = n / group;
     if (keys > 0x7fffffffLL) return hawk_internal::set_error(HK_EVALUE, who + ": too many keys");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const long long len = group;
+    auto blocks_of = [](long long waves) { return dim3(static_cast<unsigned>((waves + 3) / 4)); };
     if (group <= 64) {
         const int P = pow2_at_least(group);
-        const long long waves = (keys + 64 / P - 1) / (64 / P);
-        hipLaunchKernelGGL(hawk_keyed_small<T>, dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0, s, u,
-                           static_cast<long long>(group), P, keys, out);
+        const long long per_wave = kSmallSets * (64 / P);
+        hipLaunchKernelGGL(hawk_keyed_small<T>, blocks_of((keys + per_wave - 1) / per_wave), dim3(256), 0, s, u, len, P,
+                           keys, out);
         return launch_error("hawk_keyed_small launch");
     }
-    if (group <= kVirtualLanes) {
-        hipLaunchKernelGGL(hawk_keyed_rows<T>, dim3(static_cast<unsigned>(keys)), dim3(256), 0, s, u,
-                           static_cast<long long>(group), out);
+    if (group <= kFoldLanes) {
+        const dim3 grid = blocks_of(keys);
+        if (group <= 128) hipLaunchKernelGGL((hawk_keyed_wave<T, 2>), grid, dim3(256), 0, s, u, len, keys, out);
+        else if (group <= 256) hipLaunchKernelGGL((hawk_keyed_wave<T, 4>), grid, dim3(256), 0, s, u, len, keys, out);
+        else if (group <= 512) hipLaunchKernelGGL((hawk_keyed_wave<T, 8>), grid, dim3(256), 0, s, u, len, keys, out);
+        else hipLaunchKernelGGL((hawk_keyed_wave<T, 16>), grid, dim3(256), 0, s, u, len, keys, out);
+        return launch_error("hawk_keyed_wave launch");
+    }
+    if (group <= (keys < kFewKeys / 4 ? kOneLaunchRows : kVirtualLanes)) {
+        const dim3 grid(static_cast<unsigned>(keys));
+        if (keys < kFewKeys && group <= kOneLaunchRows)
+            hipLaunchKernelGGL((hawk_keyed_rows<T, 16>), grid, dim3(1024), 0, s, u, len, out);
+        else
+            hipLaunchKernelGGL((hawk_keyed_rows<T, 4>), grid, dim3(256), 0, s, u, len, out);
         return launch_error("hawk_keyed_rows launch");
     }
-    const long long lv = group < kVirtualLanes ? group : kVirtualLanes;
-    const long long total = keys * lv;
-    auto* lanes = static_cast<T*>(scratch);
-    long long blocks = (total + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(hawk_keyed_lanes<T>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, u,
-                       static_cast<long long>(group), lv, total, lanes);
-    int rc = launch_error("hawk_keyed_lanes launch");
+    auto* gp = static_cast<T*>(scratch);
+    const long long used = (group + kFoldLanes - 1) / kFoldLanes < kGroups ? (group + kFoldLanes - 1) / kFoldLanes
+                                                                           : kGroups;
+    hipLaunchKernelGGL(hawk_keyed_groups<T>, blocks_of(keys * used), dim3(256), 0, s, u, len, static_cast<int>(used),
+                       keys, gp);
+    int rc = launch_error("hawk_keyed_groups launch");
     if (rc != HK_OK) return rc;
-    hipLaunchKernelGGL(hawk_keyed_fold<T>, dim3(static_cast<unsigned>(keys)), dim3(256), 0, s, lanes, lv, out);
-    return launch_error("hawk_keyed_fold launch");
+    hipLaunchKernelGGL(hawk_keyed_top<T>, blocks_of(keys), dim3(256), 0, s, gp, static_cast<int>(used), keys, out);
+    return launch_error("hawk_keyed_top launch");
 }
 
 // The rows' finish in T: the leaves, then the levels into *out.
@@ -2130,9 +2185,6 @@ int rows_extreme(const T* hi, int64_t rows, int32_t op, T* out, void* scratch, v
         hipLaunchKernelGGL((hawk_rows_ext_levels<T, 2>), dim3(1), dim3(256), 0, s, buf, leaves, out);
     return launch_error("hawk_rows_ext_levels launch");
 }
-
-// Fewer keys than this leave CUs idle at four waves a key.
-constexpr long long kFewKeys = 512;
 
 // The keyed default-policy sum in T (hk_keyed_sample_sum_f64 / _f32).
 template <class T>
@@ -2327,9 +2379,8 @@ int hk_ordered_sum_f64_noalloc(const double* u, int64_t n, double* out, void* st
 size_t hk_keyed_ordered_sum_scratch_bytes(int64_t n, int64_t group) {
     if (n <= 0 || group <= 0 || n % group != 0) return 0;
     if (n == group) return kSumScratch;
-    if (group <= kVirtualLanes) return 256;                  // the keys read their rows directly
-    const long long lv = group < kVirtualLanes ? group : kVirtualLanes;
-    return sizeof(double) * static_cast<size_t>(n / group) * static_cast<size_t>(lv) + 256;
+    if (group <= kOneLaunchRows) return 256;                 // the keys read their rows directly
+    return sizeof(double) * static_cast<size_t>(n / group) * kGroups + 256;
 }
 
 int hk_keyed_ordered_sum_f64(const double* u, int64_t n, int64_t group, double* out, void* scratch, void* stream) {

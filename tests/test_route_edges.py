@@ -121,3 +121,26 @@ def test_keyed_default_sum_routes(tmp_path, gpu, mode, keys, group):
     got = out.cpu().numpy()
     nan = np.isnan(want)
     assert (np.isnan(got) == nan).all() and got[~nan].tobytes() == want[~nan].tobytes()
+
+
+@pytest.mark.parametrize("mode", ["float64", "float32"])
+@pytest.mark.parametrize("keys, group", [
+    (9, 1), (70, 3), (257, 16), (5, 17), (7, 33), (1025, 64), (5, 65), (9, 128), (5, 129), (6, 256), (5, 257),
+    (7, 512), (5, 513), (3, 1023), (5, 1024), (5, 1025), (511, 2047), (512, 2047), (2, 65_536), (2, 65_537),
+    (3, 131_073), (1, 1), (1, 1000), (1, 65_536), (1, 65_537), (1, 65_536 * 9 + 5), (1, 65_536 * 40 - 1)])
+def test_ordered_sum_routes(tmp_path, gpu, mode, keys, group):
+    """Keyed and plain ordered sums at the edges of their kernels: the fixed
+    tree's bits per key, with infinities and signed zeros among the values."""
+    import hawk_amd as hawk
+    import oracle_lib as O
+    import torch
+    dt = np.float32 if mode == "float32" else np.float64
+    g = np.random.default_rng(keys * 11 + group)
+    x = (g.normal(size=keys * group) * 2.0 ** g.integers(-20, 20, keys * group)).astype(dt)
+    x[g.random(x.size) < 0.1] = -0.0
+    if keys > 2:
+        x[group // 2] = np.inf
+    (k,) = _unit(tmp_path, [_per_key(group, "ordered")], mode)
+    out = torch.full((keys,), 7.0, dtype=torch.float32 if mode == "float32" else torch.float64, device=gpu)
+    hawk.run(k, x=torch.from_numpy(x).to(gpu), out=out)
+    assert out.cpu().numpy().tobytes() == O.keyed_ordered_sum(x, group).tobytes()
