@@ -2380,7 +2380,9 @@ size_t hk_keyed_ordered_sum_scratch_bytes(int64_t n, int64_t group) {
     if (n <= 0 || group <= 0 || n % group != 0) return 0;
     if (n == group) return kSumScratch;
     if (group <= kOneLaunchRows) return 256;                 // the keys read their rows directly
-    return sizeof(double) * static_cast<size_t>(n / group) * kGroups + 256;
+    // group values (the entry's size for longer keys, a lane partial each, holds them too)
+    return sizeof(double) * static_cast<size_t>(n / group) *
+               static_cast<size_t>(group > kVirtualLanes ? kVirtualLanes : kGroups) + 256;
 }
 
 int hk_keyed_ordered_sum_f64(const double* u, int64_t n, int64_t group, double* out, void* scratch, void* stream) {
