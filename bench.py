@@ -292,8 +292,7 @@ def workload(config: str, device):
         cells = {c: torch.zeros(1, dtype=torch.float64, device=device) for c in ("s", "s_sq", "s_ord")}
         kernels = [k.prepare(x=X, **cells)]
         rows = 16 / 32                          # a (hi, lo) band row per 32 samples
-        work = {"band_total": (8 + 2 * rows, 0), "row_sum": (rows, 1), "row_sum#2": (rows, 1),
-                "band_ordered_sum": (8, 1)}
+        work = {"band_total": (8 + 2 * rows, 0), "row_sum": (2 * rows, 2), "band_ordered_sum": (8, 1)}
 
         def cpu(threads):
             import oracle_lib as O
@@ -314,8 +313,7 @@ def workload(config: str, device):
         cells = {c: torch.zeros(1, dtype=torch.float64, device=device) for c in ("s", "s_sq", "s_ord")}
         kernels = [k.prepare(x=X, **cells)]
         rows = 16 / 32                          # a (hi, comp) row per 32 samples
-        work = {"band_total": (8 + 2 * rows, 0), "row_sum": (rows, 1), "row_sum#2": (rows, 1),
-                "ordered_sum": (8, 1)}
+        work = {"band_total": (8 + 2 * rows, 0), "row_sum": (2 * rows, 2), "ordered_sum": (8, 1)}
 
         def cpu(threads):
             import oracle_lib as O

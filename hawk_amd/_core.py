@@ -64,6 +64,9 @@ def _declare(lib) -> None:
         "hk_ordered_scatter_scratch_bytes": (SZ, [I64, I64]),
         "hk_ordered_scatter_f64": (I, [V, V, I64, V, I64, V, V, V]),
         "hk_rows_finish_scratch_bytes": (SZ, [I64]),
+        "hk_rows_finish_many_scratch_bytes": (SZ, [I64, ctypes.c_int32]),
+        "hk_rows_finish_many_f64": (I, [V, ctypes.c_int32, I64, V, V]),
+        "hk_rows_finish_many_f32": (I, [V, ctypes.c_int32, I64, V, V]),
         "hk_rows_finish_f64": (I, [V, V, I64, V, V, V]),
         "hk_rows_finish_f32": (I, [V, V, I64, V, V, V]),
         "hk_rows_extreme_f64": (I, [V, I64, ctypes.c_int32, V, V, V]),
@@ -423,6 +426,27 @@ def rows_finish_f32(hi: int, comp: int, rows: int, out: int, scratch: int, strea
     """The same finish of float32 rows, in float32."""
     check(lib().hk_rows_finish_f32(ctypes.c_void_p(hi), ctypes.c_void_p(comp), int(rows), ctypes.c_void_p(out),
                                    ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+
+
+class RowsJob(ctypes.Structure):
+    """One reduction's rows, cell and rule (``hk_rows_job``)."""
+
+    _fields_ = [("hi", ctypes.c_void_p), ("lo", ctypes.c_void_p), ("out", ctypes.c_void_p), ("op", ctypes.c_int32)]
+
+
+#: ``RowsJob.op``: the default sum, the extremes, the banded sum.
+ROWS_SUM, ROWS_MAX, ROWS_MIN, ROWS_BAND = range(4)
+
+
+def rows_finish_many_scratch_bytes(rows: int, count: int) -> int:
+    return int(lib().hk_rows_finish_many_scratch_bytes(int(rows), int(count)))
+
+
+def rows_finish_many(jobs, rows: int, f32: bool, scratch: int, stream: int = 0) -> None:
+    """The finishes of every reduction of a stage (a ctypes array of
+    :class:`RowsJob`), in float32 or float64."""
+    fn = lib().hk_rows_finish_many_f32 if f32 else lib().hk_rows_finish_many_f64
+    check(fn(jobs, len(jobs), int(rows), ctypes.c_void_p(scratch), ctypes.c_void_p(stream)))
 
 
 def rows_extreme(hi: int, rows: int, op: int, out: int, scratch: int, stream: int = 0) -> None:

@@ -369,65 +369,155 @@ __device__ __forceinline__ void pair_add(T& h, T& c, T h2, T c2) {
     h = s;
 }
 
-// Leaf j: rows [j*4096, min((j+1)*4096, rows)).  T is the rows' type: the
-// finish runs in it, as the reference's finish runs in the rows' dtype.
-template <class T>
-__global__ __launch_bounds__(kRowSlots) void hawk_rows_leaves(const T* __restrict__ hi, const T* __restrict__ comp,
-                                                              long long rows, T* __restrict__ leaf_h,
-                                                              T* __restrict__ leaf_c) {
-    __shared__ T sh[kRowSlots], sc[kRowSlots];
+// A reduction's finish: its rows (hi, and comp or a band's low parts), its cell
+// and its rule.  Every reduction of a stage has the same number of rows, so one
+// launch folds the leaves of all of them and one their levels (one launch in
+// all where the rows are a single leaf): five reductions of a stage took ten
+// launches, 9 to 10 us a reduction.
+enum RowsOp { kRowsSum = 0, kRowsMax = 1, kRowsMin = 2, kRowsBand = 3 };
+struct RowsJob {
+    const void* hi;
+    const void* lo;
+    void* out;
+    int op;
+};
+constexpr int kRowsJobs = 16;                    // reductions a launch takes
+struct RowsJobs {
+    RowsJob job[kRowsJobs];
+};
+
+// The rule of each reduction over partials (h, c): `first` of a slot's first
+// row, `add` of a further row, `join` of two partials, and the cell's `value`.
+//
+// * the default sum: Neumaier's add and the compensated join (above);
+// * hawk.max / hawk.min (reference hawk/_cells.py:66-71 and `finish`): every
+//   add the extreme a > b ? a : b (max) or a < b ? a : b (min) of (the earlier
+//   partial, the later); exact, and a NaN partial on the left gives way to the
+//   right one;
+// * the banded sum: every add a band add, the cell the final band's h.
+template <class T, int Op>
+struct RowsRule {
+    __device__ static __forceinline__ T first_c(T h, T c) { return Op == kRowsSum && !finite_bits(h) ? T(0) : c; }
+    __device__ static __forceinline__ void add(T& h, T& c, T x, T xc) {
+        if constexpr (Op == kRowsSum) neumaier_add(h, c, x, xc);
+        else join(h, c, x, xc);
+    }
+    __device__ static __forceinline__ void join(T& h, T& c, T h2, T c2) {
+        if constexpr (Op == kRowsSum) {
+            pair_add(h, c, h2, c2);
+        } else if constexpr (Op == kRowsBand) {
+            const Band b = band_add(Band{h, c}, Band{h2, c2});
+            h = b.h;
+            c = b.l;
+        } else {
+            h = Op == kRowsMax ? (h > h2 ? h : h2) : (h < h2 ? h : h2);
+        }
+    }
+    __device__ static __forceinline__ T value(T h, T c) { return Op == kRowsSum && finite_bits(h) ? h + c : h; }
+};
+
+// Leaf j of a reduction: rows [j*4096, min((j+1)*4096, rows)), thread = slot.
+// T is the rows' type: the finish runs in it, as the reference's finish runs in
+// the rows' dtype.  A slot's sixteen rows load together, then add in order; the
+// tree's levels 128 and 64 cross waves through LDS, 32 .. 1 run in one wave.  A
+// slot past the rows joins nothing.
+template <class T, int Op>
+__device__ __forceinline__ void rows_leaf(const RowsJob& job, long long rows, T* buf, long long leaves, T* sh, T* sc) {
+    typedef RowsRule<T, Op> Rule;
+    constexpr bool kPair = Op == kRowsSum || Op == kRowsBand;
     const int s = threadIdx.x;
     const long long lo = static_cast<long long>(blockIdx.x) * kRowLeaf;
+    const T* hi = static_cast<const T*>(job.hi) + lo;
+    const T* comp = kPair ? static_cast<const T*>(job.lo) + lo : nullptr;
     const long long rest = rows - lo;
     const int cnt = rest < kRowLeaf ? static_cast<int>(rest) : static_cast<int>(kRowLeaf);
     const int live = cnt < kRowSlots ? cnt : kRowSlots;
-    if (s < live) {
-        T h = hi[lo + s];
-        T c = finite_bits(h) ? comp[lo + s] : T(0);
-        for (int k = 1; k < kRowTerms; ++k) {
-            const int m = live < cnt - k * kRowSlots ? live : cnt - k * kRowSlots;
-            if (m <= 0 || s >= m) break;
-            neumaier_add(h, c, hi[lo + k * kRowSlots + s], comp[lo + k * kRowSlots + s]);
+    T x[kRowTerms], y[kRowTerms];
+#pragma unroll
+    for (int k = 0; k < kRowTerms; ++k) x[k] = y[k] = T(0);
+    if (cnt == kRowLeaf) {
+#pragma unroll
+        for (int k = 0; k < kRowTerms; ++k) {
+            x[k] = hi[k * kRowSlots + s];
+            if constexpr (kPair) y[k] = comp[k * kRowSlots + s];
         }
-        sh[s] = h;
-        sc[s] = c;
+    } else {
+#pragma unroll
+        for (int k = 0; k < kRowTerms; ++k)
+            if (k * kRowSlots + s < cnt) {
+                x[k] = hi[k * kRowSlots + s];
+                if constexpr (kPair) y[k] = comp[k * kRowSlots + s];
+            }
     }
-    __syncthreads();
-    for (int off = kRowSlots / 2; off > 0; off >>= 1) {
-        const int lim = live > off ? (off < live - off ? off : live - off) : 0;
-        if (s < lim) {
-            T h = sh[s], c = sc[s];
-            pair_add(h, c, sh[s + off], sc[s + off]);
+    T h = x[0], c = Rule::first_c(x[0], y[0]);
+#pragma unroll
+    for (int k = 1; k < kRowTerms; ++k)
+        if (k * kRowSlots + s < cnt) Rule::add(h, c, x[k], y[k]);
+    auto lim = [&](int off) { return live > off ? (off < live - off ? off : live - off) : 0; };
+#pragma unroll
+    for (int off = kRowSlots / 2; off > 32; off >>= 1) {
+        if (s >= off && s < 2 * off) {
             sh[s] = h;
             sc[s] = c;
         }
         __syncthreads();
+        if (s < lim(off)) Rule::join(h, c, sh[s + off], sc[s + off]);
     }
-    if (s == 0) {
-        leaf_h[blockIdx.x] = sh[0];
-        leaf_c[blockIdx.x] = sc[0];
+    if (s >= 64) return;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const T h2 = __shfl_down(h, off, 64), c2 = __shfl_down(c, off, 64);
+        if (s < lim(off)) Rule::join(h, c, h2, c2);
+    }
+    if (s != 0) return;
+    if (leaves == 1) {
+        *static_cast<T*>(job.out) = Rule::value(h, c);
+    } else {
+        buf[blockIdx.x] = h;
+        buf[leaves + blockIdx.x] = c;
     }
 }
 
-// The leaves folded pairwise level by level by one workgroup, ping-ponging
-// between the two halves of the scratch; the cell gets hi + comp (hi alone
-// when it is not finite).
+// The rows' rule picked once a workgroup; the band rule is double only.
+#define HK_ROWS_RULE(op, call)                                  \
+    if ((op) == kRowsSum) call(kRowsSum);                       \
+    else if ((op) == kRowsMax) call(kRowsMax);                  \
+    else if ((op) == kRowsMin) call(kRowsMin);                  \
+    else if constexpr (sizeof(T) == 8) call(kRowsBand)
+
 template <class T>
-__global__ __launch_bounds__(256) void hawk_rows_levels(T* __restrict__ buf, long long leaves, T* __restrict__ out) {
+__global__ __launch_bounds__(kRowSlots) void hawk_rows_leaves(RowsJobs jobs, long long rows, T* __restrict__ buf,
+                                                              long long leaves) {
+    __shared__ T sh[kRowSlots], sc[kRowSlots];
+    const RowsJob job = jobs.job[blockIdx.y];
+    T* mine = buf + 4 * leaves * blockIdx.y;
+#define HK_LEAF(op) rows_leaf<T, op>(job, rows, mine, leaves, sh, sc)
+    HK_ROWS_RULE(job.op, HK_LEAF);
+#undef HK_LEAF
+}
+
+// The leaves folded pairwise level by level by one workgroup a reduction: in
+// the scratch's two halves while they are more than kLevelLds, then in LDS, the
+// last 128 by one wave with no barrier.
+constexpr int kLevelLds = 1024;
+template <class T, int Op>
+__device__ __forceinline__ void rows_levels(const RowsJob& job, T* buf, long long leaves, T* sh, T* sc) {
+    typedef RowsRule<T, Op> Rule;
+    const int t = threadIdx.x;
     T* vh = buf;
     T* vc = buf + leaves;
     T* nh = buf + 2 * leaves;
     T* nc = buf + 3 * leaves;
     long long m = leaves;
-    while (m > 1) {
+    while (m > kLevelLds) {
         const long long pairs = m / 2;
-        for (long long p = threadIdx.x; p < pairs; p += 256) {
+        for (long long p = t; p < pairs; p += 256) {
             T h = vh[2 * p], c = vc[2 * p];
-            pair_add(h, c, vh[2 * p + 1], vc[2 * p + 1]);
+            Rule::join(h, c, vh[2 * p + 1], vc[2 * p + 1]);
             nh[p] = h;
             nc[p] = c;
         }
-        if ((m & 1) && threadIdx.x == 0) {
+        if ((m & 1) && t == 0) {
             nh[pairs] = vh[m - 1];
             nc[pairs] = vc[m - 1];
         }
@@ -436,121 +526,72 @@ __global__ __launch_bounds__(256) void hawk_rows_levels(T* __restrict__ buf, lon
         T* tc = vc; vc = nc; nc = tc;
         m = pairs + (m & 1);
     }
-    if (threadIdx.x == 0) *out = finite_bits(vh[0]) ? vh[0] + vc[0] : vh[0];
-}
-
-// The rows' finish of hawk.max / hawk.min (reference hawk/_cells.py:66-71 and
-// `finish`): the same tree, every add the extreme a > b ? a : b (max) or
-// a < b ? a : b (min) of (the earlier partial, the later); exact, and a NaN
-// partial on the left gives way to the right one.  OP 1 is max, 2 min.
-template <int OP, class T>
-__device__ __forceinline__ T tree_extreme(T a, T b) {
-    return OP == 1 ? (a > b ? a : b) : (a < b ? a : b);
-}
-
-template <class T, int OP>
-__global__ __launch_bounds__(kRowSlots) void hawk_rows_ext_leaves(const T* __restrict__ hi, long long rows,
-                                                                  T* __restrict__ leaf_h) {
-    __shared__ T sh[kRowSlots];
-    const int s = threadIdx.x;
-    const long long lo = static_cast<long long>(blockIdx.x) * kRowLeaf;
-    const long long rest = rows - lo;
-    const int cnt = rest < kRowLeaf ? static_cast<int>(rest) : static_cast<int>(kRowLeaf);
-    const int live = cnt < kRowSlots ? cnt : kRowSlots;
-    if (s < live) {
-        T h = hi[lo + s];
-        for (int k = 1; k < kRowTerms; ++k) {
-            const int m = live < cnt - k * kRowSlots ? live : cnt - k * kRowSlots;
-            if (m <= 0 || s >= m) break;
-            h = tree_extreme<OP>(h, hi[lo + k * kRowSlots + s]);
-        }
-        sh[s] = h;
+    for (int p = t; p < m; p += 256) {
+        sh[p] = vh[p];
+        sc[p] = vc[p];
     }
     __syncthreads();
-    for (int off = kRowSlots / 2; off > 0; off >>= 1) {
-        const int lim = live > off ? (off < live - off ? off : live - off) : 0;
-        if (s < lim) sh[s] = tree_extreme<OP>(sh[s], sh[s + off]);
-        __syncthreads();
-    }
-    if (s == 0) leaf_h[blockIdx.x] = sh[0];
-}
-
-template <class T, int OP>
-__global__ __launch_bounds__(256) void hawk_rows_ext_levels(T* __restrict__ buf, long long leaves,
-                                                            T* __restrict__ out) {
-    T* vh = buf;
-    T* nh = buf + leaves;
-    long long m = leaves;
-    while (m > 1) {
-        const long long pairs = m / 2;
-        for (long long p = threadIdx.x; p < pairs; p += 256) nh[p] = tree_extreme<OP>(vh[2 * p], vh[2 * p + 1]);
-        if ((m & 1) && threadIdx.x == 0) nh[pairs] = vh[m - 1];
-        __syncthreads();
-        T* th = vh; vh = nh; nh = th;
-        m = pairs + (m & 1);
-    }
-    if (threadIdx.x == 0) *out = vh[0];
-}
-
-// The banded rows' finish: the canonical tree above (leaves of 4096 rows over
-// 256 slots, the in-leaf halving tree, the leaves pairwise level by level)
-// with every add a band add; the cell is the final band's h.  Row r of the
-// stage is the band (hi[r], lo[r]).
-__global__ __launch_bounds__(kRowSlots) void hawk_band_rows_leaves(const double* __restrict__ hi,
-                                                                   const double* __restrict__ lo, long long rows,
-                                                                   double* __restrict__ leaf_h,
-                                                                   double* __restrict__ leaf_l) {
-    __shared__ Band sh[kRowSlots];
-    const int s = threadIdx.x;
-    const long long first = static_cast<long long>(blockIdx.x) * kRowLeaf;
-    const long long rest = rows - first;
-    const int cnt = rest < kRowLeaf ? static_cast<int>(rest) : static_cast<int>(kRowLeaf);
-    const int live = cnt < kRowSlots ? cnt : kRowSlots;
-    if (s < live) {
-        Band b{hi[first + s], lo[first + s]};
-        for (int k = 1; k < kRowTerms; ++k) {
-            const int m = live < cnt - k * kRowSlots ? live : cnt - k * kRowSlots;
-            if (m <= 0 || s >= m) break;
-            b = band_add(b, Band{hi[first + k * kRowSlots + s], lo[first + k * kRowSlots + s]});
-        }
-        sh[s] = b;
-    }
-    __syncthreads();
-    for (int off = kRowSlots / 2; off > 0; off >>= 1) {
-        const int lim = live > off ? (off < live - off ? off : live - off) : 0;
-        if (s < lim) sh[s] = band_add(sh[s], sh[s + off]);
-        __syncthreads();
-    }
-    if (s == 0) {
-        leaf_h[blockIdx.x] = sh[0].h;
-        leaf_l[blockIdx.x] = sh[0].l;
-    }
-}
-
-__global__ __launch_bounds__(256) void hawk_band_rows_levels(double* __restrict__ buf, long long leaves,
-                                                             double* __restrict__ out) {
-    double* vh = buf;
-    double* vl = buf + leaves;
-    double* nh = buf + 2 * leaves;
-    double* nl = buf + 3 * leaves;
-    long long m = leaves;
-    while (m > 1) {
-        const long long pairs = m / 2;
-        for (long long p = threadIdx.x; p < pairs; p += 256) {
-            const Band b = band_add(Band{vh[2 * p], vl[2 * p]}, Band{vh[2 * p + 1], vl[2 * p + 1]});
-            nh[p] = b.h;
-            nl[p] = b.l;
-        }
-        if ((m & 1) && threadIdx.x == 0) {
-            nh[pairs] = vh[m - 1];
-            nl[pairs] = vl[m - 1];
+    int left = static_cast<int>(m);
+    while (left > 128) {
+        const int pairs = left / 2;
+        T h[kLevelLds / 512], c[kLevelLds / 512];
+#pragma unroll
+        for (int q = 0; q < kLevelLds / 512; ++q) {
+            const int p = t + 256 * q;
+            if (p < pairs) {
+                h[q] = sh[2 * p];
+                c[q] = sc[2 * p];
+                Rule::join(h[q], c[q], sh[2 * p + 1], sc[2 * p + 1]);
+            } else if (p == pairs && (left & 1)) {
+                h[q] = sh[left - 1];
+                c[q] = sc[left - 1];
+            }
         }
         __syncthreads();
-        double* th = vh; vh = nh; nh = th;
-        double* tl = vl; vl = nl; nl = tl;
-        m = pairs + (m & 1);
+#pragma unroll
+        for (int q = 0; q < kLevelLds / 512; ++q) {
+            const int p = t + 256 * q;
+            if (p < pairs + (left & 1)) {
+                sh[p] = h[q];
+                sc[p] = c[q];
+            }
+        }
+        __syncthreads();
+        left = pairs + (left & 1);
     }
-    if (threadIdx.x == 0) *out = vh[0];
+    if (t >= 64) return;
+    while (left > 1) {                       // a lane a pair; the wave's reads precede its writes
+        const int pairs = left / 2;
+        T h = T(0), c = T(0);
+        if (t < pairs) {
+            h = sh[2 * t];
+            c = sc[2 * t];
+            Rule::join(h, c, sh[2 * t + 1], sc[2 * t + 1]);
+        }
+        const T lh = sh[left - 1], lc = sc[left - 1];
+        __builtin_amdgcn_wave_barrier();
+        if (t < pairs) {
+            sh[t] = h;
+            sc[t] = c;
+        }
+        if ((left & 1) && t == 0) {
+            sh[pairs] = lh;
+            sc[pairs] = lc;
+        }
+        __builtin_amdgcn_wave_barrier();
+        left = pairs + (left & 1);
+    }
+    if (t == 0) *static_cast<T*>(job.out) = Rule::value(sh[0], sc[0]);
+}
+
+template <class T>
+__global__ __launch_bounds__(256) void hawk_rows_levels(RowsJobs jobs, T* __restrict__ buf, long long leaves) {
+    __shared__ T sh[kLevelLds], sc[kLevelLds];
+    const RowsJob job = jobs.job[blockIdx.x];
+    T* mine = buf + 4 * leaves * blockIdx.x;
+#define HK_LEVELS(op) rows_levels<T, op>(job, mine, leaves, sh, sc)
+    HK_ROWS_RULE(job.op, HK_LEVELS);
+#undef HK_LEVELS
 }
 
 // hawk.sum(x, over=<trailing lane axes>) under the default policy: key k's
@@ -2142,48 +2183,63 @@ int keyed_ordered_sum(const T* u, int64_t n, int64_t group, T* out, void* scratc
     return launch_error("hawk_keyed_top launch");
 }
 
-// The rows' finish in T: the leaves, then the levels into *out.
+// The finishes of `count` reductions of `rows` rows each, in T: the leaves of
+// all of them, then the levels (kRowsJobs reductions a launch).
 template <class T>
-int rows_finish(const T* hi, const T* comp, int64_t rows, T* out, void* scratch, void* stream, const char* name) {
-    if (rows < 1) return hawk_internal::set_error(HK_EVALUE, std::string(name) + ": rows must be >= 1");
-    if (!hi || !comp || !out || !scratch)
-        return hawk_internal::set_error(HK_EVALUE, std::string(name) + ": hi, comp, out and scratch are required");
-    const long long leaves = (rows + kRowLeaf - 1) / kRowLeaf;
-    if (leaves > 0x7fffffffLL) return hawk_internal::set_error(HK_EVALUE, std::string(name) + ": too many rows");
-    auto* buf = static_cast<T*>(scratch);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(hawk_rows_leaves<T>, dim3(static_cast<unsigned>(leaves)), dim3(kRowSlots), 0, s, hi, comp,
-                       static_cast<long long>(rows), buf, buf + leaves);
-    int rc = launch_error("hawk_rows_leaves launch");
-    if (rc != HK_OK) return rc;
-    hipLaunchKernelGGL(hawk_rows_levels<T>, dim3(1), dim3(256), 0, s, buf, leaves, out);
-    return launch_error("hawk_rows_levels launch");
-}
-
-// The rows' extreme in T (op 1 max, 2 min): the leaves, then the levels.
-template <class T>
-int rows_extreme(const T* hi, int64_t rows, int32_t op, T* out, void* scratch, void* stream, const char* name) {
+int rows_finish(const hk_rows_job* jobs, int count, int64_t rows, void* scratch, void* stream, const char* name) {
     const std::string who(name);
     if (rows < 1) return hawk_internal::set_error(HK_EVALUE, who + ": rows must be >= 1");
-    if (op != 1 && op != 2) return hawk_internal::set_error(HK_EVALUE, who + ": op must be 1 (max) or 2 (min)");
-    if (!hi || !out || !scratch) return hawk_internal::set_error(HK_EVALUE, who + ": hi, out and scratch are required");
+    if (count < 0 || (count > 0 && (!jobs || !scratch)))
+        return hawk_internal::set_error(HK_EVALUE, who + ": jobs and scratch are required");
+    for (int i = 0; i < count; ++i) {
+        const int32_t op = jobs[i].op;
+        if (op < kRowsSum || op > kRowsBand || (op == kRowsBand && sizeof(T) != 8))
+            return hawk_internal::set_error(HK_EVALUE, who + ": op must be 0 (sum), 1 (max), 2 (min) or, in float64, "
+                                                             "3 (band)");
+        if (!jobs[i].hi || !jobs[i].out || ((op == kRowsSum || op == kRowsBand) && !jobs[i].lo))
+            return hawk_internal::set_error(HK_EVALUE, who + ": a job's hi, lo (of a sum) and out are required");
+    }
     const long long leaves = (rows + kRowLeaf - 1) / kRowLeaf;
     if (leaves > 0x7fffffffLL) return hawk_internal::set_error(HK_EVALUE, who + ": too many rows");
-    auto* buf = static_cast<T*>(scratch);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (op == 1)
-        hipLaunchKernelGGL((hawk_rows_ext_leaves<T, 1>), dim3(static_cast<unsigned>(leaves)), dim3(kRowSlots), 0, s,
-                           hi, static_cast<long long>(rows), buf);
-    else
-        hipLaunchKernelGGL((hawk_rows_ext_leaves<T, 2>), dim3(static_cast<unsigned>(leaves)), dim3(kRowSlots), 0, s,
-                           hi, static_cast<long long>(rows), buf);
-    int rc = launch_error("hawk_rows_ext_leaves launch");
-    if (rc != HK_OK) return rc;
-    if (op == 1)
-        hipLaunchKernelGGL((hawk_rows_ext_levels<T, 1>), dim3(1), dim3(256), 0, s, buf, leaves, out);
-    else
-        hipLaunchKernelGGL((hawk_rows_ext_levels<T, 2>), dim3(1), dim3(256), 0, s, buf, leaves, out);
-    return launch_error("hawk_rows_ext_levels launch");
+    for (int first = 0; first < count; first += kRowsJobs) {
+        const int here = count - first < kRowsJobs ? count - first : kRowsJobs;
+        RowsJobs all{};
+        for (int i = 0; i < here; ++i)
+            all.job[i] = RowsJob{jobs[first + i].hi, jobs[first + i].lo, jobs[first + i].out, jobs[first + i].op};
+        T* buf = static_cast<T*>(scratch) + 4 * leaves * first;
+        hipLaunchKernelGGL(hawk_rows_leaves<T>, dim3(static_cast<unsigned>(leaves), static_cast<unsigned>(here)),
+                           dim3(kRowSlots), 0, s, all, static_cast<long long>(rows), buf, leaves);
+        int rc = launch_error("hawk_rows_leaves launch");
+        if (rc != HK_OK || leaves == 1) {
+            if (rc != HK_OK) return rc;
+            continue;
+        }
+        hipLaunchKernelGGL(hawk_rows_levels<T>, dim3(static_cast<unsigned>(here)), dim3(256), 0, s, all, buf, leaves);
+        rc = launch_error("hawk_rows_levels launch");
+        if (rc != HK_OK) return rc;
+    }
+    return HK_OK;
+}
+
+// One reduction's finish, refusing by its own entry's argument names.
+template <class T>
+int rows_finish_one(const T* hi, const T* lo, int32_t op, int64_t rows, T* out, void* scratch, void* stream,
+                    const char* name, const char* planes) {
+    const std::string who(name);
+    if (rows < 1) return hawk_internal::set_error(HK_EVALUE, who + ": rows must be >= 1");
+    if (!hi || !out || !scratch || ((op == kRowsSum || op == kRowsBand) && !lo))
+        return hawk_internal::set_error(HK_EVALUE, who + ": " + planes + ", out and scratch are required");
+    const hk_rows_job job{hi, lo, out, op};
+    return rows_finish<T>(&job, 1, rows, scratch, stream, name);
+}
+
+// The rows' extreme in T (op 1 max, 2 min).
+template <class T>
+int rows_extreme(const T* hi, int64_t rows, int32_t op, T* out, void* scratch, void* stream, const char* name) {
+    if (rows >= 1 && op != kRowsMax && op != kRowsMin)
+        return hawk_internal::set_error(HK_EVALUE, std::string(name) + ": op must be 1 (max) or 2 (min)");
+    return rows_finish_one<T>(hi, nullptr, op, rows, out, scratch, stream, name, "hi");
 }
 
 // The keyed default-policy sum in T (hk_keyed_sample_sum_f64 / _f32).
@@ -2409,12 +2465,12 @@ size_t hk_rows_finish_scratch_bytes(int64_t rows) {
 
 int hk_rows_finish_f64(const double* hi, const double* comp, int64_t rows, double* out, void* scratch,
                        void* stream) {
-    return rows_finish(hi, comp, rows, out, scratch, stream, "hk_rows_finish_f64");
+    return rows_finish_one<double>(hi, comp, kRowsSum, rows, out, scratch, stream, "hk_rows_finish_f64", "hi, comp");
 }
 
 int hk_rows_finish_f32(const float* hi, const float* comp, int64_t rows, float* out, void* scratch,
                        void* stream) {
-    return rows_finish(hi, comp, rows, out, scratch, stream, "hk_rows_finish_f32");
+    return rows_finish_one<float>(hi, comp, kRowsSum, rows, out, scratch, stream, "hk_rows_finish_f32", "hi, comp");
 }
 
 int hk_rows_extreme_f64(const double* hi, int64_t rows, int32_t op, double* out, void* scratch, void* stream) {
@@ -2429,19 +2485,19 @@ size_t hk_band_rows_finish_scratch_bytes(int64_t rows) { return hk_rows_finish_s
 
 int hk_band_rows_finish_f64(const double* hi, const double* lo, int64_t rows, double* out, void* scratch,
                             void* stream) {
-    if (rows < 1) return hawk_internal::set_error(HK_EVALUE, "hk_band_rows_finish_f64: rows must be >= 1");
-    if (!hi || !lo || !out || !scratch)
-        return hawk_internal::set_error(HK_EVALUE, "hk_band_rows_finish_f64: hi, lo, out and scratch are required");
-    const long long leaves = (rows + kRowLeaf - 1) / kRowLeaf;
-    if (leaves > 0x7fffffffLL) return hawk_internal::set_error(HK_EVALUE, "hk_band_rows_finish_f64: too many rows");
-    auto* buf = static_cast<double*>(scratch);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(hawk_band_rows_leaves, dim3(static_cast<unsigned>(leaves)), dim3(kRowSlots), 0, s, hi, lo,
-                       static_cast<long long>(rows), buf, buf + leaves);
-    int rc = launch_error("hawk_band_rows_leaves launch");
-    if (rc != HK_OK) return rc;
-    hipLaunchKernelGGL(hawk_band_rows_levels, dim3(1), dim3(256), 0, s, buf, leaves, out);
-    return launch_error("hawk_band_rows_levels launch");
+    return rows_finish_one<double>(hi, lo, kRowsBand, rows, out, scratch, stream, "hk_band_rows_finish_f64", "hi, lo");
+}
+
+size_t hk_rows_finish_many_scratch_bytes(int64_t rows, int32_t count) {
+    return count <= 0 ? 0 : hk_rows_finish_scratch_bytes(rows) * static_cast<size_t>(count);
+}
+
+int hk_rows_finish_many_f64(const hk_rows_job* jobs, int32_t count, int64_t rows, void* scratch, void* stream) {
+    return rows_finish<double>(jobs, count, rows, scratch, stream, "hk_rows_finish_many_f64");
+}
+
+int hk_rows_finish_many_f32(const hk_rows_job* jobs, int32_t count, int64_t rows, void* scratch, void* stream) {
+    return rows_finish<float>(jobs, count, rows, scratch, stream, "hk_rows_finish_many_f32");
 }
 
 size_t hk_band_ordered_sum_scratch_bytes(void) { return kBandSumScratch; }

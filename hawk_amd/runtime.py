@@ -33,6 +33,8 @@ def _bound_length(role: str, x, n: int) -> int:
     return int(x.shape[-1]) if role == "key_out" else n
 
 
+#: The team ops that fold the rows a stage writes (one launch set for them all).
+_ROW_OPS = ("row_sum", "band_rows", "row_extreme")
 _PER_SAMPLE = ("per_sample", "vec_in", "mat_in", "mutable", "out", "wide_out", "terminated")
 #: The per-sample roles a launch writes.
 _WRITTEN = ("mutable", "out", "wide_out", "terminated")
@@ -91,6 +93,7 @@ class DeviceKernel:
         self.name = sidecar["kernel"]
         self.planes = sidecar["planes"]
         self.team = sidecar.get("team") or []
+        self._row_ops = [t for t in self.team if t["op"] in _ROW_OPS]
         self.arg_spec = [tuple(p) for p in sidecar.get("arg_spec") or []]
         self.mode = sidecar.get("mode", "float64")
         self.launch_shape = sidecar.get("launch", {"block": 256, "per_thread": 1})
@@ -358,32 +361,34 @@ class DeviceKernel:
         cell (``hawk.sum`` of a vector commits one entry a column)."""
         return out.data_ptr() + (t.get("column") or 0) * out.element_size()
 
-    def _row_sum(self, t: dict, bound: dict, n: int, device, stream: int) -> None:
-        """Fold the stage's row partials into the cell: compensated (hi, comp)
-        rows, band rows (hi, lo) in the banded mode, or one extreme a row
-        (``hawk.max`` / ``hawk.min``).  A run of no samples leaves the
-        reduction's identity: 0, -inf (max), +inf (min)."""
-        out = bound[t["out"]]
+    def _row_finish_args(self, bound: dict, n: int, device, stream: int) -> tuple:
+        """``(jobs, rows, f32, scratch)`` of the finish of every reduction whose
+        rows the stage writes (:func:`hawk_amd._core.rows_finish_many`):
+        compensated (hi, comp) rows, band rows (hi, lo) in the banded mode, or
+        one extreme a row (``hawk.max`` / ``hawk.min``).  The rows are the
+        stage's Real, so the finish runs in it."""
         rows = -(-n // 32)
-        col = t.get("column")
-        if rows == 0:
-            empty = {"max": float("-inf"), "min": float("inf")}.get(t.get("red"), 0.0)
-            with _on(stream):
-                (out.view(-1)[col:col + 1] if col is not None else out).fill_(empty)
-            return
-        band = t["op"] == "band_rows"
-        f32 = self.planes[t["hi"]]["dtype"] == "f32"      # the rows are the stage's Real: the finish runs in it
+        jobs = (_core.RowsJob * len(self._row_ops))()
+        for job, t in zip(jobs, self._row_ops):
+            job.hi, job.out = bound[t["hi"]].data_ptr(), self._cell_ptr(t, bound[t["out"]])
+            if t["op"] == "row_extreme":
+                job.op = _core.ROWS_MAX if t["red"] == "max" else _core.ROWS_MIN
+            else:
+                job.lo = bound[t["comp"]].data_ptr()
+                job.op = _core.ROWS_BAND if t["op"] == "band_rows" else _core.ROWS_SUM
         with _on(stream):
-            nbytes = (_core.band_rows_finish_scratch_bytes if band else _core.rows_finish_scratch_bytes)(rows)
-            scratch = self._buffer(("rows", t["hi"], rows), nbytes, device, zero=False)
-        if t["op"] == "row_extreme":
-            (_core.rows_extreme_f32 if f32 else _core.rows_extreme)(
-                bound[t["hi"]].data_ptr(), rows, 1 if t["red"] == "max" else 2, self._cell_ptr(t, out),
-                scratch.data_ptr(), stream)
-            return
-        finish = _core.band_rows_finish if band else _core.rows_finish_f32 if f32 else _core.rows_finish
-        finish(bound[t["hi"]].data_ptr(), bound[t["comp"]].data_ptr(), rows, self._cell_ptr(t, out),
-               scratch.data_ptr(), stream)
+            scratch = self._buffer(("rows", rows), _core.rows_finish_many_scratch_bytes(rows, len(jobs)), device,
+                                   zero=False)
+        return jobs, rows, self.planes[self._row_ops[0]["hi"]]["dtype"] == "f32", scratch
+
+    def _row_identities(self, bound: dict, stream: int) -> None:
+        """A run of no samples leaves each reduction's identity: 0, -inf (max),
+        +inf (min)."""
+        with _on(stream):
+            for t in self._row_ops:
+                out, col = bound[t["out"]], t.get("column")
+                empty = {"max": float("-inf"), "min": float("inf")}.get(t.get("red"), 0.0)
+                (out.view(-1)[col:col + 1] if col is not None else out).fill_(empty)
 
     def _term_plane(self, name: str, n: int, device):
         torch = _torch()
@@ -541,8 +546,14 @@ class DeviceKernel:
             elif t["op"] == "mm16":
                 _core.mm16([bound[p].data_ptr() for p in t["in"]], [bound[p].data_ptr() for p in t["out"]],
                            t["products"], n, stream, t.get("dtype", "f32"))
-            elif t["op"] in ("row_sum", "band_rows", "row_extreme"):
-                self._row_sum(t, bound, n, device, stream)
+            elif t["op"] in _ROW_OPS:
+                if t is not self._row_ops[0]:
+                    continue                  # the first finishes them all
+                if n == 0:
+                    self._row_identities(bound, stream)
+                else:
+                    jobs, rows, f32, scratch = self._row_finish_args(bound, n, device, stream)
+                    _core.rows_finish_many(jobs, rows, f32, scratch.data_ptr(), stream)
             elif t["op"] == "band_ordered_sum":
                 u = bound[t["u"]]
                 scratch = self._buffer(("band_sum", t["out"]), _core.band_ordered_sum_scratch_bytes(), device,
@@ -888,8 +899,15 @@ class Prepared:
                 args = ([bound[p].data_ptr() for p in t["in"]], [bound[p].data_ptr() for p in t["out"]],
                         t["products"], self.n)
                 self.steps.append((_core.mm16_f64 if t.get("dtype") == "f64" else _core.mm16, args))
-            elif t["op"] in ("row_sum", "band_rows", "row_extreme"):
-                self.steps.append((kernel._row_sum, (t, bound, self.n, device)))
+            elif t["op"] in _ROW_OPS:
+                if t is not kernel._row_ops[0]:
+                    continue                  # the first finishes them all
+                if self.n == 0:
+                    self.steps.append((kernel._row_identities, (bound,)))
+                else:
+                    jobs, rows, f32, scratch = kernel._row_finish_args(bound, self.n, device, self.stream)
+                    self.rows_scratch = scratch          # alive as long as the launcher
+                    self.steps.append((_core.rows_finish_many, (jobs, rows, f32, scratch.data_ptr())))
             elif t["op"] == "band_ordered_sum":
                 scratch = kernel._buffer(("band_sum", t["out"]), _core.band_ordered_sum_scratch_bytes(), device,
                                          zero=False)

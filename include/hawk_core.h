@@ -249,6 +249,25 @@ int hk_rows_extreme_f64(const double* hi, int64_t rows, int32_t op, double* out,
 int hk_rows_extreme_f32(const float* hi, int64_t rows, int32_t op, float* out,
                         void* scratch, void* stream);
 
+/* The finishes of `count` reductions of one stage, each over `rows` rows, in
+ * two launches (one when the rows are a single leaf of 4096): job i folds its
+ * rows by op 0 (hk_rows_finish: hi and the compensations lo), 1 or 2
+ * (hk_rows_extreme: hi alone), or in float64 3 (hk_band_rows_finish: hi and
+ * lo), into *out, the bits of those entries.  Scratch:
+ * hk_rows_finish_many_scratch_bytes(rows, count) bytes, no initial contents
+ * needed.  HK_EVALUE for rows < 1, another op or a missing plane. */
+typedef struct hk_rows_job {
+    const void* hi;
+    const void* lo;
+    void* out;
+    int32_t op;
+} hk_rows_job;
+size_t hk_rows_finish_many_scratch_bytes(int64_t rows, int32_t count);
+int hk_rows_finish_many_f64(const hk_rows_job* jobs, int32_t count, int64_t rows,
+                            void* scratch, void* stream);
+int hk_rows_finish_many_f32(const hk_rows_job* jobs, int32_t count, int64_t rows,
+                            void* scratch, void* stream);
+
 /* Banded reductions: the sample sums of the banded scalar mode (reference
  * `hawk/emit/wrapper.py:140` BANDED and its row sum `:542-665`,
  * `hawk/emit/team.py:26-49` and `:225-245`: band partials folded in the
@@ -282,9 +301,10 @@ int hk_band_ordered_sum_f64(const double* u, int64_t n, double* out, void* scrat
  * a bad key was met: the caller reads status[1..256] (the reference's
  * `check_scatter_status`, `hawk/_lane_bind.py:148-154`).
  * Scratch: hk_ordered_scatter_scratch_bytes(n, cells) bytes, no initial
- * contents needed: the per-(chunk, cell) partials, then (for 12288 < cells
- * <= 65536) the bins that carry each tile's lanes of keys past the first
- * 12288 from the first walk to the second. */
+ * contents needed: the per-(chunk, cell) partials, then the bins that carry
+ * each tile's lanes from the first walk to the second (for 12288 < cells <=
+ * 65536 in many chunks, the lanes of keys past the first 12288; for few chunks
+ * or more cells, all of them; otherwise none). */
 int hk_scatter_chunks(int64_t n, int64_t cells);
 size_t hk_ordered_scatter_scratch_bytes(int64_t n, int64_t cells);
 int hk_ordered_scatter_f64(const int32_t* key, const double* v, int64_t n,

@@ -144,3 +144,42 @@ def test_ordered_sum_routes(tmp_path, gpu, mode, keys, group):
     out = torch.full((keys,), 7.0, dtype=torch.float32 if mode == "float32" else torch.float64, device=gpu)
     hawk.run(k, x=torch.from_numpy(x).to(gpu), out=out)
     assert out.cpu().numpy().tobytes() == O.keyed_ordered_sum(x, group).tobytes()
+
+
+@pytest.mark.parametrize("mode", ["float64", "float32"])
+@pytest.mark.parametrize("rows", [1, 255, 256, 257, 4095, 4096, 4097, 2 * 4096, 128 * 4096 + 1, 129 * 4096,
+                                  1024 * 4096, 1025 * 4096 + 17])
+def test_rows_finish_together(gpu, mode, rows):
+    """Every kind of reduction's rows finished in one call, at the edges of the
+    leaves and of the levels' forms: each the oracle's bits, NaN and infinities
+    included (seventeen jobs: more than one launch takes)."""
+    import oracle_lib as O
+    import torch
+    from hawk_amd import _core
+    f32 = mode == "float32"
+    dt = np.float32 if f32 else np.float64
+    g = np.random.default_rng(rows)
+    hi = (g.normal(size=rows) * 2.0 ** g.integers(-10, 10, rows)).astype(dt)
+    lo = (hi * g.uniform(-1, 1, rows) * (2.0 ** -25 if f32 else 2.0 ** -54)).astype(dt)
+    odd = hi.copy()
+    odd[g.integers(0, rows, 3)] = (np.nan, np.inf, -np.inf)
+    inf = hi.copy()
+    inf[rows // 2] = np.inf
+    planes = {k: torch.from_numpy(v).to(gpu) for k, v in (("hi", hi), ("lo", lo), ("odd", odd), ("inf", inf))}
+    finish = O.rows_finish_f32 if f32 else O.rows_finish
+    jobs = [("hi", _core.ROWS_SUM, finish(hi, lo)), ("odd", _core.ROWS_MAX, O.rows_extreme(odd, "max")),
+            ("odd", _core.ROWS_MIN, O.rows_extreme(odd, "min")), ("inf", _core.ROWS_SUM, finish(inf, lo))]
+    if not f32:
+        jobs.append(("hi", _core.ROWS_BAND, O.band_rows_finish(hi, lo)))
+    jobs += [jobs[i % 3] for i in range(17 - len(jobs))]
+    out = torch.full((len(jobs),), 7.0, dtype=planes["hi"].dtype, device=gpu)
+    call = (_core.RowsJob * len(jobs))()
+    for i, (plane, op, _want) in enumerate(jobs):
+        call[i].hi, call[i].lo, call[i].op = planes[plane].data_ptr(), planes["lo"].data_ptr(), op
+        call[i].out = out.data_ptr() + i * out.element_size()
+    scratch = torch.empty(_core.rows_finish_many_scratch_bytes(rows, len(jobs)), dtype=torch.uint8, device=gpu)
+    _core.rows_finish_many(call, rows, f32, scratch.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    got = out.cpu().numpy()
+    want = np.array([w for *_, w in jobs], dt)
+    nan = np.isnan(want)
+    assert (np.isnan(got) == nan).all() and got[~nan].tobytes() == want[~nan].tobytes()
