@@ -26,8 +26,11 @@ constexpr int kVirtualLanes = 65536;   // reference hawk/emit/team.py:21-23
 constexpr int kFoldLanes = 1024;
 constexpr int kGroups = 64;            // reference hawk/ir/team.py:649 GROUPS
 constexpr int kLaneBlock = 256;
-constexpr int kSumUnroll = 32;
-constexpr int kSumTail = 8;
+// Rows a lane keeps in flight twice over: 32 in float64, 64 in float32 (with 32,
+// a float sum of 2^26 rows took 58 us, with 64 47, one batch at a time 88), 8
+// up to that many rows (testing 64 loads that read nothing costs 1.3 us).
+template <class T> constexpr int kSumBatch = 256 / static_cast<int>(sizeof(T));
+constexpr int kSumFew = 8;
 
 // Scratch layout (bytes): lanes[65536] f64 | gp[64] f64 | ticket u32 (+pad).
 constexpr size_t kLanesBytes = sizeof(double) * kVirtualLanes;
@@ -35,36 +38,45 @@ constexpr size_t kGpBytes = sizeof(double) * kGroups;
 constexpr size_t kSumScratch = kLanesBytes + kGpBytes + 256;
 
 // Virtual lane l = blockIdx.x*256 + threadIdx.x adds u[l], u[l+65536], ... in
-// order from +0.0.  The loads of kSumUnroll rows are issued before their adds
-// so each lane keeps kSumUnroll loads in flight; the adds stay in row order.
-// The fold's ticket is cleared here, one launch ahead of the fold that takes
-// it, so a sum never depends on what an earlier call left in its scratch.
-template <class T>
+// order from +0.0.  A batch of rows is in flight while the one
+// before it is added (one wave a SIMD holds the lanes, so nothing else covers
+// the loads' latency); a row past the end adds +0.0, which leaves a sum that is
+// never -0.0 as it is.  The fold's ticket is cleared here, one launch ahead of
+// the fold that takes it, so a sum never depends on what an earlier call left
+// in its scratch.
+template <class T, int Batch>
 __global__ __launch_bounds__(kLaneBlock) void hawk_sum_lanes(const T* __restrict__ u,
                                                               long long n,
                                                               T* __restrict__ lanes,
                                                               unsigned* __restrict__ ticket) {
     const long long l = static_cast<long long>(blockIdx.x) * kLaneBlock + threadIdx.x;
     if (l == 0) *ticket = 0u;
-    T s = T(0);
-    long long r = l;
     constexpr long long kStep = kVirtualLanes;
-    for (; r + (kSumUnroll - 1) * kStep < n; r += kSumUnroll * kStep) {
-        T a[kSumUnroll];
+    const long long rows = (n + kStep - 1) / kStep;         // of the first lane, the longest
+    T s = T(0);
+    auto load = [&](long long r, T (&a)[Batch]) {
+        const T* p = u + r * kStep + l;
+        if ((r + Batch) * kStep <= n) {
 #pragma unroll
-        for (int k = 0; k < kSumUnroll; ++k) a[k] = __builtin_nontemporal_load(u + r + k * kStep);
+            for (int k = 0; k < Batch; ++k) a[k] = __builtin_nontemporal_load(p + k * kStep);
+        } else if (r < rows) {
+            const int left = n - r * kStep - l <= 0 ? 0 : static_cast<int>((n - r * kStep - l + kStep - 1) / kStep);
 #pragma unroll
-        for (int k = 0; k < kSumUnroll; ++k) s += a[k];
-    }
-    // the rows left, eight loads in flight; a row past the end adds +0.0, which
-    // leaves a sum that is never -0.0 as it is.  One load at a time they took
-    // 14 of the kernel's 23 us at n = 10^7 (24 rows past four full blocks).
-    for (; r < n; r += kSumTail * kStep) {
-        T a[kSumTail];
+            for (int k = 0; k < Batch; ++k) a[k] = k < left ? __builtin_nontemporal_load(p + k * kStep) : T(0);
+        }
+    };
+    auto add = [&](long long r, const T (&a)[Batch]) {
+        if (r >= rows) return;
 #pragma unroll
-        for (int k = 0; k < kSumTail; ++k) a[k] = r + k * kStep < n ? __builtin_nontemporal_load(u + r + k * kStep) : T(0);
-#pragma unroll
-        for (int k = 0; k < kSumTail; ++k) s += a[k];
+        for (int k = 0; k < Batch; ++k) s += a[k];
+    };
+    T a[Batch], b[Batch];
+    load(0, a);
+    for (long long r = 0; r < rows; r += 2 * Batch) {
+        load(r + Batch, b);
+        add(r, a);
+        load(r + 2 * Batch, a);
+        add(r + Batch, b);
     }
     lanes[l] = s;
 }
@@ -2125,8 +2137,12 @@ int ordered_sum(const T* u, int64_t n, T* out, void* scratch, void* stream, cons
         hipLaunchKernelGGL((hawk_keyed_rows<T, 16>), dim3(1), dim3(1024), 0, s, u, static_cast<long long>(n), out);
         return launch_error("hawk_keyed_rows launch");
     }
-    hipLaunchKernelGGL(hawk_sum_lanes<T>, dim3(kVirtualLanes / kLaneBlock), dim3(kLaneBlock), 0, s, u,
-                       static_cast<long long>(n), lanes, ticket);
+    const dim3 grid(kVirtualLanes / kLaneBlock), block(kLaneBlock);
+    const long long len = n;
+    if (n <= kSumFew * static_cast<long long>(kVirtualLanes))
+        hipLaunchKernelGGL((hawk_sum_lanes<T, kSumFew>), grid, block, 0, s, u, len, lanes, ticket);
+    else
+        hipLaunchKernelGGL((hawk_sum_lanes<T, kSumBatch<T>>), grid, block, 0, s, u, len, lanes, ticket);
     int rc = launch_error("hawk_sum_lanes launch");
     if (rc != HK_OK) return rc;
     hipLaunchKernelGGL(hawk_sum_fold<T>, dim3(kGroups), dim3(256), 0, s, lanes, gp, ticket, out);
