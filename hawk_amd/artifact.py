@@ -21,7 +21,7 @@ from . import compile as _compile
 from . import policy as _policy
 from .emit_hip import fp_ops_per_sample
 from .resources import kernel_resources
-from .emit_hip import plan_kernel
+from .emit_hip import plan_kernel, sample_major_entry, sample_major_name, sample_major_planes
 from .ir import AUTO_K_MAX, FINISHED_PLANE, Finish, HawkError
 from .targets import TARGETS, row
 from .trace import Kernel
@@ -309,10 +309,20 @@ def build_bundle(kernels, directory, *, targets=("hip",), mode: str = "float64",
         if plan.stage is not None and min_blocks > 1:
             plan.source = _with_waves(plan.source, shape[0], waves_per_eu(shape[0], min_blocks))
         plans.append((k, plan, shape))
-    staged = [(k, p) for k, p, _ in plans if p.stage is not None]
-    compiled = dict(zip([k.name for k, _ in staged],
-                        _compile.compile_units([(k.name, p.source) for k, p in staged], options=options,
-                                               cache_dir=cache_dir)))
+    units = {}
+    for k, plan, shape in plans:
+        if plan.stage is None:
+            continue
+        units[k.name] = plan.source
+        major = sample_major_planes(plan.stage)
+        if major:
+            # a second entry in the unit: the same stage over (N, w) planes
+            # (hawk.run's layout="samples_first")
+            entry = sample_major_entry(plan.stage, "float64" if mode == "banded" else mode, *shape, target=target)
+            if min_blocks > 1:
+                entry = _with_waves(entry, shape[0], waves_per_eu(shape[0], min_blocks))
+            units[k.name] += "\n" + entry
+    compiled = dict(zip(units, _compile.compile_units(list(units.items()), options=options, cache_dir=cache_dir)))
     for k, plan, shape in plans:
         sidecar = {
             "kernel": k.name, "target": target.id, "offload_arch": target.offload_arch, "mode": mode,
@@ -326,7 +336,7 @@ def build_bundle(kernels, directory, *, targets=("hip",), mode: str = "float64",
         }
         if plan.stage is not None:
             code, key, _hit = compiled[k.name]
-            _write(directory / f"{k.name}{target.source}", plan.source.encode())
+            _write(directory / f"{k.name}{target.source}", units[k.name].encode())
             _write(directory / f"{k.name}{target.artifact}", code)
             sidecar.update({
                 "entry": k.name,
@@ -334,7 +344,7 @@ def build_bundle(kernels, directory, *, targets=("hip",), mode: str = "float64",
                 "descriptor": [plan.stage.planes[n]["kind"] for _, n in plan.stage.arg_spec],
                 "source": f"{k.name}{target.source}", "code_object": f"{k.name}{target.artifact}",
                 "format": target.format, "entry_kind": target.entry,
-                "source_sha256": hashlib.sha256(plan.source.encode()).hexdigest(),
+                "source_sha256": hashlib.sha256(units[k.name].encode()).hexdigest(),
                 "code_sha256": hashlib.sha256(code).hexdigest(),
                 "cache_key": key, "compile_options": list(options),
                 "toolchain": _compile.toolchain(),
@@ -344,6 +354,9 @@ def build_bundle(kernels, directory, *, targets=("hip",), mode: str = "float64",
                 "fp_ops_per_sample": plan.algorithmic_ops,
                 "fp_ops_emitted": fp_ops_per_sample(plan.source),
             })
+            major = sample_major_planes(plan.stage)
+            if major:
+                sidecar["sample_major"] = {"entry": sample_major_name(k.name), "planes": major}
         finish = next((s for s in k.program.sinks if isinstance(s, Finish)), None)
         if plan.stage is not None and plan.stage.guard is not None:
             # reference tests/test_finish_own_sample.py:98-106

@@ -28,7 +28,7 @@ import re
 
 import math
 import dataclasses
-from dataclasses import dataclass, field
+from dataclasses import dataclass, field, replace
 
 from . import ir
 from .ir import (FINISHED_PLANE, GUARD_MASK, AccumWrite, Assign, Deps, Finish, HawkError, Node, OrderedFold,
@@ -112,8 +112,9 @@ class _Scope:
 class _Writer:
     """Scalarises nodes into C++ statements."""
 
-    def __init__(self, stage: Stage, mode: str, nontemporal: bool = False, spell=HIP_WRITER):
+    def __init__(self, stage: Stage, mode: str, nontemporal: bool = False, spell=HIP_WRITER, widths=None):
         self.stage = stage
+        self.widths = widths or {}           # plane variable -> components, of the planes read sample-major
         self.mode = mode
         self.nontemporal = nontemporal
         self.spell = spell                   # the target row's writer: every piece of text
@@ -606,18 +607,53 @@ def component_planes(stage: Stage) -> int:
     return total
 
 
+def sample_major_planes(stage: Stage | None) -> list:
+    """The vector and matrix planes of the caller's that a stage can also read
+    and write sample-major, ``(N, w)``: all of a stage's, or none where a part
+    of its text indexes them by component (a guard's entries, a fold)."""
+    if stage is None or stage.guard is not None or stage.finish is not None or stage.fused_folds or stage.key_writes:
+        return []
+    return [name for name, info in stage.planes.items()
+            if info["shape"] and not name.startswith("hk_")
+            and info["role"] in ("vec_in", "mat_in", "mutable", "out", "wide_out", "per_sample")]
+
+
+def sample_major_name(name: str) -> str:
+    return f"{name}__rows"
+
+
+def sample_major_entry(stage: Stage, mode: str, block: int, per_thread: int, target=None) -> str:
+    """The stage over sample-major planes: one more entry for the stage's unit.
+    Its loads and stores go through the cache: a lane reads and writes its
+    sample's components side by side, so a wave's accesses to one line are
+    spread over as many instructions as the line holds components.  Measured on
+    MI355X (fp64): the energy forward and VJP over 4 000 037 samples 18.8 and
+    32.9 us (streaming 22.2 and 41.0), the 6x6 solve and its VJP over 500 009
+    45.7 and 103 us (streaming 127 and 368), where torch's component-major copy
+    of the vector plane alone takes 56 us and of the matrix plane 325 us."""
+    named = replace(stage, name=sample_major_name(stage.name))
+    text = render_stage(named, mode, block, per_thread, nontemporal=False, target=target,
+                        sample_major=sample_major_planes(stage))
+    return text[text.index('extern "C" __global__'):]
+
+
 def render_stage(stage: Stage, mode: str, block: int, per_thread: int, unroll_taped: bool = True,
-                 nontemporal: bool = False, xcd_order: bool | None = None, target=None) -> str:
+                 nontemporal: bool = False, xcd_order: bool | None = None, target=None,
+                 sample_major=()) -> str:
     """The HIP source of one per-sample stage.  ``nontemporal`` marks the
     plane loads and stores as streaming (read or written once, not kept in
     cache); ``xcd_order`` (default: at least ``XCD_ORDER_PLANES`` component
     planes) hands each XCD a contiguous eighth of the blocks.  ``target`` is
     the row whose writer spells the body and whose wrapper makes the entry
-    (default: the ``hip`` row)."""
+    (default: the ``hip`` row).  The planes named in ``sample_major`` hold a
+    sample's components side by side (:func:`sample_major_planes`)."""
     target = TARGETS["hip"] if target is None else target
+    widths = {}
+    for name in sample_major:
+        widths[stage.planes[name]["var"]] = len(_entries(tuple(stage.planes[name]["shape"])))
     if xcd_order is None:
         xcd_order = component_planes(stage) >= XCD_ORDER_PLANES
-    w = _Writer(stage, mode, nontemporal, spell=target.writer)
+    w = _Writer(stage, mode, nontemporal, spell=target.writer, widths=widths)
     roots = ([node for _, node in stage.writes] + [node for _, node, _, _, _ in stage.row_sums]
              + [node for _, nodes, _ in stage.key_writes for node in nodes]
              + [node for f in stage.fused_folds for node in tuple(f[2]) + tuple(f[3])]

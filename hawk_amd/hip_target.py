@@ -238,8 +238,14 @@ class HipWriter:
         from .emit_hip import _entries, _flat
         if not leaf.ttype.shape:
             return [self.load(r, f"{p}[hk_i]")]
-        return [self.load(r, f"{p}[{_flat(leaf.ttype.shape, e)} * {p}_cs + hk_i]")
-                for e in _entries(leaf.ttype.shape)]
+        return [self.load(r, self.component(r, p, _flat(leaf.ttype.shape, e))) for e in _entries(leaf.ttype.shape)]
+
+    def component(self, r, p: str, c: int) -> str:
+        """Component ``c`` of the sample's entry of plane ``p``: component-major,
+        or in the sample-major form of a stage ``w`` consecutive components a
+        sample."""
+        w = getattr(r, "widths", {}).get(p)
+        return f"{p}[{c} * {p}_cs + hk_i]" if w is None else f"{p}[hk_i * {w} + {c}]"
 
     def load(self, r, ref: str) -> str:
         return f"__builtin_nontemporal_load(&{ref})" if r.nontemporal else ref
@@ -376,7 +382,7 @@ class HipWriter:
         return f"            if ({cond}) {{ {mask}[hk_i] = 1; hk_new = true; }}"
 
     def component_commit(self, r, target: str, at, op: str, value: str) -> str:
-        ref = f"{target}[hk_i]" if at is None else f"{target}[{at} * {target}_cs + hk_i]"
+        ref = f"{target}[hk_i]" if at is None else self.component(r, target, at)
         if op == "=":
             return self.store(r, None, ref, value)
         return f"{ref} {op} {value};"

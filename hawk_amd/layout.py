@@ -8,8 +8,11 @@ load instruction of a wave reads 64 consecutive samples of one component.
 "samples_first"`` says so for every plane of the call, ``samples_first(x)``
 for one array (the marker wins; a contradiction is refused), and a plane
 whose shape reads only one way needs neither.  A plane whose shape reads both
-ways (``N == w``) is refused unless one of them says which.  A sample-major
-plane runs through a component-major copy: its values are copied in before
+ways (``N == w``) is refused unless one of them says which.  A kernel
+whose stage was also built over sample-major planes reads and writes them in
+place where a call's vector and matrix planes are all sample-major, contiguous
+and apart from one another in memory; otherwise a sample-major plane runs
+through a component-major copy: its values are copied in before
 the launch and, for a plane the kernel writes, copied back after it, on the
 launch's stream.  ``prepare`` binds planes by address and takes
 component-major planes only.
@@ -55,16 +58,35 @@ def resolve(kernel, arrays: dict, layout, per_sample_roles, written_roles):
     """``(arrays, write_back)``: every marker removed and every sample-major
     plane replaced by a component-major copy; ``write_back`` lists
     ``(caller's array, copy)`` for the planes the kernel writes."""
+    out, major = classify(kernel, arrays, layout, per_sample_roles)
+    return component_major(kernel, out, major, written_roles)
+
+
+def component_major(kernel, arrays: dict, major: list, written_roles):
+    """``(arrays, write_back)`` with the sample-major planes ``major`` of
+    :func:`classify` replaced by component-major copies (see :func:`resolve`)."""
+    out, back = dict(arrays), []
+    for name in major:
+        x = arrays[name]
+        out[name] = copy = x.movedim(0, -1).contiguous()
+        if kernel.planes[name]["role"] in written_roles:
+            back.append((x, copy))
+    return out, back
+
+
+def classify(kernel, arrays: dict, layout, per_sample_roles):
+    """``(arrays, major)``: every marker removed, and the names of the planes
+    that are sample-major."""
     check_layout(layout)
-    out, back, pending = {}, [], []
+    out, major = {}, []
     for name, value in arrays.items():
         marked = value if isinstance(value, Marked) else None
         x = marked.array if marked else value
+        out[name] = x
         info = kernel.planes.get(name)
         if info is None or info["role"] not in per_sample_roles or not hasattr(x, "dim"):
             if marked is not None and info is not None and info["role"] not in per_sample_roles:
                 raise HawkError(f"{name!r} is not a per-sample plane: it has no sample axis to mark")
-            out[name] = x
             continue
         lead = tuple(info["shape"])
         shape = tuple(x.shape)
@@ -72,7 +94,6 @@ def resolve(kernel, arrays: dict, layout, per_sample_roles, written_roles):
         first = len(shape) == len(lead) + 1 and shape[1:] == lead
         axis = marked.axis if marked else layout  # the array's marker beats the call's layout
         if not lead:                              # a scalar plane (N,) reads the same either way
-            out[name] = x
             continue
         if axis is None:
             if first and last:
@@ -85,12 +106,6 @@ def resolve(kernel, arrays: dict, layout, per_sample_roles, written_roles):
                 said = "is marked samples_first" if marked else "is sample-major under layout='samples_first'"
                 raise HawkError(f"{name!r} {said} but has shape {shape}; a {lead} plane is "
                                 f"({', '.join(['N'] + [str(e) for e in lead])})")
-            out[name] = x
             continue
-        pending.append((name, x, info))
-    for name, x, info in pending:
-        copy = x.movedim(0, -1).contiguous()
-        out[name] = copy
-        if info["role"] in written_roles:
-            back.append((x, copy))
-    return out, back
+        major.append(name)
+    return out, major

@@ -107,6 +107,7 @@ class DeviceKernel:
         # What each slot of self.block holds: ("p", ptr, samples, device) or
         # ("v", value); None before the first bind.
         self._held_slots: list = [None] * len(self.arg_spec)
+        self._rows = None         # the sample-major stage, bound by the first call that takes it
         self._scratch: dict = {}
         self._lock = threading.Lock()
         self.scatter_chunks = None
@@ -218,8 +219,46 @@ class DeviceKernel:
         self.finished = held
         return {**arrays, FINISHED_PLANE: held}, held
 
-    def check_planes(self, arrays: dict, n_samples=None) -> int:
-        """Validate every bound plane against the sidecar; return the sample count."""
+    def takes_rows(self, arrays: dict, major: list, entry: str) -> bool:
+        """Whether a call whose planes ``major`` are sample-major runs on the
+        stage built over ``(N, w)`` planes: every vector and matrix plane of the
+        stage is sample-major and contiguous, and no plane the call writes
+        shares memory with another (the copies of the general path keep them
+        apart)."""
+        rows = self.sidecar.get("sample_major")
+        if not rows or entry != "plain" or set(rows["planes"]) != set(major):
+            return False
+        torch = _torch()
+        spans = []
+        for name, x in arrays.items():
+            if not isinstance(x, torch.Tensor):
+                continue
+            if not x.is_contiguous() or not x.is_cuda:
+                return False
+            start = x.data_ptr()
+            spans.append((start, start + x.numel() * x.element_size(),
+                          self.planes[name]["role"] in _WRITTEN + ("cell", "accum_out") if name in self.planes
+                          else False))
+        spans.sort()
+        reach, reach_written = 0, 0           # the furthest end so far, of any plane and of a written one
+        for start, end, written in spans:
+            if start < (reach if written else reach_written):
+                return False
+            reach = max(reach, end)
+            if written:
+                reach_written = max(reach_written, end)
+        return True
+
+    def _rows_stage(self) -> tuple:
+        """``(entry, argument block, held slots)`` of the sample-major stage."""
+        if self._rows is None:
+            self._rows = (self.library.entry(self.sidecar["sample_major"]["entry"]),
+                          _core.ArgBlock(self.sidecar["descriptor"]), [None] * len(self.arg_spec))
+        return self._rows
+
+    def check_planes(self, arrays: dict, n_samples=None, rows=()) -> int:
+        """Validate every bound plane against the sidecar (those named in
+        ``rows`` as sample-major); return the sample count."""
         torch = _torch()
         grid = self.sidecar.get("grid")
         n_grid = None
@@ -280,14 +319,15 @@ class DeviceKernel:
                 continue
             if role in _PER_SAMPLE:
                 lead = tuple(info["shape"])
-                if x.dim() != len(lead) + 1 or tuple(x.shape[:-1]) != lead:
+                if x.dim() != len(lead) + 1 or tuple(x.shape[1:] if name in rows else x.shape[:-1]) != lead:
                     problems.append(f"{name!r} has shape {tuple(x.shape)}; a {lead or 'scalar'} plane is "
                                     f"({', '.join(str(e) for e in lead + ('N',))})")
                     continue
+                here = int(x.shape[0 if name in rows else -1])
                 if n is None:
-                    n = int(x.shape[-1])
-                elif int(x.shape[-1]) != n:
-                    problems.append(f"{name!r} holds {int(x.shape[-1])} samples, other planes {n}")
+                    n = here
+                elif here != n:
+                    problems.append(f"{name!r} holds {here} samples, other planes {n}")
             elif role == "cell" and info.get("group"):
                 keyed.append((name, x, info["group"]))
             elif role == "cell":
@@ -436,24 +476,27 @@ class DeviceKernel:
         return args, status, cells
 
     # -- launch --------------------------------------------------------------
-    def bind_all(self, arrays: dict, n: int) -> None:
-        """Bind the per-sample stage's slots to validated ``arrays``, crossing
+    def bind_all(self, arrays: dict, n: int, block=None, slots=None) -> None:
+        """Bind the per-sample stage's slots (or another argument block's, with
+        what its ``slots`` hold) to validated ``arrays``, crossing
         the C-ABI only for what changed since the last bind: a slot whose
         length, device or by-value number changed is bound on its own; every
         slot whose pointer alone moved is swapped in ONE bulk rebind.  So a
         run over the planes of the last run adds no crossing to its launch,
         and a run over moved planes adds one (reference ``hawk/runtime.py:330-345``,
         the stable-binding and rebind arms of its launch-crossing contract)."""
+        block = self.block if block is None else block
+        slots = self._held_slots if slots is None else slots
         moved_slots, moved_ptrs = [], []
         for slot, (role, name) in enumerate(self.arg_spec):
-            kind = self.block.descriptor[slot]
+            kind = block.descriptor[slot]
             x = arrays[name]
-            held = self._held_slots[slot]
+            held = slots[slot]
             if kind in ("f64", "f32"):
                 value = float(x)
                 if held != ("v", value):
-                    self.block.bind_value(slot, value)
-                    self._held_slots[slot] = ("v", value)
+                    block.bind_value(slot, value)
+                    slots[slot] = ("v", value)
                 continue
             ptr, samples, device = x.data_ptr(), _bound_length(role, x, n), x.device.index or 0
             if held is not None and held[0] == "p" and held[2:] == (samples, device):
@@ -461,10 +504,10 @@ class DeviceKernel:
                     moved_slots.append(slot)
                     moved_ptrs.append(ptr)
                 continue
-            self.block.bind(slot, ptr, samples, 1, _contracts.DEVICE_ROCM, device)
-            self._held_slots[slot] = ("p", ptr, samples, device)
+            block.bind(slot, ptr, samples, 1, _contracts.DEVICE_ROCM, device)
+            slots[slot] = ("p", ptr, samples, device)
         if moved_slots:
-            self.rebind(moved_slots, moved_ptrs)
+            self._swap(block, slots, moved_slots, moved_ptrs)
 
     def rebind(self, slots, ptrs) -> None:
         """The bulk pointer swap: every (slot, pointer) pair in ONE crossing
@@ -472,22 +515,24 @@ class DeviceKernel:
         design: it only moves slots a validated bind already shaped, so each
         slot keeps the length and device it was bound with.  A by-value slot
         is refused (by the C-ABI, naming the slot)."""
-        slots = [int(s) for s in slots]
-        ptrs = [int(p) for p in ptrs]
-        self.block.rebind(slots, ptrs)
+        self._swap(self.block, self._held_slots, [int(s) for s in slots], [int(p) for p in ptrs])
+
+    @staticmethod
+    def _swap(block, held_slots: list, slots: list, ptrs: list) -> None:
+        block.rebind(slots, ptrs)
         for slot, ptr in zip(slots, ptrs):
-            held = self._held_slots[slot]
+            held = held_slots[slot]
             if held is not None and held[0] == "p":
-                self._held_slots[slot] = ("p", ptr, held[2], held[3])
+                held_slots[slot] = ("p", ptr, held[2], held[3])
 
     def _run(self, arrays: dict, base: int, count: int, n: int, stream: int, check: bool, steps=None,
-             entry: str = "plain", chunk: int = PERSIST_CHUNK) -> None:
+             entry: str = "plain", chunk: int = PERSIST_CHUNK, rows: bool = False) -> None:
         # every reset, scratch fill and status read is issued on the launch's stream
         with _on(stream):
-            self._run_on(arrays, base, count, n, stream, check, steps, entry, chunk)
+            self._run_on(arrays, base, count, n, stream, check, steps, entry, chunk, rows)
 
     def _run_on(self, arrays: dict, base: int, count: int, n: int, stream: int, check: bool, steps,
-                entry: str, chunk: int) -> None:
+                entry: str, chunk: int, rows: bool = False) -> None:
         torch = _torch()
         device = next((x.device for x in arrays.values() if isinstance(x, torch.Tensor)), None)
         if device is None:
@@ -519,9 +564,10 @@ class DeviceKernel:
                 _core.keyed_log_fold(*args, stream)
                 statuses.append((t, status, cells))
         if self.entry is not None:
-            self.bind_all(bound, n)
-            self.entry.run(self.block, base, count, n, threads=self.launch_shape["block"],
-                           per_thread=self.launch_shape["per_thread"], stream=stream)
+            fn, block, slots = self._rows_stage() if rows else (self.entry, self.block, self._held_slots)
+            self.bind_all(bound, n, block, slots)
+            fn.run(block, base, count, n, threads=self.launch_shape["block"],
+                   per_thread=self.launch_shape["per_thread"], stream=stream)
         for t in self.team:
             if t.get("before"):
                 continue
@@ -774,9 +820,12 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
         stream = torch.cuda.current_stream().cuda_stream
     elif hasattr(stream, "cuda_stream"):
         stream = stream.cuda_stream
-    with _on(int(stream)):
-        arrays, write_back = _layout.resolve(kernel, arrays, layout, _PER_SAMPLE, _WRITTEN)
-    n = kernel.check_planes(arrays, n_samples)
+    arrays, major = _layout.classify(kernel, arrays, layout, _PER_SAMPLE)
+    rows, write_back = bool(major) and kernel.takes_rows(arrays, major, entry), []
+    if major and not rows:
+        with _on(int(stream)):
+            arrays, write_back = _layout.component_major(kernel, arrays, major, _WRITTEN)
+    n = kernel.check_planes(arrays, n_samples, major if rows else ())
     if kernel.team and (base != 0 or count not in (None, n)):
         raise HawkError(f"{kernel.name}: this kernel reduces over every sample, so it runs over every "
                         "sample (no base= or count=)")
@@ -786,7 +835,7 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
         raise HawkError(f"{kernel.name}: [base, base+count) = [{base}, {base + count}) is outside [0, {n})")
     with kernel._lock:
         kernel._run(arrays, int(base), int(count), int(n), int(stream), check, steps=steps, entry=entry,
-                    chunk=chunk)
+                    chunk=chunk, rows=rows)
     if write_back:
         with _on(int(stream)):
             for dst, copy in write_back:       # a sample-major plane the kernel wrote

@@ -183,3 +183,77 @@ def test_rows_finish_together(gpu, mode, rows):
     want = np.array([w for *_, w in jobs], dt)
     nan = np.isnan(want)
     assert (np.isnan(got) == nan).all() and got[~nan].tobytes() == want[~nan].tobytes()
+
+
+@pytest.mark.parametrize("mode", ["float64", "float32"])
+@pytest.mark.parametrize("n", [1, 6, 127, 1001, 70_003])
+def test_sample_major_stage(tmp_path, gpu, mode, n):
+    """Every vector and matrix plane sample-major: the stage over (N, w) planes
+    gives the component-major run's bits; so does the copying path (a plane
+    marked the other way, a strided plane, planes that share memory), which the
+    rule must pick there, and a partial range touches only its samples."""
+    import hawk_amd as hawk
+    import torch
+    from hawk_amd import Mutable, Scalar, Vector
+    from hawk_amd import examples as E
+    from hawk_amd.runtime import _PER_SAMPLE, _WRITTEN
+
+    @hawk.kernel
+    def total_vec(v: Vector[3], w: Mutable[Vector[2]], s: Mutable[Vector[3]]):
+        w = hawk.math.vec(v[0] + v[1], v[2])
+        s = hawk.sum(v * 2.0)
+
+    dt = torch.float32 if mode == "float32" else torch.float64
+    g = torch.Generator(device=gpu).manual_seed(n)
+    for k in _unit(tmp_path, [E.energy, E.energy_vjp, E.spd_solve, E.spd_solve_vjp, E.twobody, total_vec], mode):
+        ins, major = {}, set()
+        for name in k.caller_planes():
+            info = k.planes[name]
+            if info["role"] == "uniform":
+                ins[name] = 1.0
+                continue
+            shape = tuple(info["shape"]) + ((n,) if info["role"] in _PER_SAMPLE else ())
+            ins[name] = torch.randn(shape, dtype=dt, device=gpu, generator=g)
+            if name == "A":
+                ins[name] += 20.0 * torch.eye(6, dtype=dt, device=gpu)[:, :, None]
+            if info["shape"] and info["role"] in _PER_SAMPLE:
+                major.add(name)
+        assert set(k.sidecar["sample_major"]["planes"]) == major
+
+        def run(change=lambda planes: planes, direct=True, **kw):
+            planes = {name: x.movedim(-1, 0).contiguous() if name in major else x.clone() if torch.is_tensor(x) else x
+                      for name, x in ins.items()}
+            call = change(dict(planes))
+            first = [name for name in major if not isinstance(call[name], hawk.layout.Marked)
+                     or call[name].axis == "samples_first"]
+            plain = {name: getattr(x, "array", x) for name, x in call.items()}
+            assert k.takes_rows(plain, first, "plain") == direct
+            hawk.run(k, layout="samples_first", **call, **kw)
+            return {name: x.movedim(0, -1).contiguous() if name in first else x
+                    for name, x in plain.items() if torch.is_tensor(x)}
+
+        want = {name: x.clone() for name, x in ins.items() if torch.is_tensor(x)}
+        hawk.run(k, layout="samples_last", **{**ins, **want})
+
+        def same(got):
+            for name, x in want.items():
+                assert got[name].cpu().numpy().tobytes() == x.cpu().numpy().tobytes(), (k.name, name)
+        same(run())
+        one = sorted(major)[0]
+        if len(major) > 1 and n != 6:
+            same(run(lambda p: {**p, one: hawk.samples_last(ins[one].clone())}, direct=False))
+        read = [m for m in sorted(major) if k.planes[m]["role"] not in _WRITTEN]
+        if n > 1:
+            wide = torch.empty((2 * n,) + tuple(k.planes[read[0]]["shape"]), dtype=dt, device=gpu)
+            wide[::2] = ins[read[0]].movedim(-1, 0)
+            same(run(lambda p: {**p, read[0]: wide[::2]}, direct=False))
+        if k.name == "twobody":                          # stepping a state in place
+            got = run(lambda p: {**p, "r": p["r0"], "v": p["v0"]}, direct=False)
+            assert got["r"].cpu().numpy().tobytes() == want["r"].cpu().numpy().tobytes()
+            assert got["v"].cpu().numpy().tobytes() == want["v"].cpu().numpy().tobytes()
+        if n > 100 and not k.team:
+            part = run(base=5, count=n - 60)
+            for name, x in want.items():
+                assert torch.equal(part[name][..., 5:n - 55], x[..., 5:n - 55])
+                assert torch.equal(part[name][..., :5], ins[name][..., :5])
+                assert torch.equal(part[name][..., n - 55:], ins[name][..., n - 55:])
