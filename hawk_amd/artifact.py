@@ -90,6 +90,16 @@ GATHER_SHAPE = (1024, 2)
 PAIR_SHAPE = (64, 2)
 STREAM_SHAPE = (256, 4)
 
+#: A float32 stream of a few operations more (the energy forward: three rows
+#: in, one out): 4 bytes a lane leave a thread of one sample half the bytes in
+#: flight that a float64 one has, so a thread takes two.  Over 2^25 samples
+#: 101.7 us at 128 x 1, 100.9 at 256 x 1, 85.8 at 256 x 2, 88.2 at 256 x 4; over
+#: 10 000 019 32.9, 33.6, 27.5 and 26.5.  Its VJP (seven float32 rows) over
+#: 10 000 019 samples: 56.0 at 128 x 1, 52.1 at 256 x 1, 53.5 at 256 x 2; its
+#: JVP 50.0, 47.7 and 48.8.
+LIGHT_OPS = 8
+LIGHT_SHAPE = (256, 2)
+
 
 def launch_shape(plan, mode: str) -> tuple:
     """``(block, per_thread)`` a stage runs with when the build does not fix them."""
@@ -101,7 +111,12 @@ def launch_shape(plan, mode: str) -> tuple:
     nbytes = _stage_bytes(plan, mode)
     if nbytes <= STREAM_BYTES and fp_ops_per_sample(plan.source) <= STREAM_OPS:
         return PAIR_SHAPE if pair_candidate(stage, mode) else STREAM_SHAPE
-    shape = (256, 1) if 32 < nbytes <= 64 else (128, 1)
+    if mode == "float32" and nbytes <= STREAM_BYTES and fp_ops_per_sample(plan.source) <= LIGHT_OPS:
+        shape = LIGHT_SHAPE
+    else:
+        # five to eight 8-byte planes, or float32 ones
+        low, high = (16, 32) if mode == "float32" else (32, 64)
+        shape = (256, 1) if low < nbytes <= high else (128, 1)
     if stage.row_sums and not stage.fused_folds:
         # row reductions take two samples a lane (the paired layout)
         shape = (shape[0], 2)
