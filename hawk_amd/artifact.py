@@ -81,6 +81,13 @@ def _stage_bytes(plan, mode: str) -> int:
 #: 0.36 at 512 x 2, 0.28 at 1024 x 2, 0.41 at 1024 x 4).
 GATHER_SHAPE = (1024, 2)
 
+#: The launch shape of a stage whose tables are read by its lane axes alone (no
+#: index plane): a wave reads few cells, so nothing waits on a gather, and
+#: workgroups of 2048 samples leave a last round nearly empty.  The nets' losses
+#: at 1024 x 2 and 256 x 1: 16384 nets of 40 samples 21.2 and 14.4 us, 8192 of 96
+#: 23.7 and 16.1, 16384 of 64 22.8 and 21.4, 32768 of 16 12.3 and 12.2.
+LANE_TABLE_SHAPE = (256, 1)
+
 #: The launch shape of a light stream whose planes are all scalar float64
 #: planes: 64 threads of one pair of adjacent samples, read and written 16
 #: bytes a lane (``emit_hip._pair_lines``).  A copy of ``scale``'s pattern
@@ -105,9 +112,11 @@ def launch_shape(plan, mode: str) -> tuple:
     """``(block, per_thread)`` a stage runs with when the build does not fix them."""
     from .emit_hip import fp_ops_per_sample, pair_candidate
     stage = plan.stage
-    if (any(info["role"] == "lookup" for info in stage.planes.values()) and not stage.row_sums
+    infos = stage.planes.values()
+    if (any(info["role"] == "lookup" for info in infos) and not stage.row_sums
             and not stage.fused_folds and not stage.key_writes and stage.guard is None and stage.finish is None):
-        return GATHER_SHAPE
+        keyed = any(info["role"] == "per_sample" and info["dtype"] in ("i32", "u32") for info in infos)
+        return GATHER_SHAPE if keyed else LANE_TABLE_SHAPE
     nbytes = _stage_bytes(plan, mode)
     if nbytes <= STREAM_BYTES and fp_ops_per_sample(plan.source) <= STREAM_OPS:
         return PAIR_SHAPE if pair_candidate(stage, mode) else STREAM_SHAPE
