@@ -211,6 +211,7 @@ class ArgBlock:
         self._h = handle
         self.descriptor = list(descriptor)
         self._values = []
+        self._swap = None
 
     @property
     def size(self) -> int:
@@ -235,8 +236,15 @@ class ArgBlock:
         n = len(slots)
         if len(ptrs) != n:
             raise ValueError("hawk_core.ArgBlock.rebind: slots and ptrs must be the same length")
-        s = (ctypes.c_int64 * max(1, n))(*[int(x) for x in slots])
-        p = (ctypes.c_int64 * max(1, n))(*[int(x) for x in ptrs])
+        # the (slot, pointer) arrays are made once and reused by every call (the
+        # caller's lock keeps a block to one thread at a time)
+        if self._swap is None or len(self._swap[0]) < n:
+            size = max(1, n, len(self.descriptor))
+            self._swap = (ctypes.c_int64 * size)(), (ctypes.c_int64 * size)()
+        s, p = self._swap
+        for i in range(n):
+            s[i] = int(slots[i])
+            p[i] = int(ptrs[i])
         check(lib().hk_rebind(self._h, s, p, n), ValueError)
 
     @property
@@ -257,19 +265,32 @@ class DeviceEntry:
         handle = ctypes.c_void_p()
         check(lib().hk_entry_get(library.handle, name.encode(), ctypes.byref(handle)))
         self._h = handle
+        self._launch = lib().hk_launch
         self.name = name
         self.library = library
 
     def run(self, block: ArgBlock, base: int, count: int, n_samples: int, *, threads: int = 256,
             per_thread: int = 1, stream: int = 0) -> None:
         """THE launch crossing: ``[base, base+count)`` of ``n_samples`` on ``stream``."""
-        check(lib().hk_launch(self._h, block.handle, int(base), int(count), int(n_samples), int(threads),
-                              int(per_thread), ctypes.c_void_p(stream or None)))
+        check(self._launch(self._h, block.handle, int(base), int(count), int(n_samples), int(threads),
+                           int(per_thread), stream or None))
+
+    def prepared(self, block: ArgBlock, base: int, count: int, n_samples: int, *, threads: int, per_thread: int,
+                 stream: int = 0):
+        """:meth:`run` with its arguments bound once: a callable that is the crossing alone."""
+        launch, args = self._launch, (self._h, block.handle, int(base), int(count), int(n_samples), int(threads),
+                                      int(per_thread), stream or None)
+
+        def crossing(keep=(self, block)):       # the entry and the block live as long as the callable
+            rc = launch(*args)
+            if rc != HK_OK:
+                check(rc)
+        return crossing
 
     def run_grid(self, block: ArgBlock, base: int, count: int, n_samples: int, grid: int, threads: int,
                  stream: int = 0) -> None:
         check(lib().hk_launch_grid(self._h, block.handle, int(base), int(count), int(n_samples), int(grid),
-                                   int(threads), ctypes.c_void_p(stream or None)))
+                                   int(threads), stream or None))
 
 
 class DeviceLibrary:
@@ -299,21 +320,21 @@ def ordered_sum_scratch_bytes() -> int:
 
 
 def ordered_sum(u: int, n: int, out: int, scratch: int, stream: int = 0) -> None:
-    check(lib().hk_ordered_sum_f64(ctypes.c_void_p(u or None), int(n), ctypes.c_void_p(out),
-                                   ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_ordered_sum_f64(u or None, int(n), out,
+                                   scratch, stream or None))
 
 
 def ordered_sum_f32(u: int, n: int, out: int, scratch: int, stream: int = 0) -> None:
     """:func:`ordered_sum` of a float32 plane into a float32 cell."""
-    check(lib().hk_ordered_sum_f32(ctypes.c_void_p(u or None), int(n), ctypes.c_void_p(out),
-                                   ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_ordered_sum_f32(u or None, int(n), out,
+                                   scratch, stream or None))
 
 
 def ordered_sum_noalloc(u: int, n: int, out: int, stream: int = 0) -> None:
     """The ordered sum on the library's static per-GPU scratch: no device
     memory is allocated (for callers that cannot allocate)."""
-    check(lib().hk_ordered_sum_f64_noalloc(ctypes.c_void_p(u or None), int(n), ctypes.c_void_p(out),
-                                           ctypes.c_void_p(stream or None)))
+    check(lib().hk_ordered_sum_f64_noalloc(u or None, int(n), out,
+                                           stream or None))
 
 
 def scatter_chunks(n: int, cells: int) -> int:
@@ -326,17 +347,17 @@ def ordered_scatter_scratch_bytes(n: int, cells: int) -> int:
 
 def ordered_scatter(key: int, v: int, n: int, target: int, cells: int, scratch: int, status: int,
                     stream: int = 0) -> None:
-    check(lib().hk_ordered_scatter_f64(ctypes.c_void_p(key or None), ctypes.c_void_p(v or None), int(n),
-                                       ctypes.c_void_p(target), int(cells), ctypes.c_void_p(scratch),
-                                       ctypes.c_void_p(status), ctypes.c_void_p(stream or None)))
+    check(lib().hk_ordered_scatter_f64(key or None, v or None, int(n),
+                                       target, int(cells), scratch,
+                                       status, stream or None))
 
 
 def ordered_scatter_f32(key: int, v: int, n: int, target: int, cells: int, scratch: int, status: int,
                         stream: int = 0) -> None:
     """:func:`ordered_scatter` of float32 values into a float32 target."""
-    check(lib().hk_ordered_scatter_f32(ctypes.c_void_p(key or None), ctypes.c_void_p(v or None), int(n),
-                                       ctypes.c_void_p(target), int(cells), ctypes.c_void_p(scratch),
-                                       ctypes.c_void_p(status), ctypes.c_void_p(stream or None)))
+    check(lib().hk_ordered_scatter_f32(key or None, v or None, int(n),
+                                       target, int(cells), scratch,
+                                       status, stream or None))
 
 
 def mm16(ins: list, outs: list, products: list, n: int, stream: int = 0, dtype: str = "f32") -> None:
@@ -348,11 +369,11 @@ def mm16(ins: list, outs: list, products: list, n: int, stream: int = 0, dtype: 
     flat = []
     for lhs, rhs, tl, tr in products:
         flat += [int(lhs), int(rhs), (1 if tl else 0) | (2 if tr else 0)]
-    c_in = (ctypes.c_void_p * len(ins))(*[ctypes.c_void_p(p) for p in ins])
-    c_out = (ctypes.c_void_p * len(outs))(*[ctypes.c_void_p(p) for p in outs])
+    c_in = (ctypes.c_void_p * len(ins))(*[p for p in ins])
+    c_out = (ctypes.c_void_p * len(outs))(*[p for p in outs])
     c_prod = (ctypes.c_int32 * len(flat))(*flat)
     entry = lib().hk_mm16_f64 if dtype == "f64" else lib().hk_mm16_f32
-    check(entry(c_in, len(ins), c_out, len(outs), c_prod, int(n), ctypes.c_void_p(stream or None)))
+    check(entry(c_in, len(ins), c_out, len(outs), c_prod, int(n), stream or None))
 
 
 def mm16_f64(ins: list, outs: list, products: list, n: int, stream: int = 0) -> None:
@@ -366,26 +387,26 @@ def keyed_ordered_sum_scratch_bytes(n: int, group: int) -> int:
 
 def keyed_ordered_sum(u: int, n: int, group: int, out: int, scratch: int, stream: int = 0) -> None:
     """``out[k]`` = key k's ``group`` rows by the ordered sum's tree, k < n / group."""
-    check(lib().hk_keyed_ordered_sum_f64(ctypes.c_void_p(u or None), int(n), int(group), ctypes.c_void_p(out),
-                                         ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_keyed_ordered_sum_f64(u or None, int(n), int(group), out,
+                                         scratch, stream or None))
 
 
 def keyed_ordered_sum_f32(u: int, n: int, group: int, out: int, scratch: int, stream: int = 0) -> None:
     """:func:`keyed_ordered_sum` of a float32 plane into float32 cells."""
-    check(lib().hk_keyed_ordered_sum_f32(ctypes.c_void_p(u or None), int(n), int(group), ctypes.c_void_p(out),
-                                         ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_keyed_ordered_sum_f32(u or None, int(n), int(group), out,
+                                         scratch, stream or None))
 
 
 def keyed_sample_sum(u: int, n: int, group: int, out: int, stream: int = 0) -> None:
     """``out[k]`` = key k's ``group`` rows as a default-policy sample sum of their own."""
-    check(lib().hk_keyed_sample_sum_f64(ctypes.c_void_p(u or None), int(n), int(group), ctypes.c_void_p(out or None),
-                                        ctypes.c_void_p(stream or None)))
+    check(lib().hk_keyed_sample_sum_f64(u or None, int(n), int(group), out or None,
+                                        stream or None))
 
 
 def keyed_sample_sum_f32(u: int, n: int, group: int, out: int, stream: int = 0) -> None:
     """keyed_sample_sum of a float32 plane into float32 cells."""
-    check(lib().hk_keyed_sample_sum_f32(ctypes.c_void_p(u or None), int(n), int(group), ctypes.c_void_p(out or None),
-                                        ctypes.c_void_p(stream or None)))
+    check(lib().hk_keyed_sample_sum_f32(u or None, int(n), int(group), out or None,
+                                        stream or None))
 
 
 def keyed_log_fold_scratch_bytes(cells: int) -> int:
@@ -397,19 +418,19 @@ def keyed_log_fold(values: int, stride: int, cells_log: int, keys: int, rows: in
     """``out[cells_log[e*keys + k]]`` = key k's ``rows`` contributions of slot e
     (``values[e*stride + k*rows + r]``) added in lane order from +0; status[0]
     bit 0 = a cell outside ``[0, cells)``, bit 1 = a cell named twice."""
-    check(lib().hk_keyed_log_fold_f64(ctypes.c_void_p(values or None), int(stride), ctypes.c_void_p(cells_log or None),
-                                      int(keys), int(rows), int(width), ctypes.c_void_p(out or None), int(cells),
-                                      ctypes.c_void_p(scratch or None), ctypes.c_void_p(status or None),
-                                      ctypes.c_void_p(stream or None)))
+    check(lib().hk_keyed_log_fold_f64(values or None, int(stride), cells_log or None,
+                                      int(keys), int(rows), int(width), out or None, int(cells),
+                                      scratch or None, status or None,
+                                      stream or None))
 
 
 def keyed_log_fold_f32(values: int, stride: int, cells_log: int, keys: int, rows: int, width: int, out: int,
                        cells: int, scratch: int, status: int, stream: int = 0) -> None:
     """:func:`keyed_log_fold` of float32 contributions into a float32 gradient plane."""
-    check(lib().hk_keyed_log_fold_f32(ctypes.c_void_p(values or None), int(stride), ctypes.c_void_p(cells_log or None),
-                                      int(keys), int(rows), int(width), ctypes.c_void_p(out or None), int(cells),
-                                      ctypes.c_void_p(scratch or None), ctypes.c_void_p(status or None),
-                                      ctypes.c_void_p(stream or None)))
+    check(lib().hk_keyed_log_fold_f32(values or None, int(stride), cells_log or None,
+                                      int(keys), int(rows), int(width), out or None, int(cells),
+                                      scratch or None, status or None,
+                                      stream or None))
 
 
 def rows_finish_scratch_bytes(rows: int) -> int:
@@ -418,14 +439,14 @@ def rows_finish_scratch_bytes(rows: int) -> int:
 
 def rows_finish(hi: int, comp: int, rows: int, out: int, scratch: int, stream: int = 0) -> None:
     """Fold ``rows`` compensated row pairs into the cell ``out`` (canonical ordered tree)."""
-    check(lib().hk_rows_finish_f64(ctypes.c_void_p(hi), ctypes.c_void_p(comp), int(rows), ctypes.c_void_p(out),
-                                   ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_rows_finish_f64(hi, comp, int(rows), out,
+                                   scratch, stream or None))
 
 
 def rows_finish_f32(hi: int, comp: int, rows: int, out: int, scratch: int, stream: int = 0) -> None:
     """The same finish of float32 rows, in float32."""
-    check(lib().hk_rows_finish_f32(ctypes.c_void_p(hi), ctypes.c_void_p(comp), int(rows), ctypes.c_void_p(out),
-                                   ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_rows_finish_f32(hi, comp, int(rows), out,
+                                   scratch, stream or None))
 
 
 class RowsJob(ctypes.Structure):
@@ -446,21 +467,21 @@ def rows_finish_many(jobs, rows: int, f32: bool, scratch: int, stream: int = 0) 
     """The finishes of every reduction of a stage (a ctypes array of
     :class:`RowsJob`), in float32 or float64."""
     fn = lib().hk_rows_finish_many_f32 if f32 else lib().hk_rows_finish_many_f64
-    check(fn(jobs, len(jobs), int(rows), ctypes.c_void_p(scratch), ctypes.c_void_p(stream)))
+    check(fn(jobs, len(jobs), int(rows), scratch, stream))
 
 
 def rows_extreme(hi: int, rows: int, op: int, out: int, scratch: int, stream: int = 0) -> None:
     """The finish of ``hawk.max`` (op 1) / ``hawk.min`` (op 2): ``rows``
     row extremes folded in the canonical tree, the extreme stored at ``out``.
     Scratch: :func:`rows_finish_scratch_bytes` bytes."""
-    check(lib().hk_rows_extreme_f64(ctypes.c_void_p(hi), int(rows), int(op), ctypes.c_void_p(out),
-                                    ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_rows_extreme_f64(hi, int(rows), int(op), out,
+                                    scratch, stream or None))
 
 
 def rows_extreme_f32(hi: int, rows: int, op: int, out: int, scratch: int, stream: int = 0) -> None:
     """The same finish of float32 rows."""
-    check(lib().hk_rows_extreme_f32(ctypes.c_void_p(hi), int(rows), int(op), ctypes.c_void_p(out),
-                                    ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_rows_extreme_f32(hi, int(rows), int(op), out,
+                                    scratch, stream or None))
 
 
 def band_rows_finish_scratch_bytes(rows: int) -> int:
@@ -468,8 +489,8 @@ def band_rows_finish_scratch_bytes(rows: int) -> int:
 
 
 def band_rows_finish(hi: int, lo: int, rows: int, out: int, scratch: int, stream: int = 0) -> None:
-    check(lib().hk_band_rows_finish_f64(ctypes.c_void_p(hi), ctypes.c_void_p(lo), int(rows), ctypes.c_void_p(out),
-                                        ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_band_rows_finish_f64(hi, lo, int(rows), out,
+                                        scratch, stream or None))
 
 
 def band_ordered_sum_scratch_bytes() -> int:
@@ -477,5 +498,5 @@ def band_ordered_sum_scratch_bytes() -> int:
 
 
 def band_ordered_sum(u: int, n: int, out: int, scratch: int, stream: int = 0) -> None:
-    check(lib().hk_band_ordered_sum_f64(ctypes.c_void_p(u or None), int(n), ctypes.c_void_p(out),
-                                        ctypes.c_void_p(scratch), ctypes.c_void_p(stream or None)))
+    check(lib().hk_band_ordered_sum_f64(u or None, int(n), out,
+                                        scratch, stream or None))

@@ -24,6 +24,7 @@ from pathlib import Path
 
 from . import _contracts, _core
 from .ir import HawkError
+from .layout import LAYOUTS
 
 def _bound_length(role: str, x, n: int) -> int:
     """The length a slot is bound with: its cells for a lookup plane (the
@@ -72,6 +73,15 @@ def _torch():
     return torch
 
 
+def _current_stream() -> int:
+    """The current HIP stream's handle on the current device."""
+    torch = _torch()
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch.cuda.current_device())
+
+
 def _on(stream: int):
     """A context in which torch's own work (a counter's ``zero_()``, a cell's
     ``fill_()``) is issued on ``stream``, the stream the next launch uses, so
@@ -114,6 +124,8 @@ class DeviceKernel:
         self.finished = None      # the runtime's finish counter when the caller binds none
         self.steps_max = None     # a fast entry's largest trips a sample (one int32 cell)
         self.steps_sum = None     # a fast entry's trips over every sample (one int64 cell)
+        self._major = (sidecar.get("sample_major") or {}).get("planes") or []
+        self._direct = self._direct_plan()
 
     # -- validation ----------------------------------------------------------
     def _real_dtype(self):
@@ -122,6 +134,109 @@ class DeviceKernel:
 
     def caller_planes(self) -> list:
         return [n for n, p in self.planes.items() if not p.get("scratch") and n != FUSED_STEPS_PLANE]
+
+    def _direct_plan(self):
+        """What :meth:`run_direct` checks per plane, in ``arg_spec`` order:
+        ``(name, leading shape, dimensions, dtype)``, the dtype ``None``
+        for a ``Param``.  ``None`` for a kernel whose run is more than its
+        per-sample stage over the caller's planes (team stages, a finish or a
+        trip count, a Grid, tables, planes of the runtime's own)."""
+        torch = _torch()
+        if (self.entry is None or self.team or self.sidecar.get("grid") or self.sidecar.get("finish")
+                or FINISHED_PLANE in self.planes or set(self.planes) != {name for _, name in self.arg_spec}):
+            return None
+        plan = []
+        for _role, name in self.arg_spec:
+            info = self.planes[name]
+            if info["role"] == "uniform":
+                plan.append((name, (), 0, None))
+                continue
+            if info["role"] not in _PER_SAMPLE or info.get("scratch"):
+                return None
+            want = (torch.int32 if info["dtype"] in ("i32", "u32") else torch.bool if info["dtype"] == "bool"
+                    else self._real_dtype())
+            lead = tuple(info["shape"])
+            plan.append((name, lead, len(lead) + 1, want))
+        return plan
+
+    def run_direct(self, arrays: dict, base, count, n_samples, layout, stream) -> bool:
+        """One pass over the planes of a plain call: each plane's type, dtype,
+        place and shape tested, its pointer bound where it moved, the stage
+        launched.  ``False``, with nothing done, where any test fails or the
+        call is not plain: :func:`run`'s general path then runs it or says what
+        is wrong."""
+        plan = self._direct
+        if plan is None or len(arrays) != len(plan) or type(base) is not int:
+            return False
+        if layout is not None and layout not in LAYOUTS:
+            return False
+        tensor = _torch().Tensor
+        n, major, bound = n_samples, None, []
+        for name, lead, dims, dtype in plan:
+            x = arrays.get(name)
+            if dtype is None:
+                if type(x) is not float and type(x) is not int:
+                    return False
+                bound.append(x)
+                continue
+            if type(x) is not tensor or x.dtype is not dtype or not x.is_cuda or not x.is_contiguous():
+                return False
+            shape = x.shape
+            if len(shape) != dims:
+                return False
+            if lead:
+                first, last = shape[1:] == lead, shape[:-1] == lead
+                if layout is None:
+                    if first == last:
+                        return False
+                elif layout == "samples_last":
+                    first = False
+                if not first and (layout == "samples_first" or not last):
+                    return False
+                if major is None:
+                    major = first
+                elif major != first:
+                    return False
+                here = shape[0] if first else shape[-1]
+            else:
+                here = shape[0]
+            if n is None:
+                n = here
+            elif n != here:
+                return False
+            bound.append(x)
+        if n is None or type(n) is not int:
+            return False
+        if count is None:
+            count = n - base
+        if type(count) is not int or base < 0 or count < 0 or base + count > n:
+            return False
+        if major and not self.takes_rows(arrays, self._major, "plain"):
+            return False
+        with self._lock:
+            fn, block, slots = self._rows_stage() if major else (self.entry, self.block, self._held_slots)
+            moved = []
+            for slot, x in enumerate(bound):
+                held = slots[slot]
+                if plan[slot][3] is None:
+                    value = float(x)
+                    if held is None or held[1] != value:
+                        block.bind_value(slot, value)
+                        slots[slot] = ("v", value)
+                    continue
+                ptr, device = x.data_ptr(), x.get_device()
+                if held is not None and held[2] == n and held[3] == device:
+                    if held[1] != ptr:
+                        moved.append(slot)
+                        slots[slot] = ("p", ptr, n, device)
+                    continue
+                block.bind(slot, ptr, n, 1, _contracts.DEVICE_ROCM, device)
+                slots[slot] = ("p", ptr, n, device)
+            if moved:
+                block.rebind(moved, [slots[slot][1] for slot in moved])
+            fn.run(block, base, count, n, threads=self.launch_shape["block"],
+                   per_thread=self.launch_shape["per_thread"], stream=stream)
+        return True
 
     @property
     def automatic(self) -> bool:
@@ -795,6 +910,10 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
     ``layout`` (``"samples_first"`` / ``"samples_last"``) and the markers
     :func:`hawk_amd.samples_first` / :func:`~hawk_amd.samples_last` say which
     axis of a per-sample plane holds the samples (:mod:`hawk_amd.layout`)."""
+    if steps is None and entry == "plain" and type(kernel) is DeviceKernel and kernel._direct is not None:
+        if kernel.run_direct(arrays, base, count, n_samples, layout,
+                             _current_stream() if stream is None else int(getattr(stream, "cuda_stream", stream))):
+            return
     from . import layout as _layout
     torch = _torch()
     if isinstance(kernel, ChainedKernel):
@@ -840,6 +959,15 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
         with _on(int(stream)):
             for dst, copy in write_back:       # a sample-major plane the kernel wrote
                 dst.copy_(copy.movedim(-1, 0))
+
+
+#: The stage label of each team stage's entry (any other is the rows' finish).
+_STEP_LABELS = {_core.ordered_sum: "ordered_sum", _core.ordered_sum_f32: "ordered_sum",
+                _core.band_ordered_sum: "band_ordered_sum", _core.ordered_scatter: "ordered_scatter",
+                _core.ordered_scatter_f32: "ordered_scatter", _core.mm16: "mm16", _core.mm16_f64: "mm16",
+                _core.keyed_ordered_sum: "keyed_sum", _core.keyed_ordered_sum_f32: "keyed_sum",
+                _core.keyed_log_fold: "ordered_fold", _core.keyed_log_fold_f32: "ordered_fold",
+                _core.keyed_sample_sum: "keyed_comp", _core.keyed_sample_sum_f32: "keyed_comp"}
 
 
 class Prepared:
@@ -921,6 +1049,7 @@ class Prepared:
         self.steps = []
         self.before = []
         self.statuses = []
+        self.rows_scratch = None
         for t in kernel.team:
             if t.get("before"):
                 args, status, cells = kernel._fold_clear_args(t, bound)
@@ -979,9 +1108,10 @@ class Prepared:
                                    args))
             else:
                 raise HawkError(f"kernel {kernel.name!r}: unknown team stage {t['op']!r}")
+        self._stages = self._make_stages()
 
     def __call__(self) -> None:
-        for _label, launch in self.stages():
+        for _label, launch in self._stages:
             launch()
 
     def stages(self) -> list:
@@ -989,33 +1119,34 @@ class Prepared:
         (``"fold_clear"``), the per-sample stage (labelled with the kernel's
         name) and each team stage (``"ordered_sum"``, ``"ordered_scatter"``,
         ...); calling every ``launch`` in order is one run."""
-        k = self.kernel
-        out = [("fold_clear", lambda fn=fn, args=args: fn(*args, self.stream)) for fn, args in self.before]
+        return list(self._stages)
+
+    def _make_stages(self) -> list:
+        # The launches hold what they use (the kernel, its blocks, the bound
+        # planes), not this object: a launcher let go frees its planes at once.
+        k, n, stream = self.kernel, self.n, self.stream
+        keep = (k, self.bound, self.rows_scratch)
+
+        def call(fn, args):
+            return lambda fn=fn, args=(*args, stream), keep=keep: fn(*args)
+        out = [("fold_clear", call(fn, args)) for fn, args in self.before]
         if self.fast is not None:
             entry, fn, block, cells = self.fast
             resets = list(cells) + ([self.held_counter] if self.held_counter is not None else [])
 
-            def fast_stage():
-                with _on(self.stream):          # claims from sample 0 again; this call's reports and count
+            def fast_stage(keep=keep):
+                with _on(stream):               # claims from sample 0 again; this call's reports and count
                     for c in resets:
                         c.zero_()
-                k._launch_fast(entry, fn, block, 0, self.n, self.n, self.stream)
+                k._launch_fast(entry, fn, block, 0, n, n, stream)
             out.append((f"{k.name}_{entry}", fast_stage))
             return out
         if k.entry is not None:
-            def stage():
-                k.entry.run(self.block, 0, self.n, self.n, threads=k.launch_shape["block"],
-                            per_thread=k.launch_shape["per_thread"], stream=self.stream)
-            out.append((k.name, stage))
-        labels = {_core.ordered_sum: "ordered_sum", _core.ordered_sum_f32: "ordered_sum",
-                  _core.band_ordered_sum: "band_ordered_sum",
-                  _core.ordered_scatter: "ordered_scatter", _core.ordered_scatter_f32: "ordered_scatter",
-                  _core.mm16: "mm16", _core.mm16_f64: "mm16",
-                  _core.keyed_ordered_sum: "keyed_sum", _core.keyed_ordered_sum_f32: "keyed_sum", _core.keyed_log_fold: "ordered_fold", _core.keyed_log_fold_f32: "ordered_fold",
-                  _core.keyed_sample_sum: "keyed_comp", _core.keyed_sample_sum_f32: "keyed_comp"}
+            launch = k.entry.prepared(self.block, 0, n, n, threads=k.launch_shape["block"],
+                                      per_thread=k.launch_shape["per_thread"], stream=stream)
+            out.append((k.name, lambda launch=launch, keep=keep: launch()))
         for fn, args in self.steps:
-            label = labels.get(fn, "row_sum")
-            out.append((label, lambda fn=fn, args=args: fn(*args, self.stream)))
+            out.append((_STEP_LABELS.get(fn, "row_sum"), call(fn, args)))
         return out
 
     def check(self) -> None:

@@ -257,3 +257,60 @@ def test_sample_major_stage(tmp_path, gpu, mode, n):
                 assert torch.equal(part[name][..., 5:n - 55], x[..., 5:n - 55])
                 assert torch.equal(part[name][..., :5], ins[name][..., :5])
                 assert torch.equal(part[name][..., n - 55:], ins[name][..., n - 55:])
+
+
+def test_plain_calls_direct_and_general(tmp_path, gpu):
+    """hawk.run's direct path for plain calls and its general path: the same
+    planes or the same refusal, call by call."""
+    import hawk_amd as hawk
+    import torch
+    from hawk_amd import examples as E
+    n = 1001
+    direct, general = (_unit(tmp_path, [E.scale, E.energy_vjp, E.spd_solve]) for _ in range(2))
+    for k in general:
+        k._direct = None
+    for k in direct:
+        assert k._direct is not None
+
+    def t(*shape, dtype=torch.float64, device=gpu):
+        return torch.randn(*shape, dtype=torch.float64, generator=torch.Generator().manual_seed(3)).to(dtype).to(device)
+    x, v, bar = t(n), t(3, n), t(n)
+    scale = dict(x=x, a=2.0, b=1.0)
+    vjp = dict(v=v, bar_out=bar, bar_v=t(3, n))
+    rows = dict(v=v.t().contiguous(), bar_out=bar, bar_v=t(n, 3))
+    a = t(6, 6, 6) + 20.0 * torch.eye(6, dtype=torch.float64, device=gpu)[:, :, None]
+    calls = [(0, dict(scale, out=t(n))), (0, dict(scale, out=t(n), base=7, count=500)),
+             (0, dict(scale, out=t(n), base=7)), (0, dict(scale, out=t(n), count=0)), (0, dict(scale, a=3, out=t(n))),
+             (0, dict(scale, out=t(n), n_samples=n)), (0, dict(scale, out=t(n), n_samples=n - 1)),
+             (0, dict(scale, out=t(n), base=-1)), (0, dict(scale, out=t(n), count=n + 1)),
+             (0, dict(scale, out=t(n), base=True)), (0, dict(scale, a=True, out=t(n))),
+             (0, dict(scale, a=np.float64(2.0), out=t(n))), (0, dict(scale, a=x, out=t(n))),
+             (0, dict(scale)), (0, dict(scale, out=t(n), other=x)), (0, dict(scale, out=t(n - 1))),
+             (0, dict(scale, out=t(n, 1))), (0, dict(scale, out=t(n, dtype=torch.float32))),
+             (0, dict(scale, out=t(n, device="cpu"))), (0, dict(scale, out=t(2 * n)[::2])),
+             (0, dict(scale, out=torch.nn.Parameter(t(n)))), (0, dict(x=t(0), a=1.0, b=1.0, out=t(0))),
+             (0, dict(scale, out=t(n), layout="rows")), (0, dict(scale, out=t(n), steps=1)),
+             (0, dict(scale, out=t(n), entry="range")), (0, dict(scale, out=t(n), stream=torch.cuda.Stream())),
+             (1, vjp), (1, rows), (1, dict(vjp, layout="samples_last")), (1, dict(rows, layout="samples_first")),
+             (1, dict(rows, layout="samples_last")), (1, dict(vjp, layout="samples_first")),
+             (1, dict(vjp, v=rows["v"])), (1, dict(rows, v=hawk.samples_first(rows["v"]))),
+             (1, dict(v=t(3, 3), bar_out=t(3), bar_v=t(3, 3))),
+             (1, dict(v=t(3, 3), bar_out=t(3), bar_v=t(3, 3), layout="samples_first")),
+             (1, dict(v=t(3, 3), bar_out=t(3), bar_v=t(3, 3), layout="samples_last")),
+             (2, dict(A=a, b=t(6, 6), x=t(6, 6))), (2, dict(A=a, b=t(6, 6), x=t(6, 6), layout="samples_last")),
+             (2, dict(A=a.movedim(-1, 0).contiguous(), b=t(6, 6), x=t(6, 6), layout="samples_first"))]
+    for which, call in calls * 2:                    # twice: fresh and held bindings
+        done = []
+        for k in (direct[which], general[which]):
+            # fresh output planes a side, the same values in both
+            planes = {name: p.clone() if isinstance(p, torch.Tensor) and p.is_contiguous()
+                      and name in ("out", "bar_v", "x") and which + (name == "out") else p for name, p in call.items()}
+            torch.cuda.synchronize()
+            try:
+                hawk.run(k, **planes)
+                torch.cuda.synchronize()
+                done.append({name: p.detach().cpu().numpy().tobytes() for name, p in planes.items()
+                             if isinstance(p, torch.Tensor)})
+            except Exception as e:
+                done.append((type(e), str(e)))
+        assert done[0] == done[1], (which, {name: getattr(p, "shape", p) for name, p in call.items()}, done)
