@@ -1065,11 +1065,11 @@ __global__ __launch_bounds__(256) void hawk_scatter_cells(const T* __restrict__ 
 //   tile of 4096 lanes is split stably into buckets in one pass: window keys
 //   0..31 each a bucket of their own, keys 32..kSplitHot-1 fifteen classes by
 //   (key - 32) % 15, and keys from kSplitHot up one bucket per tail range of
-//   kTailRange keys.  Wave 0 then folds the head buckets (lane c the chain of
-//   key c over its contiguous run) and wave w class w - 1 (64 entries at a
-//   time: equal keys find each other, and the lowest lane adds its group in
-//   lane order onto the key's accumulator; a wave's LDS operations complete in
-//   issue order, so a key's groups meet the accumulator window after window).
+//   kTailRange keys.  Waves 0..7 then add the head buckets' chains, four a
+//   wave, and wave w > 0 folds class w - 1 (64 entries at a time: equal keys
+//   find each other, and the lowest lane adds its group in lane order onto the
+//   key's accumulator; a wave's LDS operations complete in issue order, so a
+//   key's groups meet the accumulator window after window).
 //   The tail buckets go from registers to the tile's slot of the chunk's bin,
 //   with the offset of each range.
 // * hawk_split_tail: one workgroup of 8 waves per (chunk, tail range), the
@@ -1103,9 +1103,8 @@ static_assert(kSplitNone >= kHotStride && kSplitNone >= kTailStride, "the no-buc
 static_assert(kTailRange < (1 << 16), "bins hold window-local keys as u16");
 
 constexpr int kSplitPad = 72;                    // entries read (and ignored) past a run's end
+constexpr int kPeerBlock = 4;                    // a key's peers read at once (at most kPeerBlock - 1 past their run)
 constexpr unsigned kPeerSlots = 128;             // hawk_split_hot's match slots a wave: class-index bits 0..6
-constexpr int kHeadBlock = 8;                    // a head chain's reads in flight: four blocks of kHeadBlock
-static_assert(4 * kHeadBlock <= kSplitPad, "a head chain reads at most kSplitPad entries past its run");
 
 // A split walk workgroup's LDS: Waves waves, Window accumulators, count rows
 // of Stride buckets, and the split tile (Waves * 256 entries); Peers match
@@ -1268,71 +1267,66 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
 }
 
-// The head keys' chains, by one wave: lane c (c < kSplitHeads) adds bucket c
-// (window key c: one contiguous run, lane order) onto acc[c], one addition at
-// a time from its own registers.  Its reads run 32 values ahead of its adds
-// in four rotating blocks of 8, so the chain waits on the adds' latency, not
-// on the LDS.  A lane's loop ends with its run; the wave runs as long as the
-// longest run.  Reads go at most 63 entries past a run's end (the padding).
-template <class T>
-__device__ __forceinline__ void head_block(T (&r)[kHeadBlock], T& a, const T* src) {
-#pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q) a = a + r[q];
-    // the block's next reads go into the registers its adds just used: no
-    // copies, so the other blocks' reads stay in flight
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q) r[q] = src[q];
-    __builtin_amdgcn_sched_barrier(0);
+// a + x0 + x1 + ... + x15, one addition at a time, x_q the value lane q of
+// each row of 16 lanes holds: every row adds its own lanes' values, each
+// handed to the whole row by the add itself (DPP row_newbcast), so a value
+// costs one instruction and no LDS read: 4.9 cycles an add on MI355X (5.6
+// in float32), where a chain fed from LDS takes 11 to 25 and one fed by
+// readlane 13.5.  The fp64 add is the fused x * 1 + a, which rounds x + a once.
+// The leading s_nop covers a DPP read's wait on the lane's last write of x.
+__device__ __forceinline__ double row_chain(double a, double x) {
+    const double one = 1.0;
+#define HK_STEP(q) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #q " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" HK_STEP(0) HK_STEP(1) HK_STEP(2) HK_STEP(3) HK_STEP(4) HK_STEP(5) HK_STEP(6) HK_STEP(7)
+        HK_STEP(8) HK_STEP(9) HK_STEP(10) HK_STEP(11) HK_STEP(12) HK_STEP(13) HK_STEP(14) HK_STEP(15)
+        : "+v"(a) : "v"(x), "v"(one));
+#undef HK_STEP
+    return a;
+}
+__device__ __forceinline__ float row_chain(float a, float x) {
+#define HK_STEP(q) "v_add_f32_dpp %0, %1, %0 row_newbcast:" #q " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" HK_STEP(0) HK_STEP(1) HK_STEP(2) HK_STEP(3) HK_STEP(4) HK_STEP(5) HK_STEP(6) HK_STEP(7)
+        HK_STEP(8) HK_STEP(9) HK_STEP(10) HK_STEP(11) HK_STEP(12) HK_STEP(13) HK_STEP(14) HK_STEP(15)
+        : "+v"(a) : "v"(x));
+#undef HK_STEP
+    return a;
 }
 
+// The chains of the split tile's head buckets c .. c + 3 (a key each: one
+// contiguous run, lane order), by one wave: row r of 16 lanes adds bucket
+// c + r onto acc[c + r], one addition at a time through row_chain, 64 values a
+// step with the next step's reads in flight.  The wave runs as long as the
+// longest of its four runs; a run that has ended adds +0.0, which changes no
+// sum (none is ever -0.0: each started at +0.0).  A lane a chain, 32 values of
+// its own ahead, took 2^23 lanes into 64 Zipf cells 80.7 us against 72.2.
 template <class T, class Sh>
-__device__ void fold_heads(Sh& sh) {
+__device__ __forceinline__ void fold_heads(Sh& sh, int c) {
     const int lane = threadIdx.x & 63;
-    if (lane >= kSplitHeads) return;
-    const int s = static_cast<int>(sh.bstart[lane]);
-    const int e = static_cast<int>(sh.bstart[lane + 1]);
-    if (s >= e) return;
-    T a = sh.acc[lane];
-    T r0[kHeadBlock], r1[kHeadBlock], r2[kHeadBlock], r3[kHeadBlock];
-    const T* x = sh.val + s;
-    // the first reads in block order, as the loop issues them: the loop's
-    // waits count LDS operations, and on its entry they follow this order
-    __builtin_amdgcn_sched_barrier(0);
+    const int k = c + (lane >> 4);
+    const int s = static_cast<int>(sh.bstart[k]) + (lane & 15);
+    const int e = static_cast<int>(sh.bstart[k + 1]);
+    const int own = static_cast<int>(sh.bstart[k + 1] - sh.bstart[k]);
+    const int top = max(__builtin_amdgcn_readlane(own, 0), __builtin_amdgcn_readlane(own, 16));
+    const int low = max(__builtin_amdgcn_readlane(own, 32), __builtin_amdgcn_readlane(own, 48));
+    const int longest = max(top, low);
+    if (longest == 0) return;
+    T a = sh.acc[k];
+    T x[4];
+    auto load = [&](int m) {                         // in bounds past the run: its end is at most the tile's
 #pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q) r0[q] = x[q];
-    __builtin_amdgcn_sched_barrier(0);
+        for (int q = 0; q < 4; ++q) x[q] = sh.val[min(s + m + 16 * q, e)];
+    };
+    load(0);
+    for (int m = 0; m < longest; m += 64) {
+        T y[4];
 #pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q) r1[q] = x[kHeadBlock + q];
-    __builtin_amdgcn_sched_barrier(0);
+        for (int q = 0; q < 4; ++q) y[q] = s + m + 16 * q < e ? x[q] : T(0);
+        load(m + 64);
 #pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q) r2[q] = x[2 * kHeadBlock + q];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q) r3[q] = x[3 * kHeadBlock + q];
-    __builtin_amdgcn_sched_barrier(0);
-    constexpr int kAhead = 4 * kHeadBlock;
-    int left = e - s;
-    for (; left >= kAhead; left -= kAhead, x += kAhead) {
-        head_block(r0, a, x + kAhead);
-        head_block(r1, a, x + kAhead + kHeadBlock);
-        head_block(r2, a, x + kAhead + 2 * kHeadBlock);
-        head_block(r3, a, x + kAhead + 3 * kHeadBlock);
+        for (int q = 0; q < 4; ++q)
+            if (m + 16 * q < longest) a = row_chain(a, y[q]);
     }
-    // fewer than kAhead left, held in r0..r3 in order
-#pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q)
-        if (q < left) a = a + r0[q];
-#pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q)
-        if (kHeadBlock + q < left) a = a + r1[q];
-#pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q)
-        if (2 * kHeadBlock + q < left) a = a + r2[q];
-#pragma unroll
-    for (int q = 0; q < kHeadBlock; ++q)
-        if (3 * kHeadBlock + q < left) a = a + r3[q];
-    sh.acc[lane] = a;
+    if ((lane & 15) == 0) sh.acc[k] = a;
 }
 
 // The caller's wave folds class c of the split tile, 64 entries a window in
@@ -1341,10 +1335,18 @@ __device__ void fold_heads(Sh& sh) {
 // through the wave's match table: bits 0..6 of m pick one of kPeerSlots
 // slots, every lane ORs its bit into its slot, and three ballots over bits
 // 7..9 keep the lanes whose whole key is equal.  The lowest lane of each key
-// adds its own value and then its peers' (read back from the class's run, in
-// lane order) onto the accumulator it read with the match.  A wave's LDS
-// operations complete in issue order, so a key's windows meet its
-// accumulator one after another.
+// adds its own value onto the accumulator it read with the match.  Where no
+// key has more than one peer, the peer then adds its value onto what that lane
+// left.  Otherwise every key's peers move, in lane order, to a run of their own
+// in the window's place (a scan over the keys' peer counts gives the runs'
+// starts), and the lowest lane adds its run from consecutive reads: finding
+// each peer in the match mask instead (count trailing zeros, clear the bit)
+// took most of a window's instructions.  A wave's LDS operations complete in
+// issue order, so a key's windows meet its accumulator one after another.
+// With the head chains by rows, on MI355X in float64: 2^23 lanes into 64
+// uniform cells 120.5 -> 82.1 us, into 64 Zipf cells 99.0 -> 72.2, into 4096
+// uniform cells 84.6 -> 73.7, 2^26 Zipf lanes into 65536 cells 571 -> 524, and
+// the wide walk's 2^22 lanes into 2^18 cells 74.0 -> 68.4.
 template <class T, class Sh, bool Hot>
 __device__ void fold_class(Sh& sh, int c) {
     const int wave = threadIdx.x >> 6;
@@ -1381,48 +1383,55 @@ __device__ void fold_class(Sh& sh, int c) {
         if (valid) peer[h] = 0ull;
 #pragma unroll
         for (int bit = kLow; bit < kBits; ++bit) {
-            const bool one = (m >> bit) & 1u;
-            const unsigned long long ones = __ballot(valid && one);
-            pm &= one ? ones : ~ones;
+            const unsigned long long ones = __ballot(valid && ((m >> bit) & 1u));
+            const unsigned long long own = 0ull - static_cast<unsigned long long>((m >> bit) & 1u);
+            pm &= ~(ones ^ own);
         }
-        if (valid && (pm & (me - 1ull)) == 0ull) {
-            // the key's lowest lane: its value, then its peers' in lane order
-            T a = a0 + x;
-            unsigned long long rest = pm & ~me;
-            while (rest != 0ull) {
-                T y[8];
-                int got = 0;
+        // equal keys below this lane: 0 for a key's lowest lane (and a lane past the run)
+        const unsigned rank = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(pm >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(pm), 0u));
+        T a = a0 + x;
+        const unsigned long long more = __ballot(rank > 1u);
+        if (more != 0ull) {
+            // a key has several peers: each key's to a run of their own in the window's place
+            const int peers = valid && rank == 0u ? static_cast<int>(__popcll(pm)) - 1 : 0;
+            const int start = static_cast<int>(wave_inclusive_scan(static_cast<unsigned>(peers))) - peers;
+            const int low = pm != 0ull ? static_cast<int>(__builtin_ctzll(pm)) : 0;
+            const int run = __builtin_amdgcn_ds_bpermute(low << 2, start);
+            if (rank != 0u) sh.val[base + run + static_cast<int>(rank) - 1] = x;
+            __builtin_amdgcn_wave_barrier();
+            const T* y = sh.val + base + start;
+            for (int left = peers; left > 0; left -= kPeerBlock, y += kPeerBlock) {
+                T r[kPeerBlock];
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    if (rest != 0ull) {
-                        y[q] = sh.val[base + static_cast<int>(__builtin_ctzll(rest))];
-                        rest &= rest - 1ull;
-                        got = q + 1;
-                    }
-                }
+                for (int q = 0; q < kPeerBlock; ++q) r[q] = y[q];
 #pragma unroll
-                for (int q = 0; q < 8; ++q)
-                    if (q < got) a = a + y[q];
+                for (int q = 0; q < kPeerBlock; ++q) a = a + (q < left ? r[q] : T(0));
             }
+        }
+        if (valid && rank == 0u) {
             sh.acc[ai] = a;
         }
+        __builtin_amdgcn_wave_barrier();
+        // at most one peer a key: it adds onto what its key's lowest lane left
+        if (more == 0ull && rank != 0u) sh.acc[ai] = sh.acc[ai] + x;
         __builtin_amdgcn_wave_barrier();
         k = nk;
         x = nx;
     }
 }
 
-// The split tile's folds in hawk_split_hot: wave 0 the head keys' chains,
-// wave w (1..15) class w - 1.  A class wave first clears its match table (it
-// shares LDS with the split's tables); each window leaves it clear.
+// The split tile's folds in hawk_split_hot: wave w the chains of the head keys
+// 4w .. 4w + 3 (w < 8), then (w > 0) class w - 1: a skewed histogram's first
+// four keys run longest, and wave 0 has nothing but them.  A class wave first
+// clears its match table (it shares LDS with the split's tables); each window
+// leaves it clear.
 template <class T>
 __device__ void split_fold(HotShared<T>& sh) {
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
-    if (wave == 0) {
-        fold_heads<T>(sh);
-        return;
-    }
+    if (4 * wave < kSplitHeads) fold_heads<T>(sh, 4 * wave);
+    if (wave == 0) return;
 #pragma unroll
     for (unsigned i = 0; i < kPeerSlots; i += 64) sh.f.peer[wave][i + lane] = 0ull;
     __builtin_amdgcn_wave_barrier();
@@ -1636,31 +1645,6 @@ struct TailRanges {
 };
 constexpr int kWideSingles = kTailWaves;         // 8: a wave each
 constexpr int kWideOctaves = 7;                  // [8, 16) .. [512, 1024)
-
-// a + x0 + x1 + ... + x15, one addition at a time, x_q the value lane q of
-// each row of 16 lanes holds: every row adds its own lanes' values, each
-// handed to the whole row by the add itself (DPP row_newbcast), so a value
-// costs one instruction and no LDS read: 4.9 cycles an add on MI355X (5.6
-// in float32), where a chain fed from LDS takes 11 to 25 and one fed by
-// readlane 13.5.  The fp64 add is the fused x * 1 + a, which rounds x + a once.
-// The leading s_nop covers a DPP read's wait on the lane's last write of x.
-__device__ __forceinline__ double row_chain(double a, double x) {
-    const double one = 1.0;
-#define HK_STEP(q) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #q " row_mask:0xf bank_mask:0xf\n\t"
-    asm("s_nop 1\n\t" HK_STEP(0) HK_STEP(1) HK_STEP(2) HK_STEP(3) HK_STEP(4) HK_STEP(5) HK_STEP(6) HK_STEP(7)
-        HK_STEP(8) HK_STEP(9) HK_STEP(10) HK_STEP(11) HK_STEP(12) HK_STEP(13) HK_STEP(14) HK_STEP(15)
-        : "+v"(a) : "v"(x), "v"(one));
-#undef HK_STEP
-    return a;
-}
-__device__ __forceinline__ float row_chain(float a, float x) {
-#define HK_STEP(q) "v_add_f32_dpp %0, %1, %0 row_newbcast:" #q " row_mask:0xf bank_mask:0xf\n\t"
-    asm("s_nop 1\n\t" HK_STEP(0) HK_STEP(1) HK_STEP(2) HK_STEP(3) HK_STEP(4) HK_STEP(5) HK_STEP(6) HK_STEP(7)
-        HK_STEP(8) HK_STEP(9) HK_STEP(10) HK_STEP(11) HK_STEP(12) HK_STEP(13) HK_STEP(14) HK_STEP(15)
-        : "+v"(a) : "v"(x));
-#undef HK_STEP
-    return a;
-}
 
 // Chunk b's chain of single key k, by one wave: the key's segment of every
 // tile slot in tile order, 256 values a step through the wave's LDS (so each

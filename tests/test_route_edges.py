@@ -87,6 +87,40 @@ def test_ordered_scatter_walks(tmp_path, gpu, mode, cells, n, keys):
         assert acc.cpu().numpy().tobytes() == want.tobytes()
 
 
+@pytest.mark.parametrize("mode", ["float64", "float32"])
+@pytest.mark.parametrize("cells, n", [(33, 4097), (64, 64 * 300 + 5), (1000, 1000 * 256 + 63), (20_000, 20_000 * 192)])
+@pytest.mark.parametrize("each", [1, 2, 3, 5, 8, 9, 64, "heads"])
+def test_ordered_scatter_peers(gpu, mode, cells, n, each):
+    """Windows whose keys have no peers, one, a block's worth, one more and a
+    whole window's, and head keys of unequal runs: the serial walk's bits,
+    negative zeros among the values."""
+    import oracle_lib as O
+    import torch
+    from hawk_amd import _core
+    dt = np.float32 if mode == "float32" else np.float64
+    g = np.random.default_rng(cells + n)
+    if each == "heads":
+        key = np.minimum(g.geometric(0.5, n) - 1, 32)
+    else:
+        # a stride of 15 and of 8 keeps neighbours in one class of either split
+        key = (np.arange(n) // each * 120) % cells
+        key[n // 2:] = np.roll(key[n // 2:], 7)
+    key = key.astype(np.int32)
+    x = (g.normal(size=n) * np.exp(g.normal(size=n))).astype(dt)
+    x[::3] = -0.0
+    acc0 = np.full(cells, -0.0, dt)
+    want, _ = O.ordered_scatter(key, x, acc0)
+    fn = _core.ordered_scatter_f32 if mode == "float32" else _core.ordered_scatter
+    kd, xd, acc = (torch.from_numpy(a).to(gpu) for a in (key, x, acc0))
+    scratch = torch.empty(_core.ordered_scatter_scratch_bytes(n, cells), dtype=torch.uint8, device=gpu)
+    status = torch.zeros(257, dtype=torch.int32, device=gpu)
+    print(f"scatter peers cells={cells} n={n} each={each} {mode}", flush=True)
+    fn(kd.data_ptr(), xd.data_ptr(), n, acc.data_ptr(), cells, scratch.data_ptr(), status.data_ptr(),
+       torch.cuda.current_stream().cuda_stream)
+    assert acc.cpu().numpy().tobytes() == want.tobytes()
+    assert not status[1:].any()
+
+
 def _per_key(group, policy):
     import hawk_amd as hawk
     from hawk_amd import Grid, Kernel, Scalar
