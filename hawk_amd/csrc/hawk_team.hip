@@ -1813,8 +1813,9 @@ constexpr int kWideGroups = 2048;                // workgroups hawk_split_tail g
 // 225 / 238; 20000 cells in 104 chunks 73 / 51, in 209 83 / 87.  Up to 12288
 // cells (no tail ranges) a chunk is at most three tiles: 10000 cells in 20
 // chunks 29 / 23, in 50 31 / 34; 4000 cells in 16 chunks 16 / 18.  Past 65536
-// cells, against the sorted walk this replaced: 2^18 cells, 2^22 lanes 1470 us
-// uniform and 1395 us Zipf -> 74 and 166 us.
+// cells, against a sorted walk of each chunk: 2^18 cells, 2^22 lanes 1470 us uniform
+// and 1395 us Zipf -> 74 and 166 us (uniform 68 since the folds gather peers
+// into runs, which both walks share).
 bool wide_walk(int64_t cells, int chunks) {
     return cells > kSplitCells || chunks < (cells > kSplitHot ? 192 : cells > 2 * kTile ? 32 : 0);
 }
