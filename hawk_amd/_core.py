@@ -211,7 +211,7 @@ class ArgBlock:
         self._h = handle
         self.descriptor = list(descriptor)
         self._values = []
-        self._swap = None
+        self._swap = []
 
     @property
     def size(self) -> int:
@@ -236,16 +236,22 @@ class ArgBlock:
         n = len(slots)
         if len(ptrs) != n:
             raise ValueError("hawk_core.ArgBlock.rebind: slots and ptrs must be the same length")
-        # the (slot, pointer) arrays are made once and reused by every call (the
-        # caller's lock keeps a block to one thread at a time)
-        if self._swap is None or len(self._swap[0]) < n:
+        # the (slot, pointer) arrays are made once and taken by one call at a
+        # time; a call of another thread meanwhile makes a pair of its own
+        try:
+            pair = self._swap.pop()
+        except IndexError:
+            pair = None
+        if pair is None or len(pair[0]) < n:
             size = max(1, n, len(self.descriptor))
-            self._swap = (ctypes.c_int64 * size)(), (ctypes.c_int64 * size)()
-        s, p = self._swap
+            pair = (ctypes.c_int64 * size)(), (ctypes.c_int64 * size)()
+        s, p = pair
         for i in range(n):
             s[i] = int(slots[i])
             p[i] = int(ptrs[i])
-        check(lib().hk_rebind(self._h, s, p, n), ValueError)
+        rc = lib().hk_rebind(self._h, s, p, n)
+        self._swap.append(pair)
+        check(rc, ValueError)
 
     @property
     def handle(self):

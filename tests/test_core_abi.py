@@ -69,6 +69,24 @@ def test_argblock_bind_and_rebind_refusals():
     ab.rebind([0, 1], [0x5000, 0x6000])
 
 
+def test_a_rebind_within_a_rebind_keeps_its_slots():
+    """A rebind that runs while another fills its arrays (here from a pointer's
+    own conversion, as from another thread) leaves the other's alone: the
+    refused by-value slot of the inner one is not the outer one's."""
+    ab = _core.ArgBlock(["gref", "handle", "f64"])
+    ab.bind(0, 0x1000, 128)
+    ab.bind(1, 0x2000, 128)
+    ab.bind_value(2, 2.5)
+    ab.rebind([0, 1], [0x5000, 0x6000])
+
+    class Pointer:
+        def __int__(self):
+            with pytest.raises(ValueError, match="by-value 'f64' slot"):
+                ab.rebind([2], [0x3000])
+            return 0x7000
+    ab.rebind([0, 1], [0x8000, Pointer()])
+
+
 @pytest.mark.parametrize("slots", [1, 2, 5, 17])
 def test_a_bulk_rebind_is_one_crossing_whatever_the_slot_count(slots):
     """The rebind arm of the reference's launch-crossing card
