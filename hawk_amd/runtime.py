@@ -215,7 +215,7 @@ class DeviceKernel:
             return False
         with self._lock:
             fn, block, slots = self._rows_stage() if major else (self.entry, self.block, self._held_slots)
-            moved = []
+            moved, ptrs = [], []
             for slot, x in enumerate(bound):
                 held = slots[slot]
                 if plan[slot][3] is None:
@@ -228,12 +228,13 @@ class DeviceKernel:
                 if held is not None and held[2] == n and held[3] == device:
                     if held[1] != ptr:
                         moved.append(slot)
-                        slots[slot] = ("p", ptr, n, device)
+                        ptrs.append(ptr)
                     continue
                 block.bind(slot, ptr, n, 1, _contracts.DEVICE_ROCM, device)
                 slots[slot] = ("p", ptr, n, device)
             if moved:
-                block.rebind(moved, [slots[slot][1] for slot in moved])
+                # noted as held once swapped: a Param that no float holds raises above
+                self._swap(block, slots, moved, ptrs)
             fn.run(block, base, count, n, threads=self.launch_shape["block"],
                    per_thread=self.launch_shape["per_thread"], stream=stream)
         return True

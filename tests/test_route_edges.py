@@ -348,3 +348,24 @@ def test_plain_calls_direct_and_general(tmp_path, gpu):
             except Exception as e:
                 done.append((type(e), str(e)))
         assert done[0] == done[1], (which, {name: getattr(p, "shape", p) for name, p in call.items()}, done)
+
+
+def test_refused_param_leaves_bindings(tmp_path, gpu):
+    """A call refused at a Param, after a plane before it has moved, leaves the
+    binding of the last run: the next call over the moved plane reads it."""
+    import hawk_amd as hawk
+    import torch
+    from hawk_amd import examples as E
+    scale, = _unit(tmp_path, [E.scale])
+    first, second = (torch.full((1001,), value, dtype=torch.float64, device=gpu) for value in (1.0, 5.0))
+    out = torch.empty_like(first)
+    hawk.run(scale, x=first, a=2.0, b=1.0, out=out)
+    want = out.clone()
+    hawk.run(scale, x=second, a=2.0, b=1.0, out=out)
+    moved = out.clone()
+    assert not torch.equal(want, moved)
+    hawk.run(scale, x=first, a=2.0, b=1.0, out=out)
+    with pytest.raises(OverflowError):
+        hawk.run(scale, x=second, a=10 ** 400, b=1.0, out=out)
+    hawk.run(scale, x=second, a=2.0, b=1.0, out=out)
+    assert torch.equal(out, moved)
