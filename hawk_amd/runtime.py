@@ -19,6 +19,7 @@ the kernel's lock over bind and launch (reference ``hawk/runtime.py:46-53``).
 from __future__ import annotations
 
 import json
+import math
 import threading
 from pathlib import Path
 
@@ -71,6 +72,13 @@ FAST_MAX = 1 << 30
 def _torch():
     import torch
     return torch
+
+
+def _holds(held, value: float) -> bool:
+    """Whether a by-value slot's entry ``("v", number)`` is ``value``, the sign
+    of a zero included (0.0 == -0.0, but 1/a and a*x tell them apart)."""
+    return held is not None and held[1] == value and (value != 0.0 or
+                                                      math.copysign(1.0, held[1]) == math.copysign(1.0, value))
 
 
 def _current_stream() -> int:
@@ -220,7 +228,7 @@ class DeviceKernel:
                 held = slots[slot]
                 if plan[slot][3] is None:
                     value = float(x)
-                    if held is None or held[1] != value:
+                    if not _holds(held, value):
                         block.bind_value(slot, value)
                         slots[slot] = ("v", value)
                     continue
@@ -610,7 +618,7 @@ class DeviceKernel:
             held = slots[slot]
             if kind in ("f64", "f32"):
                 value = float(x)
-                if held != ("v", value):
+                if not _holds(held, value):
                     block.bind_value(slot, value)
                     slots[slot] = ("v", value)
                 continue

@@ -369,3 +369,26 @@ def test_refused_param_leaves_bindings(tmp_path, gpu):
         hawk.run(scale, x=second, a=10 ** 400, b=1.0, out=out)
     hawk.run(scale, x=second, a=2.0, b=1.0, out=out)
     assert torch.equal(out, moved)
+
+
+@pytest.mark.parametrize("mode", ["float64", "float32"])
+def test_a_param_of_the_other_zero_is_bound(tmp_path, gpu, mode):
+    """A call with -0.0 after one with 0.0 (and the reverse) runs on its own
+    zero, on the direct path and the general one: 1 * a keeps the sign."""
+    import hawk_amd as hawk
+    import torch
+    from hawk_amd import Param, Scalar
+
+    @hawk.kernel
+    def times(x: Scalar, a: Param) -> Scalar:
+        return x * a
+    x = torch.ones(100, dtype=torch.float32 if mode == "float32" else torch.float64, device=gpu)
+    for direct in (True, False):
+        (k,) = _unit(tmp_path, [times], mode)
+        if not direct:
+            k._direct = None
+        for a in (0.0, -0.0, -0.0, 0.0, 1.0, -0.0, 0):
+            out = torch.full_like(x, 7.0)
+            hawk.run(k, x=x, a=a, out=out)
+            want = np.full(100, a, out.cpu().numpy().dtype)
+            assert out.cpu().numpy().tobytes() == want.tobytes(), (direct, a)
