@@ -525,15 +525,27 @@ class DeviceKernel:
         cell (``hawk.sum`` of a vector commits one entry a column)."""
         return out.data_ptr() + (t.get("column") or 0) * out.element_size()
 
-    def _row_finish_args(self, bound: dict, n: int, device, stream: int) -> tuple:
-        """``(jobs, rows, f32, scratch)`` of the finish of every reduction whose
-        rows the stage writes (:func:`hawk_amd._core.rows_finish_many`):
+    def _row_calls(self, bound: dict) -> dict:
+        """The row reductions finished by each call, by the first of them: all
+        in one call where every reduction has a cell of its own.  Cells that
+        share memory are written one after another, in the kernel's order, so
+        the last reduction's value stays."""
+        if len(self._row_ops) > 1:
+            cells = [self._cell_ptr(t, bound[t["out"]]) for t in self.team
+                     if "out" in t and self.planes[t["out"]]["role"] == "cell"]
+            if len(set(cells)) != len(cells):
+                return {id(t): [t] for t in self._row_ops}
+        return {id(t): self._row_ops for t in self._row_ops[:1]}
+
+    def _row_finish_args(self, ops: list, bound: dict, n: int, device, stream: int) -> tuple:
+        """``(jobs, rows, f32, scratch)`` of the finish of the reductions ``ops``,
+        whose rows the stage writes (:func:`hawk_amd._core.rows_finish_many`):
         compensated (hi, comp) rows, band rows (hi, lo) in the banded mode, or
         one extreme a row (``hawk.max`` / ``hawk.min``).  The rows are the
         stage's Real, so the finish runs in it."""
         rows = -(-n // 32)
-        jobs = (_core.RowsJob * len(self._row_ops))()
-        for job, t in zip(jobs, self._row_ops):
+        jobs = (_core.RowsJob * len(ops))()
+        for job, t in zip(jobs, ops):
             job.hi, job.out = bound[t["hi"]].data_ptr(), self._cell_ptr(t, bound[t["out"]])
             if t["op"] == "row_extreme":
                 job.op = _core.ROWS_MAX if t["red"] == "max" else _core.ROWS_MIN
@@ -541,15 +553,15 @@ class DeviceKernel:
                 job.lo = bound[t["comp"]].data_ptr()
                 job.op = _core.ROWS_BAND if t["op"] == "band_rows" else _core.ROWS_SUM
         with _on(stream):
-            scratch = self._buffer(("rows", rows), _core.rows_finish_many_scratch_bytes(rows, len(jobs)), device,
-                                   zero=False)
-        return jobs, rows, self.planes[self._row_ops[0]["hi"]]["dtype"] == "f32", scratch
+            scratch = self._buffer(("rows", rows, len(jobs)), _core.rows_finish_many_scratch_bytes(rows, len(jobs)),
+                                   device, zero=False)
+        return jobs, rows, self.planes[ops[0]["hi"]]["dtype"] == "f32", scratch
 
-    def _row_identities(self, bound: dict, stream: int) -> None:
+    def _row_identities(self, ops: list, bound: dict, stream: int) -> None:
         """A run of no samples leaves each reduction's identity: 0, -inf (max),
         +inf (min)."""
         with _on(stream):
-            for t in self._row_ops:
+            for t in ops:
                 out, col = bound[t["out"]], t.get("column")
                 empty = {"max": float("-inf"), "min": float("inf")}.get(t.get("red"), 0.0)
                 (out.view(-1)[col:col + 1] if col is not None else out).fill_(empty)
@@ -692,6 +704,7 @@ class DeviceKernel:
             self.bind_all(bound, n, block, slots)
             fn.run(block, base, count, n, threads=self.launch_shape["block"],
                    per_thread=self.launch_shape["per_thread"], stream=stream)
+        row_calls = self._row_calls(bound)
         for t in self.team:
             if t.get("before"):
                 continue
@@ -717,12 +730,13 @@ class DeviceKernel:
                 _core.mm16([bound[p].data_ptr() for p in t["in"]], [bound[p].data_ptr() for p in t["out"]],
                            t["products"], n, stream, t.get("dtype", "f32"))
             elif t["op"] in _ROW_OPS:
-                if t is not self._row_ops[0]:
-                    continue                  # the first finishes them all
+                ops = row_calls.get(id(t))
+                if ops is None:
+                    continue                  # finished with an earlier one
                 if n == 0:
-                    self._row_identities(bound, stream)
+                    self._row_identities(ops, bound, stream)
                 else:
-                    jobs, rows, f32, scratch = self._row_finish_args(bound, n, device, stream)
+                    jobs, rows, f32, scratch = self._row_finish_args(ops, bound, n, device, stream)
                     _core.rows_finish_many(jobs, rows, f32, scratch.data_ptr(), stream)
             elif t["op"] == "band_ordered_sum":
                 u = bound[t["u"]]
@@ -1058,7 +1072,8 @@ class Prepared:
         self.steps = []
         self.before = []
         self.statuses = []
-        self.rows_scratch = None
+        self.rows_scratch = []
+        row_calls = kernel._row_calls(bound)
         for t in kernel.team:
             if t.get("before"):
                 args, status, cells = kernel._fold_clear_args(t, bound)
@@ -1087,13 +1102,14 @@ class Prepared:
                         t["products"], self.n)
                 self.steps.append((_core.mm16_f64 if t.get("dtype") == "f64" else _core.mm16, args))
             elif t["op"] in _ROW_OPS:
-                if t is not kernel._row_ops[0]:
-                    continue                  # the first finishes them all
+                ops = row_calls.get(id(t))
+                if ops is None:
+                    continue                  # finished with an earlier one
                 if self.n == 0:
-                    self.steps.append((kernel._row_identities, (bound,)))
+                    self.steps.append((kernel._row_identities, (ops, bound)))
                 else:
-                    jobs, rows, f32, scratch = kernel._row_finish_args(bound, self.n, device, self.stream)
-                    self.rows_scratch = scratch          # alive as long as the launcher
+                    jobs, rows, f32, scratch = kernel._row_finish_args(ops, bound, self.n, device, self.stream)
+                    self.rows_scratch.append(scratch)    # alive as long as the launcher
                     self.steps.append((_core.rows_finish_many, (jobs, rows, f32, scratch.data_ptr())))
             elif t["op"] == "band_ordered_sum":
                 scratch = kernel._buffer(("band_sum", t["out"]), _core.band_ordered_sum_scratch_bytes(), device,

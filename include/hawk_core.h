@@ -250,12 +250,13 @@ int hk_rows_extreme_f32(const float* hi, int64_t rows, int32_t op, float* out,
                         void* scratch, void* stream);
 
 /* The finishes of `count` reductions of one stage, each over `rows` rows, in
- * two launches (one when the rows are a single leaf of 4096): job i folds its
- * rows by op 0 (hk_rows_finish: hi and the compensations lo), 1 or 2
- * (hk_rows_extreme: hi alone), or in float64 3 (hk_band_rows_finish: hi and
- * lo), into *out, the bits of those entries.  Scratch:
- * hk_rows_finish_many_scratch_bytes(rows, count) bytes, no initial contents
- * needed.  HK_EVALUE for rows < 1, another op or a missing plane. */
+ * two launches for every sixteen of them (one when the rows are a single leaf
+ * of 4096): job i folds its rows by op 0 (hk_rows_finish: hi and the
+ * compensations lo), 1 or 2 (hk_rows_extreme: hi alone), or in float64 3
+ * (hk_band_rows_finish: hi and lo), into *out, the bits of those entries.  The
+ * cells are apart from one another: the jobs of a launch have no order.
+ * Scratch: hk_rows_finish_many_scratch_bytes(rows, count) bytes, no initial
+ * contents needed.  HK_EVALUE for rows < 1, another op or a missing plane. */
 typedef struct hk_rows_job {
     const void* hi;
     const void* lo;

@@ -392,3 +392,25 @@ def test_a_param_of_the_other_zero_is_bound(tmp_path, gpu, mode):
             hawk.run(k, x=x, a=a, out=out)
             want = np.full(100, a, out.cpu().numpy().dtype)
             assert out.cpu().numpy().tobytes() == want.tobytes(), (direct, a)
+
+
+@pytest.mark.parametrize("n", [1, 5000, 300_000])
+def test_reductions_into_one_cell_leave_the_last(tmp_path, gpu, n):
+    """Reductions that share a cell are written in the kernel's order."""
+    import hawk_amd as hawk
+    import torch
+    from hawk_amd import Mutable, Scalar
+
+    @hawk.kernel
+    def three(x: Scalar, a: Mutable[Scalar], o: Mutable[Scalar], b: Mutable[Scalar]):
+        a = hawk.sum(x * 2.0)
+        o = hawk.sum(x, policy="ordered")
+        b = hawk.max(x)
+    (k,) = _unit(tmp_path, [three])
+    x = torch.arange(n, dtype=torch.float64, device=gpu) % 1024 + 1.0
+    one, two = (torch.zeros(1, dtype=torch.float64, device=gpu) for _ in range(2))
+    for cells, want in (((one, two, one), x.max()), ((one, one, one), x.max()), ((two, one, one), x.max()),
+                        ((one, one, two), x.sum())):
+        for call in (lambda **p: hawk.run(k, **p), lambda **p: k.prepare(**p)()):
+            call(x=x, a=cells[0], o=cells[1], b=cells[2])
+            assert float(one) == float(want), (n, call)
