@@ -10,10 +10,13 @@ fixed-tree ordered sum, the ordered scatter) on the same HIP stream.
 Ownership as in the reference (``hawk/runtime.py:20-22``, ``:655-696``): the
 planes are the caller's and are written in place; the runtime owns only its
 scratch (term planes of a split kernel, the sum's lane partials, the
-scatter's chunk partials and status plane), made once per sample count.
+scatter's chunk partials and status plane), made once per stream and sample
+count.
 
 Threading: one :class:`DeviceKernel` shared by threads is safe: ``run`` holds
 the kernel's lock over bind and launch (reference ``hawk/runtime.py:46-53``).
+Streams: calls on different streams work in scratch of their own, so they may
+run at once.
 """
 
 from __future__ import annotations
@@ -98,6 +101,28 @@ def _on(stream: int):
     return torch.cuda.stream(torch.cuda.ExternalStream(stream)) if stream else _nullcontext()
 
 
+class _Workspace(dict):
+    """What a kernel's launches on one stream of one GPU work in: its scratch
+    tensors by ``(what, name, *sizes)``, each made when first asked for.  A
+    stream's launches run one after another, so they share these; the launches
+    of another stream, which may run at the same time, have their own."""
+
+    def __init__(self, device):
+        super().__init__()
+        self.device = device
+        self.word = None          # the value the trip-count word holds
+
+    def take(self, key: tuple, shape, dtype, zero: bool = False):
+        held = self.get(key)
+        if held is None:
+            torch = _torch()
+            held = self[key] = (torch.zeros if zero else torch.empty)(shape, dtype=dtype, device=self.device)
+        return held
+
+    def bytes(self, key: tuple, nbytes: int, zero: bool = False):
+        return self.take(key, max(1, nbytes), _torch().uint8, zero)
+
+
 class DeviceKernel:
     """One kernel of a built unit, loaded for the gfx950 target."""
 
@@ -126,7 +151,7 @@ class DeviceKernel:
         # ("v", value); None before the first bind.
         self._held_slots: list = [None] * len(self.arg_spec)
         self._rows = None         # the sample-major stage, bound by the first call that takes it
-        self._scratch: dict = {}
+        self._workspaces: dict = {}
         self._lock = threading.Lock()
         self.scatter_chunks = None
         self.finished = None      # the runtime's finish counter when the caller binds none
@@ -252,33 +277,34 @@ class DeviceKernel:
         """Whether the kernel reads its trip count at launch (``hawk.steps(k, "auto")``)."""
         return (self.sidecar.get("finish") or {}).get("steps") == "auto"
 
-    def _word(self, steps, device, stream: int):
+    def _workspace(self, stream: int, device) -> _Workspace:
+        """The workspace of the launches on ``stream`` of ``device``."""
+        held = self._workspaces.get((stream, device))
+        if held is None:
+            held = self._workspaces.setdefault((stream, device), _Workspace(device))
+        return held
+
+    @property
+    def _scratch(self) -> _Workspace:
+        """The workspace of the current stream."""
+        torch = _torch()
+        return self._workspace(_current_stream(), torch.device("cuda", torch.cuda.current_device()))
+
+    def _word(self, steps, work: _Workspace, stream: int):
         """The trip-count word, set to ``steps`` on ``stream`` (held; rewritten
         only when the value changes)."""
         torch = _torch()
         if isinstance(steps, bool) or not isinstance(steps, int):
             raise HawkError(f"kernel {self.name!r}: steps= is an int (the trips this launch runs), got {steps!r}")
-        held = self._scratch.get(("word", device))
-        if held is None:
-            held = torch.zeros(1, dtype=torch.int32, device=device)
-            self._scratch[("word", device)] = held
-            self._word_value = None
+        held = work.take(("word", ""), 1, torch.int32, zero=True)
         value = max(-(1 << 31), min(steps, (1 << 31) - 1))
-        if getattr(self, "_word_value", None) != value:
+        if work.word != value:
             with _on(stream):
                 held.fill_(value)
-            self._word_value = value
+            work.word = value
         return held
 
-    def _held(self, key, dtype, device):
-        torch = _torch()
-        t = self._scratch.get((key, device))
-        if t is None:
-            t = torch.zeros(1, dtype=dtype, device=device)
-            self._scratch[(key, device)] = t
-        return t
-
-    def _fast(self, entry: str, bound: dict, n: int, chunk: int, device, stream: int, cells=None):
+    def _fast(self, entry: str, bound: dict, n: int, chunk: int, work: _Workspace, stream: int, cells=None):
         """``(DeviceEntry, ArgBlock, cells)`` of the fast entry ``entry`` bound
         to ``bound``.  ``cells`` are its claim counter (the persistent entry's
         only) and report cells (steps max, steps sum), zeroed here on
@@ -296,8 +322,8 @@ class DeviceKernel:
         block = _core.ArgBlock(list(self.sidecar["descriptor"]) + list(FAST_SLOTS[entry]))
         self._bind(block, bound, n)
         if cells is None:
-            cells = (self._held("claims", torch.int32, device), self._held("steps_max", torch.int32, device),
-                     self._held("steps_sum", torch.int64, device))
+            cells = tuple(work.take((what, ""), 1, dtype, zero=True) for what, dtype in
+                          (("claims", torch.int32), ("steps_max", torch.int32), ("steps_sum", torch.int64)))
             self.steps_max, self.steps_sum = cells[1], cells[2]
         with _on(stream):
             for c in cells:
@@ -329,17 +355,13 @@ class DeviceKernel:
         grid = max(1, min(-(-count // threads), PERSIST_BLOCKS))
         fn.run_grid(block, base, count, n, grid, threads, stream=stream)
 
-    def _counter(self, arrays: dict, device):
+    def _counter(self, arrays: dict, work: _Workspace):
         """``arrays`` with the finish counter bound: the caller's, else the
         runtime's own (zeroed by the caller of this method when it wants a count
         per run)."""
         if FINISHED_PLANE not in self.planes or FINISHED_PLANE in arrays:
             return arrays, None
-        torch = _torch()
-        held = self._scratch.get(("finished", device))
-        if held is None:
-            held = torch.zeros(1, dtype=torch.int32, device=device)
-            self._scratch[("finished", device)] = held
+        held = work.take(("finished", ""), 1, _torch().int32, zero=True)
         self.finished = held
         return {**arrays, FINISHED_PLANE: held}, held
 
@@ -511,14 +533,6 @@ class DeviceKernel:
         build's sums and scatters run in float32)."""
         return self.planes[plane]["dtype"] == "f32"
 
-    def _buffer(self, key, nbytes: int, device, zero: bool = True):
-        torch = _torch()
-        held = self._scratch.get(key)
-        if held is None or held.numel() < max(1, nbytes) or held.device != device:
-            held = (torch.zeros if zero else torch.empty)(max(1, nbytes), dtype=torch.uint8, device=device)
-            self._scratch[key] = held
-        return held
-
     @staticmethod
     def _cell_ptr(t: dict, out) -> int:
         """The address of a team stage's cell: entry ``column`` of a vector
@@ -537,7 +551,7 @@ class DeviceKernel:
                 return {id(t): [t] for t in self._row_ops}
         return {id(t): self._row_ops for t in self._row_ops[:1]}
 
-    def _row_finish_args(self, ops: list, bound: dict, n: int, device, stream: int) -> tuple:
+    def _row_finish_args(self, ops: list, bound: dict, n: int, work: _Workspace) -> tuple:
         """``(jobs, rows, f32, scratch)`` of the finish of the reductions ``ops``,
         whose rows the stage writes (:func:`hawk_amd._core.rows_finish_many`):
         compensated (hi, comp) rows, band rows (hi, lo) in the banded mode, or
@@ -552,10 +566,9 @@ class DeviceKernel:
             else:
                 job.lo = bound[t["comp"]].data_ptr()
                 job.op = _core.ROWS_BAND if t["op"] == "band_rows" else _core.ROWS_SUM
-        with _on(stream):
-            scratch = self._buffer(("rows", rows, len(jobs)), _core.rows_finish_many_scratch_bytes(rows, len(jobs)),
-                                   device, zero=False)
-        return jobs, rows, self.planes[ops[0]["hi"]]["dtype"] == "f32", scratch
+        scratch = work.bytes(("rows", ops[0]["hi"], rows, len(jobs)),
+                             _core.rows_finish_many_scratch_bytes(rows, len(jobs)))
+        return jobs, rows, self.planes[ops[0]["hi"]]["dtype"] == "f32", scratch.data_ptr()
 
     def _row_identities(self, ops: list, bound: dict, stream: int) -> None:
         """A run of no samples leaves each reduction's identity: 0, -inf (max),
@@ -566,30 +579,26 @@ class DeviceKernel:
                 empty = {"max": float("-inf"), "min": float("inf")}.get(t.get("red"), 0.0)
                 (out.view(-1)[col:col + 1] if col is not None else out).fill_(empty)
 
-    def _term_plane(self, name: str, n: int, device):
+    def _term_plane(self, name: str, n: int, work: _Workspace):
+        key = ("plane", name, n)
+        held = work.get(key)
+        if held is not None:
+            return held
         torch = _torch()
         info = self.planes[name]
         lead = tuple(info["shape"])
-        key = ("plane", name, n)
-        held = self._scratch.get(key)
-        if held is None or held.device != device:
-            if info.get("rows"):                       # one row partial per `rows` samples, in the stage's Real
-                held = torch.empty(max(1, -(-n // info["rows"])),
-                                   dtype=torch.float32 if info["dtype"] == "f32" else torch.float64, device=device)
-            elif info.get("group"):                    # one entry per key (`group` samples)
-                held = torch.empty(lead + (n // info["group"],), dtype=torch.int32, device=device)
-            else:
-                held = torch.empty(lead + (n,), dtype=torch.int32 if info["dtype"] == "i32" else self._real_dtype(),
-                                   device=device)
-            self._scratch[key] = held
-        return held
+        if info.get("rows"):                       # one row partial per `rows` samples, in the stage's Real
+            return work.take(key, (max(1, -(-n // info["rows"])),),
+                             torch.float32 if info["dtype"] == "f32" else torch.float64)
+        if info.get("group"):                      # one entry per key (`group` samples)
+            return work.take(key, lead + (n // info["group"],), torch.int32)
+        return work.take(key, lead + (n,), torch.int32 if info["dtype"] == "i32" else self._real_dtype())
 
-    def _fold_scratch(self, name: str, bound: dict, device):
+    def _fold_scratch(self, name: str, bound: dict, work: _Workspace):
         """The claims and status of a fused fold: 64 status words, then one
         claim count per cell of its gradient plane."""
-        torch = _torch()
         cells = int(bound[self.planes[name]["cells_of"]].numel())
-        return self._buffer(("fold_scratch", name, cells), 4 * (64 + cells), device, zero=False).view(torch.int32)
+        return work.take(("fold_scratch", name, cells), 64 + cells, _torch().int32)
 
     def _fold_clear_args(self, t: dict, bound: dict) -> tuple:
         """``(args, status, cells)`` of the set-up of a fused fold: its claims and
@@ -599,14 +608,13 @@ class DeviceKernel:
         args = (0, 0, 0, 0, 1, 1, bound[t["out"]].data_ptr(), cells, scratch.data_ptr() + 256, scratch.data_ptr())
         return args, scratch, cells
 
-    def _fold_args(self, t: dict, bound: dict, n: int, device) -> tuple:
+    def _fold_args(self, t: dict, bound: dict, n: int, work: _Workspace) -> tuple:
         """``(args, status, cells)`` of the ordered fold ``t`` (the stage's log
         planes, the gradient plane, its claim counts and its status words)."""
         out = bound[t["out"]]
         cells = int(out.numel())
-        scratch = self._buffer(("fold", t["out"], cells), _core.keyed_log_fold_scratch_bytes(cells), device,
-                               zero=False)
-        status = self._buffer(("fold_status", t["out"]), 8, device, zero=False)
+        scratch = work.bytes(("fold", t["out"], cells), _core.keyed_log_fold_scratch_bytes(cells))
+        status = work.bytes(("fold_status", t["out"]), 8)
         args = (bound[t["v"]].data_ptr(), n, bound[t["c"]].data_ptr(), n // t["group"], t["group"], t["width"],
                 out.data_ptr(), cells, scratch.data_ptr(), status.data_ptr())
         return args, status, cells
@@ -673,26 +681,27 @@ class DeviceKernel:
         device = next((x.device for x in arrays.values() if isinstance(x, torch.Tensor)), None)
         if device is None:
             raise HawkError(f"kernel {self.name!r}: no plane is a tensor, so there is no device to run on")
-        bound, held = self._counter(dict(arrays), device)
+        work = self._workspace(stream, device)
+        bound, held = self._counter(dict(arrays), work)
         if held is not None:
             with _on(stream):
                 held.zero_()                      # a count per run
         if self.automatic:
-            bound[FUSED_STEPS_PLANE] = self._word(1 if steps is None else steps, device, stream)
+            bound[FUSED_STEPS_PLANE] = self._word(1 if steps is None else steps, work, stream)
         elif steps is not None:
             raise HawkError(f"kernel {self.name!r}: steps= sets the trip count of a hawk.steps(k, 'auto') kernel; "
                             "this one takes a fixed number of steps")
         if entry != "plain":
             if count >= FAST_MAX:
                 raise HawkError(f"kernel {self.name!r}: the fast entries take fewer than 2^30 samples a launch")
-            fn, block, _cells = self._fast(entry, bound, n, chunk, device, stream)
+            fn, block, _cells = self._fast(entry, bound, n, chunk, work, stream)
             self._launch_fast(entry, fn, block, base, count, n, stream)
             return
         for name, info in self.planes.items():
             if info.get("cells_of"):
-                bound[name] = self._fold_scratch(name, bound, device)
+                bound[name] = self._fold_scratch(name, bound, work)
             elif info.get("scratch"):
-                bound[name] = self._term_plane(name, n, device)
+                bound[name] = self._term_plane(name, n, work)
         statuses = []
         for t in self.team:
             if t.get("before"):                  # a fused fold's claims and status, cleared first
@@ -710,7 +719,7 @@ class DeviceKernel:
                 continue
             if t["op"] == "ordered_sum":
                 u = bound[t["u"]]
-                scratch = self._buffer(("sum", t["out"]), _core.ordered_sum_scratch_bytes(), device)
+                scratch = work.bytes(("sum", t["out"]), _core.ordered_sum_scratch_bytes(), zero=True)
                 fn = _core.ordered_sum_f32 if self._is_f32(t["out"]) else _core.ordered_sum
                 fn(u.data_ptr(), n, self._cell_ptr(t, bound[t["out"]]), scratch.data_ptr(), stream)
             elif t["op"] == "ordered_scatter":
@@ -718,9 +727,8 @@ class DeviceKernel:
                 cells = int(target.numel())
                 if cells == 0:
                     continue              # an ordered scatter into no cells adds nothing
-                scratch = self._buffer(("scatter", t["target"], n, cells),
-                                       _core.ordered_scatter_scratch_bytes(n, cells), device, zero=False)
-                status = self._buffer(("status", t["target"]), 4 * 257, device)
+                scratch = work.bytes(("scatter", t["target"], n, cells), _core.ordered_scatter_scratch_bytes(n, cells))
+                status = work.bytes(("status", t["target"]), 4 * 257, zero=True)
                 fn = _core.ordered_scatter_f32 if self._is_f32(t["target"]) else _core.ordered_scatter
                 fn(bound[t["key"]].data_ptr(), bound[t["v"]].data_ptr(), n, target.data_ptr(), cells,
                    scratch.data_ptr(), status.data_ptr(), stream)
@@ -736,21 +744,19 @@ class DeviceKernel:
                 if n == 0:
                     self._row_identities(ops, bound, stream)
                 else:
-                    jobs, rows, f32, scratch = self._row_finish_args(ops, bound, n, device, stream)
-                    _core.rows_finish_many(jobs, rows, f32, scratch.data_ptr(), stream)
+                    _core.rows_finish_many(*self._row_finish_args(ops, bound, n, work), stream)
             elif t["op"] == "band_ordered_sum":
                 u = bound[t["u"]]
-                scratch = self._buffer(("band_sum", t["out"]), _core.band_ordered_sum_scratch_bytes(), device,
-                                       zero=False)
+                scratch = work.bytes(("band_sum", t["out"]), _core.band_ordered_sum_scratch_bytes())
                 _core.band_ordered_sum(u.data_ptr(), n, self._cell_ptr(t, bound[t["out"]]), scratch.data_ptr(),
                                        stream)
             elif t["op"] == "keyed_sum":
-                scratch = self._buffer(("keyed", t["out"], n), _core.keyed_ordered_sum_scratch_bytes(n, t["group"]),
-                                       device)
+                scratch = work.bytes(("keyed", t["out"], n), _core.keyed_ordered_sum_scratch_bytes(n, t["group"]),
+                                     zero=True)
                 fn = _core.keyed_ordered_sum_f32 if self._is_f32(t["out"]) else _core.keyed_ordered_sum
                 fn(bound[t["u"]].data_ptr(), n, t["group"], bound[t["out"]].data_ptr(), scratch.data_ptr(), stream)
             elif t["op"] == "ordered_fold":
-                args, status, cells = self._fold_args(t, bound, n, device)
+                args, status, cells = self._fold_args(t, bound, n, work)
                 (_core.keyed_log_fold_f32 if self._is_f32(t["out"]) else _core.keyed_log_fold)(*args, stream)
                 statuses.append((t, status, cells))
             elif t["op"] == "keyed_comp":
@@ -1022,7 +1028,7 @@ class Prepared:
         elif hasattr(stream, "cuda_stream"):
             stream = stream.cuda_stream
         self.stream = int(stream)
-        with _on(self.stream):
+        with _on(self.stream), kernel._lock:
             self._setup(kernel, arrays, steps, entry, chunk)
 
     def _setup(self, kernel, arrays: dict, steps, entry: str, chunk: int) -> None:
@@ -1030,7 +1036,8 @@ class Prepared:
         device = next((x.device for x in arrays.values() if isinstance(x, torch.Tensor)), None)
         if device is None:
             raise HawkError(f"kernel {self.name!r}: no plane is a tensor, so there is no device to run on")
-        bound, held = kernel._counter(dict(arrays), device)
+        work = kernel._workspace(self.stream, device)
+        bound, held = kernel._counter(dict(arrays), work)
         self.held_counter = held
         if held is not None:
             held.zero_()
@@ -1049,14 +1056,14 @@ class Prepared:
                 raise HawkError(f"kernel {kernel.name!r}: the fast entries take fewer than 2^30 samples a launch")
             own = (torch.zeros(1, dtype=torch.int32, device=device), torch.zeros(1, dtype=torch.int32, device=device),
                    torch.zeros(1, dtype=torch.int64, device=device))
-            fn, block, cells = kernel._fast(entry, bound, self.n, chunk, device, self.stream, cells=own)
+            fn, block, cells = kernel._fast(entry, bound, self.n, chunk, work, self.stream, cells=own)
             self.fast = (entry, fn, block, cells)
             self.steps_max, self.steps_sum = cells[1], cells[2]
         for name, info in kernel.planes.items():
             if info.get("cells_of"):
-                bound[name] = kernel._fold_scratch(name, bound, device)
+                bound[name] = kernel._fold_scratch(name, bound, work)
             elif info.get("scratch"):
-                bound[name] = kernel._term_plane(name, self.n, device)
+                bound[name] = kernel._term_plane(name, self.n, work)
         self.bound = bound
         self.block = None
         if kernel.entry is not None:
@@ -1072,7 +1079,6 @@ class Prepared:
         self.steps = []
         self.before = []
         self.statuses = []
-        self.rows_scratch = []
         row_calls = kernel._row_calls(bound)
         for t in kernel.team:
             if t.get("before"):
@@ -1081,7 +1087,7 @@ class Prepared:
                 self.statuses.append((t, status, cells))
                 continue
             if t["op"] == "ordered_sum":
-                scratch = kernel._buffer(("sum", t["out"]), _core.ordered_sum_scratch_bytes(), device)
+                scratch = work.bytes(("sum", t["out"]), _core.ordered_sum_scratch_bytes(), zero=True)
                 args = (bound[t["u"]].data_ptr(), self.n, kernel._cell_ptr(t, bound[t["out"]]), scratch.data_ptr())
                 self.steps.append((_core.ordered_sum_f32 if kernel._is_f32(t["out"]) else _core.ordered_sum, args))
             elif t["op"] == "ordered_scatter":
@@ -1089,9 +1095,9 @@ class Prepared:
                 cells = int(target.numel())
                 if cells == 0:
                     continue
-                scratch = kernel._buffer(("scatter", t["target"], self.n, cells),
-                                         _core.ordered_scatter_scratch_bytes(self.n, cells), device, zero=False)
-                status = kernel._buffer(("status", t["target"]), 4 * 257, device)
+                scratch = work.bytes(("scatter", t["target"], self.n, cells),
+                                     _core.ordered_scatter_scratch_bytes(self.n, cells))
+                status = work.bytes(("status", t["target"]), 4 * 257, zero=True)
                 args = (bound[t["key"]].data_ptr(), bound[t["v"]].data_ptr(), self.n, target.data_ptr(), cells,
                         scratch.data_ptr(), status.data_ptr())
                 self.steps.append((_core.ordered_scatter_f32 if kernel._is_f32(t["target"]) else _core.ordered_scatter,
@@ -1108,22 +1114,19 @@ class Prepared:
                 if self.n == 0:
                     self.steps.append((kernel._row_identities, (ops, bound)))
                 else:
-                    jobs, rows, f32, scratch = kernel._row_finish_args(ops, bound, self.n, device, self.stream)
-                    self.rows_scratch.append(scratch)    # alive as long as the launcher
-                    self.steps.append((_core.rows_finish_many, (jobs, rows, f32, scratch.data_ptr())))
+                    self.steps.append((_core.rows_finish_many, kernel._row_finish_args(ops, bound, self.n, work)))
             elif t["op"] == "band_ordered_sum":
-                scratch = kernel._buffer(("band_sum", t["out"]), _core.band_ordered_sum_scratch_bytes(), device,
-                                         zero=False)
+                scratch = work.bytes(("band_sum", t["out"]), _core.band_ordered_sum_scratch_bytes())
                 args = (bound[t["u"]].data_ptr(), self.n, kernel._cell_ptr(t, bound[t["out"]]), scratch.data_ptr())
                 self.steps.append((_core.band_ordered_sum, args))
             elif t["op"] == "keyed_sum":
-                scratch = kernel._buffer(("keyed", t["out"], self.n),
-                                         _core.keyed_ordered_sum_scratch_bytes(self.n, t["group"]), device)
+                scratch = work.bytes(("keyed", t["out"], self.n),
+                                     _core.keyed_ordered_sum_scratch_bytes(self.n, t["group"]), zero=True)
                 args = (bound[t["u"]].data_ptr(), self.n, t["group"], bound[t["out"]].data_ptr(), scratch.data_ptr())
                 self.steps.append((_core.keyed_ordered_sum_f32 if kernel._is_f32(t["out"]) else _core.keyed_ordered_sum,
                                    args))
             elif t["op"] == "ordered_fold":
-                args, status, cells = kernel._fold_args(t, bound, self.n, device)
+                args, status, cells = kernel._fold_args(t, bound, self.n, work)
                 self.steps.append((_core.keyed_log_fold_f32 if kernel._is_f32(t["out"]) else _core.keyed_log_fold,
                                    args))
                 self.statuses.append((t, status, cells))
@@ -1150,7 +1153,7 @@ class Prepared:
         # The launches hold what they use (the kernel, its blocks, the bound
         # planes), not this object: a launcher let go frees its planes at once.
         k, n, stream = self.kernel, self.n, self.stream
-        keep = (k, self.bound, self.rows_scratch)
+        keep = (k, self.bound)
 
         def call(fn, args):
             return lambda fn=fn, args=(*args, stream), keep=keep: fn(*args)

@@ -90,3 +90,76 @@ def test_reductions_that_share_a_cell_keep_the_kernels_order(tmp_path, recorded)
             assert [name for name, _ in recorded] == ["three", "rows_finish_many", "ordered_sum", "rows_finish_many"]
             assert [[job.out for job in recorded[i][1][0]] for i in (1, 3)] == [[a.data_ptr()], [b.data_ptr()]]
             recorded.clear()
+
+
+def _work_pointers(calls, planes) -> set:
+    """The addresses a run's calls work in: every pointer but the caller's planes'."""
+    mine = {x.data_ptr() for x in planes.values()}
+    found = set()
+    for _name, args in calls:
+        for a in args:
+            for v in ([p for job in a for p in (job.hi, job.lo, job.out)] if hasattr(a, "_length_") else [a]):
+                if isinstance(v, int) and v > 1 << 20 and v not in mine:
+                    found.add(v)
+    return found
+
+
+def _kernels_with_scratch(n):
+    import torch
+    from hawk_amd import Grid, Index, Kernel, Table
+    from hawk_amd import examples as E
+
+    @hawk.kernel
+    def keyed(lane: Grid["key", "sample":200], x: Scalar, o: Mutable["key"], c: Mutable["key"]):
+        o = hawk.sum(x * 2.0, over="sample", policy="ordered")
+        c = hawk.sum(x, over="sample")
+
+    @hawk.kernel
+    def table(lane: Grid["key", "sample":100], t: Table["key", "w":2], x: Scalar) -> Scalar:
+        return hawk.sum(t.at(key=lane.key, w=0) * x + t.at(key=lane.key, w=1), over="sample", policy="ordered")
+    back = Kernel("table_vjp", hawk.diff.vjp(table, wrt=("t",)))
+
+    def d(*shape):
+        return torch.ones(*shape, dtype=torch.float64)
+    return [(three, dict(x=d(n), a=d(1), o=d(1), b=d(1))),
+            (E.chain, dict(x=d(n), key=torch.zeros(n, dtype=torch.int32), y=d(n), total=d(1), bins=d(64))),
+            (keyed, dict(x=d(n), o=d(n // 200), c=d(n // 200))),
+            (back, dict(t=d(n // 50), x=d(n), bar_out=d(n // 100), bar_t=d(n // 50)))]
+
+
+def test_each_stream_has_its_own_workspace(tmp_path, recorded):
+    """Calls on two streams may run at once, so nothing one works in is the
+    other's: not the scratch of a team stage, not a plane the stage writes for
+    it, not a launcher's.  Calls on one stream share."""
+    cases = _kernels_with_scratch(2000)
+    for k, (_, planes) in zip(_load(tmp_path, *(c[0] for c in cases)), cases):
+        used = {}
+        for turn, stream in enumerate((0, 7, 0, 7)):
+            for way, _ in enumerate(_both_ways(k, 2000, stream, **planes)):
+                here = _work_pointers(recorded, planes)
+                assert here, k.name
+                if turn > 1 or way:
+                    assert here == used[stream], (k.name, stream)
+                used[stream] = here
+                recorded.clear()
+        assert not used[0] & used[7], k.name
+
+
+def test_each_stream_has_its_own_trip_count_and_finish_counter(tmp_path, recorded):
+    """The words the runtime itself binds: another stream's are rewritten
+    while this one's launch reads them."""
+    import torch
+    from hawk_amd import examples as E
+    (k,) = _load(tmp_path, E.osc_finish_xauto)
+    planes = {name: torch.zeros(50, dtype=torch.bool if name == "terminated" else torch.float64)
+              for name in ("t_final", "terminated", "x", "v", "t")}
+    mine = {x.data_ptr() for x in planes.values()}
+    used = {}
+    for stream in (0, 7, 0):
+        for steps in (3, 4):
+            k._run(dict(planes, dt=0.5), 0, 50, 50, stream, False, steps=steps)
+            here = {held[1] for held in k._held_slots if held[0] == "p"} - mine
+            assert len(here) == 2 and used.setdefault(stream, here) == here
+            word = k._workspace(stream, planes["x"].device)[("word", "")]
+            assert int(word) == steps and word.data_ptr() in here
+    assert not used[0] & used[7]

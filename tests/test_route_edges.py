@@ -414,3 +414,45 @@ def test_reductions_into_one_cell_leave_the_last(tmp_path, gpu, n):
         for call in (lambda **p: hawk.run(k, **p), lambda **p: k.prepare(**p)()):
             call(x=x, a=cells[0], o=cells[1], b=cells[2])
             assert float(one) == float(want), (n, call)
+
+
+def test_two_streams_of_one_kernel(tmp_path, gpu):
+    """One kernel's runs and launchers on two streams at once: each ends with
+    the cells of its own inputs."""
+    import hawk_amd as hawk
+    import torch
+    from hawk_amd import Index, Mutable, Scalar
+
+    @hawk.kernel
+    def all_of(x: Scalar, key: Index, a: Mutable[Scalar], b: Mutable[Scalar], o: Mutable[Scalar],
+               bins: Mutable[Scalar]):
+        a = hawk.sum(x * x)
+        b = hawk.max(x)
+        o = hawk.sum(x * 2.0, policy="ordered")
+        hawk.scatter(bins, policy="ordered")[key] += x * 3.0
+    (k,) = _unit(tmp_path, [all_of])
+    n, cells = 300_007, 30_000
+    streams, sides = [torch.cuda.Stream() for _ in range(2)], []
+    for i in range(2):
+        g = torch.Generator(device=gpu).manual_seed(i)
+        sides.append(dict(x=torch.randn(n, dtype=torch.float64, device=gpu, generator=g) + 10.0 * i,
+                          key=torch.randint(0, cells, (n,), dtype=torch.int32, device=gpu, generator=g),
+                          bins=torch.zeros(cells, dtype=torch.float64, device=gpu),
+                          **{c: torch.zeros(1, dtype=torch.float64, device=gpu) for c in "abo"}))
+    want = []
+    for p in sides:                                   # one stream alone
+        hawk.run(k, **p)
+        want.append({name: x.clone() for name, x in p.items()})
+    torch.cuda.synchronize()
+    launchers = [k.prepare(stream=s, **p) for s, p in zip(streams, sides)]
+    for way in ("run", "launcher"):
+        for turn in range(20):
+            for s, p, launch in zip(streams, sides, launchers):
+                with torch.cuda.stream(s):
+                    for name in ("bins", "a", "b", "o"):
+                        p[name].zero_()
+                    hawk.run(k, check=False, **p) if way == "run" else launch()
+        torch.cuda.synchronize()
+        for p, w in zip(sides, want):
+            for name in p:
+                assert torch.equal(p[name], w[name]), (way, name)
