@@ -816,7 +816,9 @@ class ChainedKernel:
     """A ``hawk.chain`` the build cut into segments: each segment is a kernel
     of its own, run in order; a value one segment passes to a later one
     crosses in a plane the runtime holds (``hwc_<name>``), made once per
-    sample count (reference ``hawk/ir/chain.py:133-179``)."""
+    stream and sample count (reference ``hawk/ir/chain.py:133-179``).  ``run``
+    holds the chain's lock over all its segments, so one thread's segments
+    read the values of its own call."""
 
     def __init__(self, directory: Path, sidecar: dict):
         self.directory = Path(directory)
@@ -826,14 +828,15 @@ class ChainedKernel:
         self.team = []
         self.segments = [load(directory, s) for s in sidecar["segments"]]
         self.crossing = sidecar["crossing"]
-        self._held: dict = {}
+        self._workspaces: dict = {}
         self._lock = threading.Lock()
 
     def caller_planes(self) -> list:
         return list(self.planes)
 
-    def _bindings(self, arrays: dict, n_samples=None) -> list:
-        """Each segment's planes: the caller's and the crossing planes it reads or writes."""
+    def _bindings(self, arrays: dict, stream: int, n_samples=None) -> list:
+        """Each segment's planes: the caller's and the crossing planes (the
+        stream's) it reads or writes."""
         torch = _torch()
         declared = set(self.planes)
         unknown = sorted(set(arrays) - declared)
@@ -851,22 +854,18 @@ class ChainedKernel:
         device = next((x.device for x in arrays.values() if isinstance(x, torch.Tensor)), None)
         if device is None:
             raise HawkError(f"kernel {self.name!r}: no plane is a tensor, so there is no device to run on")
+        work = self._workspaces.setdefault((stream, device), _Workspace(device))
         cross = {}
         for name, info in self.crossing.items():
-            key = (name, n, device)
-            held = self._held.get(key)
-            if held is None:
-                dt = torch.int32 if info["dtype"] == "i32" else torch.float64
-                held = torch.empty(tuple(info["shape"]) + (n,), dtype=dt, device=device)
-                self._held[key] = held
-            cross[name] = held
+            cross[name] = work.take(("cross", name, n), tuple(info["shape"]) + (n,),
+                                    torch.int32 if info["dtype"] == "i32" else torch.float64)
         out = []
         for seg in self.segments:
             names = seg.caller_planes()
             out.append((seg, {p: (cross[p] if p in cross else arrays[p]) for p in names}))
         return out
 
-    def resolve_call(self, arrays: dict, layout=None, n_samples=None) -> tuple:
+    def resolve_call(self, arrays: dict, stream: int, layout=None, n_samples=None) -> tuple:
         """``(bindings, write_back)`` of one call: the caller's planes made
         component-major once (:func:`hawk_amd.layout.resolve`), then each
         segment's planes (:meth:`_bindings`); ``write_back`` lists the
@@ -874,7 +873,7 @@ class ChainedKernel:
         copies, to copy back after the last segment."""
         from . import layout as _layout
         arrays, write_back = _layout.resolve(self, dict(arrays), layout, _PER_SAMPLE, _WRITTEN)
-        return self._bindings(arrays, n_samples), write_back
+        return self._bindings(arrays, stream, n_samples), write_back
 
     def prepare(self, *, stream=None, **arrays):
         return _PreparedChain(self, arrays, stream)
@@ -885,7 +884,11 @@ class _PreparedChain:
 
     def __init__(self, chain: ChainedKernel, arrays: dict, stream=None):
         self.kernel = chain
-        self.parts = [seg.prepare(stream=stream, **planes) for seg, planes in chain._bindings(dict(arrays))]
+        stream = _torch().cuda.current_stream() if stream is None else stream
+        stream = int(getattr(stream, "cuda_stream", stream))
+        with _on(stream), chain._lock:
+            bindings = chain._bindings(dict(arrays), stream)
+        self.parts = [seg.prepare(stream=stream, **planes) for seg, planes in bindings]
 
     def __call__(self) -> None:
         for part in self.parts:
@@ -953,14 +956,15 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
         # on component-major planes, and a sample-major plane the chain
         # writes is copied back after the last segment.
         sid = torch.cuda.current_stream().cuda_stream if stream is None else getattr(stream, "cuda_stream", stream)
-        with _on(int(sid)):
-            bindings, write_back = kernel.resolve_call(arrays, layout, n_samples)
-        for seg, planes in bindings:
-            run(seg, n_samples=n_samples, stream=stream, check=check, **planes)
-        if write_back:
+        with kernel._lock:
             with _on(int(sid)):
-                for dst, copy in write_back:
-                    dst.copy_(copy.movedim(-1, 0))
+                bindings, write_back = kernel.resolve_call(arrays, int(sid), layout, n_samples)
+            for seg, planes in bindings:
+                run(seg, n_samples=n_samples, stream=int(sid), check=check, **planes)
+            if write_back:
+                with _on(int(sid)):
+                    for dst, copy in write_back:
+                        dst.copy_(copy.movedim(-1, 0))
         return
     if not isinstance(kernel, DeviceKernel):
         raise HawkError("hawk.run takes a kernel loaded with hawk.load")

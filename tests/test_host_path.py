@@ -49,7 +49,9 @@ def recorded(monkeypatch):
     monkeypatch.setattr(runtime, "_on", lambda stream: runtime._nullcontext())
     monkeypatch.setattr(runtime, "_current_stream", lambda: 0)
     monkeypatch.setattr(runtime.DeviceKernel, "check_planes",
-                        lambda self, arrays, n_samples=None, rows=(): arrays["x"].shape[-1])
+                        lambda self, arrays, n_samples=None, rows=(): next(
+                            x.shape[-1] for name, x in arrays.items() if self.planes[name]["role"] in
+                            runtime._PER_SAMPLE))
     return calls
 
 
@@ -163,3 +165,30 @@ def test_each_stream_has_its_own_trip_count_and_finish_counter(tmp_path, recorde
             word = k._workspace(stream, planes["x"].device)[("word", "")]
             assert int(word) == steps and word.data_ptr() in here
     assert not used[0] & used[7]
+
+
+def test_a_cut_chain_crosses_in_planes_of_its_stream_one_call_at_a_time(tmp_path, recorded):
+    """A cut chain's crossing planes are a stream's own, and a call's segments
+    run with no other call's between them."""
+    import threading
+
+    import torch
+    from hawk_amd import examples as E
+    chained = hawk.chain(*E.CHAIN_MEMBERS, name="cut")
+    hawk.build([chained], tmp_path, register_line=32)
+    k = hawk.load(tmp_path, "cut")
+    planes = {name: torch.zeros(tuple(info["shape"]) + (40,), dtype=torch.float64)
+              for name, info in k.planes.items()}
+    mine = {x.data_ptr() for x in planes.values()}
+    used = {}
+    for stream in (0, 7, 0):
+        here = {x.data_ptr() for _, p in k._bindings(planes, stream) for x in p.values()} - mine
+        assert here and used.setdefault(stream, here) == here
+    assert not used[0] & used[7]
+    with k._lock:
+        other = threading.Thread(target=lambda: hawk.run(k, stream=7, **planes))
+        other.start()
+        other.join(0.2)
+        assert other.is_alive() and not recorded
+    other.join(10)
+    assert len(recorded) == len(k.segments) > 1
