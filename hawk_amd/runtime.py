@@ -95,10 +95,13 @@ def _current_stream() -> int:
 
 def _on(stream: int):
     """A context in which torch's own work (a counter's ``zero_()``, a cell's
-    ``fill_()``) is issued on ``stream``, the stream the next launch uses, so
-    the reset is ordered before that launch and after the previous one."""
-    torch = _torch()
-    return torch.cuda.stream(torch.cuda.ExternalStream(stream)) if stream else _nullcontext()
+    ``fill_()``, an allocation) is issued on ``stream``, the stream the next
+    launch uses, so the reset is ordered before that launch and after the
+    previous one.  0 is the default stream, whatever the current one is."""
+    if stream == _current_stream():
+        return _nullcontext()
+    cuda = _torch().cuda
+    return cuda.stream(cuda.ExternalStream(stream) if stream else cuda.default_stream())
 
 
 class _Workspace(dict):

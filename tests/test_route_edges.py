@@ -456,3 +456,17 @@ def test_two_streams_of_one_kernel(tmp_path, gpu):
         for p, w in zip(sides, want):
             for name in p:
                 assert torch.equal(p[name], w[name]), (way, name)
+
+
+def test_work_beside_a_launch_is_on_its_stream(gpu):
+    """Resets, fills and allocations go to the launch's stream, the default
+    stream inside another one's context included."""
+    import torch
+    from hawk_amd import runtime
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    for current in (torch.cuda.default_stream(), side):
+        for stream in (0, side.cuda_stream, other.cuda_stream):
+            with torch.cuda.stream(current):
+                with runtime._on(stream):
+                    assert torch.cuda.current_stream().cuda_stream == stream
+                assert torch.cuda.current_stream() == current
