@@ -868,7 +868,7 @@ class ChainedKernel:
             out.append((seg, {p: (cross[p] if p in cross else arrays[p]) for p in names}))
         return out
 
-    def resolve_call(self, arrays: dict, stream: int, layout=None, n_samples=None) -> tuple:
+    def resolve_call(self, arrays: dict, layout=None, n_samples=None, stream: int = 0) -> tuple:
         """``(bindings, write_back)`` of one call: the caller's planes made
         component-major once (:func:`hawk_amd.layout.resolve`), then each
         segment's planes (:meth:`_bindings`); ``write_back`` lists the
@@ -961,7 +961,7 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
         sid = torch.cuda.current_stream().cuda_stream if stream is None else getattr(stream, "cuda_stream", stream)
         with kernel._lock:
             with _on(int(sid)):
-                bindings, write_back = kernel.resolve_call(arrays, int(sid), layout, n_samples)
+                bindings, write_back = kernel.resolve_call(arrays, layout, n_samples, int(sid))
             for seg, planes in bindings:
                 run(seg, n_samples=n_samples, stream=int(sid), check=check, **planes)
             if write_back:
