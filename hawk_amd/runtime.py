@@ -837,7 +837,7 @@ class ChainedKernel:
     def caller_planes(self) -> list:
         return list(self.planes)
 
-    def _bindings(self, arrays: dict, stream: int, n_samples=None) -> list:
+    def _bindings(self, arrays: dict, n_samples=None, stream: int = 0) -> list:
         """Each segment's planes: the caller's and the crossing planes (the
         stream's) it reads or writes."""
         torch = _torch()
@@ -876,7 +876,7 @@ class ChainedKernel:
         copies, to copy back after the last segment."""
         from . import layout as _layout
         arrays, write_back = _layout.resolve(self, dict(arrays), layout, _PER_SAMPLE, _WRITTEN)
-        return self._bindings(arrays, stream, n_samples), write_back
+        return self._bindings(arrays, n_samples, stream), write_back
 
     def prepare(self, *, stream=None, **arrays):
         return _PreparedChain(self, arrays, stream)
@@ -890,7 +890,7 @@ class _PreparedChain:
         stream = _torch().cuda.current_stream() if stream is None else stream
         stream = int(getattr(stream, "cuda_stream", stream))
         with _on(stream), chain._lock:
-            bindings = chain._bindings(dict(arrays), stream)
+            bindings = chain._bindings(dict(arrays), stream=stream)
         self.parts = [seg.prepare(stream=stream, **planes) for seg, planes in bindings]
 
     def __call__(self) -> None:

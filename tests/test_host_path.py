@@ -182,7 +182,7 @@ def test_a_cut_chain_crosses_in_planes_of_its_stream_one_call_at_a_time(tmp_path
     mine = {x.data_ptr() for x in planes.values()}
     used = {}
     for stream in (0, 7, 0):
-        here = {x.data_ptr() for _, p in k._bindings(planes, stream) for x in p.values()} - mine
+        here = {x.data_ptr() for _, p in k._bindings(planes, stream=stream) for x in p.values()} - mine
         assert here and used.setdefault(stream, here) == here
     assert not used[0] & used[7]
     with k._lock:
