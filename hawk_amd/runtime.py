@@ -10,8 +10,8 @@ fixed-tree ordered sum, the ordered scatter) on the same HIP stream.
 Ownership as in the reference (``hawk/runtime.py:20-22``, ``:655-696``): the
 planes are the caller's and are written in place; the runtime owns only its
 scratch (term planes of a split kernel, the sum's lane partials, the
-scatter's chunk partials and status plane), made once per stream and sample
-count.
+scatter's chunk partials and status plane): for ``run`` one set a stream, as
+large as its largest call; for launchers one a stream and sample count.
 
 Threading: one :class:`DeviceKernel` shared by threads is safe: ``run`` holds
 the kernel's lock over bind and launch (reference ``hawk/runtime.py:46-53``).
@@ -93,6 +93,12 @@ def _current_stream() -> int:
     return raw(torch.cuda.current_device())
 
 
+def _stream_of(stream) -> int:
+    """The handle of a call's ``stream=``: a torch stream, a handle, or (None)
+    the current stream."""
+    return _current_stream() if stream is None else int(getattr(stream, "cuda_stream", stream))
+
+
 def _on(stream: int):
     """A context in which torch's own work (a counter's ``zero_()``, a cell's
     ``fill_()``, an allocation) is issued on ``stream``, the stream the next
@@ -108,22 +114,54 @@ class _Workspace(dict):
     """What a kernel's launches on one stream of one GPU work in: its scratch
     tensors by ``(what, name, *sizes)``, each made when first asked for.  A
     stream's launches run one after another, so they share these; the launches
-    of another stream, which may run at the same time, have their own."""
+    of another stream, which may run at the same time, have their own.
 
-    def __init__(self, device):
+    ``grows``: ``hawk.run``'s.  Each ``(what, name)`` is one buffer, as large
+    as the largest call so far asked for, so a program of many batch sizes
+    holds no more for the sizes behind it than a multiple of the largest.  A
+    buffer grows by half at least and stays alive once outgrown (a captured
+    graph may hold its address): those add up to at most twice the last.
+    Otherwise a launcher's: a tensor per key, since each launcher keeps the
+    addresses of its own size."""
+
+    #: The most tensors a growing workspace lists (each is a view of a buffer).
+    VIEWS = 1024
+
+    def __init__(self, device, grows: bool = True):
         super().__init__()
         self.device = device
         self.word = None          # the value the trip-count word holds
+        self._buffers = {} if grows else None
+        self._outgrown: list = []
 
     def take(self, key: tuple, shape, dtype, zero: bool = False):
         held = self.get(key)
-        if held is None:
-            torch = _torch()
-            held = self[key] = (torch.zeros if zero else torch.empty)(shape, dtype=dtype, device=self.device)
+        if held is not None:
+            return held
+        torch = _torch()
+        make = torch.zeros if zero else torch.empty
+        if self._buffers is None:
+            held = make(shape, dtype=dtype, device=self.device)
+        else:
+            count = 1
+            for extent in shape:
+                count *= extent
+            nbytes = count * dtype.itemsize
+            buffer = self._buffers.get(key[:2])
+            if buffer is None or buffer.numel() < nbytes:
+                if buffer is not None:
+                    self._outgrown.append(buffer)
+                grown = 0 if buffer is None else buffer.numel() * 3 // 2
+                buffer = make(max(nbytes, grown, 8), dtype=torch.uint8, device=self.device)
+                self._buffers[key[:2]] = buffer
+            if len(self) >= self.VIEWS:
+                self.clear()
+            held = buffer[:nbytes].view(dtype).view(shape)
+        self[key] = held
         return held
 
     def bytes(self, key: tuple, nbytes: int, zero: bool = False):
-        return self.take(key, max(1, nbytes), _torch().uint8, zero)
+        return self.take(key, (max(1, nbytes),), _torch().uint8, zero)
 
 
 class DeviceKernel:
@@ -280,16 +318,17 @@ class DeviceKernel:
         """Whether the kernel reads its trip count at launch (``hawk.steps(k, "auto")``)."""
         return (self.sidecar.get("finish") or {}).get("steps") == "auto"
 
-    def _workspace(self, stream: int, device) -> _Workspace:
-        """The workspace of the launches on ``stream`` of ``device``."""
-        held = self._workspaces.get((stream, device))
+    def _workspace(self, stream: int, device, launcher: bool = False) -> _Workspace:
+        """The workspace of ``hawk.run``'s launches on ``stream`` of ``device``,
+        or of the launchers bound to that stream."""
+        held = self._workspaces.get((stream, device, launcher))
         if held is None:
-            held = self._workspaces.setdefault((stream, device), _Workspace(device))
+            held = self._workspaces.setdefault((stream, device, launcher), _Workspace(device, grows=not launcher))
         return held
 
     @property
     def _scratch(self) -> _Workspace:
-        """The workspace of the current stream."""
+        """``hawk.run``'s workspace on the current stream."""
         torch = _torch()
         return self._workspace(_current_stream(), torch.device("cuda", torch.cuda.current_device()))
 
@@ -299,7 +338,7 @@ class DeviceKernel:
         torch = _torch()
         if isinstance(steps, bool) or not isinstance(steps, int):
             raise HawkError(f"kernel {self.name!r}: steps= is an int (the trips this launch runs), got {steps!r}")
-        held = work.take(("word", ""), 1, torch.int32, zero=True)
+        held = work.take(("word", ""), (1,), torch.int32, zero=True)
         value = max(-(1 << 31), min(steps, (1 << 31) - 1))
         if work.word != value:
             with _on(stream):
@@ -325,7 +364,7 @@ class DeviceKernel:
         block = _core.ArgBlock(list(self.sidecar["descriptor"]) + list(FAST_SLOTS[entry]))
         self._bind(block, bound, n)
         if cells is None:
-            cells = tuple(work.take((what, ""), 1, dtype, zero=True) for what, dtype in
+            cells = tuple(work.take((what, ""), (1,), dtype, zero=True) for what, dtype in
                           (("claims", torch.int32), ("steps_max", torch.int32), ("steps_sum", torch.int64)))
             self.steps_max, self.steps_sum = cells[1], cells[2]
         with _on(stream):
@@ -364,7 +403,7 @@ class DeviceKernel:
         per run)."""
         if FINISHED_PLANE not in self.planes or FINISHED_PLANE in arrays:
             return arrays, None
-        held = work.take(("finished", ""), 1, _torch().int32, zero=True)
+        held = work.take(("finished", ""), (1,), _torch().int32, zero=True)
         self.finished = held
         return {**arrays, FINISHED_PLANE: held}, held
 
@@ -601,7 +640,7 @@ class DeviceKernel:
         """The claims and status of a fused fold: 64 status words, then one
         claim count per cell of its gradient plane."""
         cells = int(bound[self.planes[name]["cells_of"]].numel())
-        return work.take(("fold_scratch", name, cells), 64 + cells, _torch().int32)
+        return work.take(("fold_scratch", name, cells), (64 + cells,), _torch().int32)
 
     def _fold_clear_args(self, t: dict, bound: dict) -> tuple:
         """``(args, status, cells)`` of the set-up of a fused fold: its claims and
@@ -818,8 +857,8 @@ def _status_problem(name: str, t: dict, status, cells: int) -> str | None:
 class ChainedKernel:
     """A ``hawk.chain`` the build cut into segments: each segment is a kernel
     of its own, run in order; a value one segment passes to a later one
-    crosses in a plane the runtime holds (``hwc_<name>``), made once per
-    stream and sample count (reference ``hawk/ir/chain.py:133-179``).  ``run``
+    crosses in a plane the runtime holds (``hwc_<name>``), its stream's
+    (:class:`_Workspace`; reference ``hawk/ir/chain.py:133-179``).  ``run``
     holds the chain's lock over all its segments, so one thread's segments
     read the values of its own call."""
 
@@ -837,7 +876,7 @@ class ChainedKernel:
     def caller_planes(self) -> list:
         return list(self.planes)
 
-    def _bindings(self, arrays: dict, n_samples=None, stream: int = 0) -> list:
+    def _bindings(self, arrays: dict, n_samples=None, stream: int = 0, launcher: bool = False) -> list:
         """Each segment's planes: the caller's and the crossing planes (the
         stream's) it reads or writes."""
         torch = _torch()
@@ -857,7 +896,7 @@ class ChainedKernel:
         device = next((x.device for x in arrays.values() if isinstance(x, torch.Tensor)), None)
         if device is None:
             raise HawkError(f"kernel {self.name!r}: no plane is a tensor, so there is no device to run on")
-        work = self._workspaces.setdefault((stream, device), _Workspace(device))
+        work = self._workspaces.setdefault((stream, device, launcher), _Workspace(device, grows=not launcher))
         cross = {}
         for name, info in self.crossing.items():
             cross[name] = work.take(("cross", name, n), tuple(info["shape"]) + (n,),
@@ -887,10 +926,9 @@ class _PreparedChain:
 
     def __init__(self, chain: ChainedKernel, arrays: dict, stream=None):
         self.kernel = chain
-        stream = _torch().cuda.current_stream() if stream is None else stream
-        stream = int(getattr(stream, "cuda_stream", stream))
+        stream = _stream_of(stream)
         with _on(stream), chain._lock:
-            bindings = chain._bindings(dict(arrays), stream=stream)
+            bindings = chain._bindings(dict(arrays), stream=stream, launcher=True)
         self.parts = [seg.prepare(stream=stream, **planes) for seg, planes in bindings]
 
     def __call__(self) -> None:
@@ -946,8 +984,7 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
     :func:`hawk_amd.samples_first` / :func:`~hawk_amd.samples_last` say which
     axis of a per-sample plane holds the samples (:mod:`hawk_amd.layout`)."""
     if steps is None and entry == "plain" and type(kernel) is DeviceKernel and kernel._direct is not None:
-        if kernel.run_direct(arrays, base, count, n_samples, layout,
-                             _current_stream() if stream is None else int(getattr(stream, "cuda_stream", stream))):
+        if kernel.run_direct(arrays, base, count, n_samples, layout, _stream_of(stream)):
             return
     from . import layout as _layout
     torch = _torch()
@@ -958,27 +995,24 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
         # chain: the crossing planes are (w, N), so every segment then runs
         # on component-major planes, and a sample-major plane the chain
         # writes is copied back after the last segment.
-        sid = torch.cuda.current_stream().cuda_stream if stream is None else getattr(stream, "cuda_stream", stream)
+        sid = _stream_of(stream)
         with kernel._lock:
-            with _on(int(sid)):
-                bindings, write_back = kernel.resolve_call(arrays, layout, n_samples, int(sid))
+            with _on(sid):
+                bindings, write_back = kernel.resolve_call(arrays, layout, n_samples, sid)
             for seg, planes in bindings:
-                run(seg, n_samples=n_samples, stream=int(sid), check=check, **planes)
+                run(seg, n_samples=n_samples, stream=sid, check=check, **planes)
             if write_back:
-                with _on(int(sid)):
+                with _on(sid):
                     for dst, copy in write_back:
                         dst.copy_(copy.movedim(-1, 0))
         return
     if not isinstance(kernel, DeviceKernel):
         raise HawkError("hawk.run takes a kernel loaded with hawk.load")
-    if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
-    elif hasattr(stream, "cuda_stream"):
-        stream = stream.cuda_stream
+    stream = _stream_of(stream)
     arrays, major = _layout.classify(kernel, arrays, layout, _PER_SAMPLE)
     rows, write_back = bool(major) and kernel.takes_rows(arrays, major, entry), []
     if major and not rows:
-        with _on(int(stream)):
+        with _on(stream):
             arrays, write_back = _layout.component_major(kernel, arrays, major, _WRITTEN)
     n = kernel.check_planes(arrays, n_samples, major if rows else ())
     if kernel.team and (base != 0 or count not in (None, n)):
@@ -989,10 +1023,10 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
     if base < 0 or count < 0 or base + count > n:
         raise HawkError(f"{kernel.name}: [base, base+count) = [{base}, {base + count}) is outside [0, {n})")
     with kernel._lock:
-        kernel._run(arrays, int(base), int(count), int(n), int(stream), check, steps=steps, entry=entry,
+        kernel._run(arrays, int(base), int(count), int(n), stream, check, steps=steps, entry=entry,
                     chunk=chunk, rows=rows)
     if write_back:
-        with _on(int(stream)):
+        with _on(stream):
             for dst, copy in write_back:       # a sample-major plane the kernel wrote
                 dst.copy_(copy.movedim(-1, 0))
 
@@ -1030,11 +1064,7 @@ class Prepared:
                             f"planes only; {marked} are marked (hawk.run takes a sample-major plane through a copy)")
         self.n = kernel.check_planes(arrays)
         self.arrays = dict(arrays)
-        if stream is None:
-            stream = torch.cuda.current_stream().cuda_stream
-        elif hasattr(stream, "cuda_stream"):
-            stream = stream.cuda_stream
-        self.stream = int(stream)
+        self.stream = _stream_of(stream)
         with _on(self.stream), kernel._lock:
             self._setup(kernel, arrays, steps, entry, chunk)
 
@@ -1043,8 +1073,8 @@ class Prepared:
         device = next((x.device for x in arrays.values() if isinstance(x, torch.Tensor)), None)
         if device is None:
             raise HawkError(f"kernel {self.name!r}: no plane is a tensor, so there is no device to run on")
-        work = kernel._workspace(self.stream, device)
-        bound, held = kernel._counter(dict(arrays), work)
+        work = kernel._workspace(self.stream, device, launcher=True)
+        bound, held = kernel._counter(dict(arrays), kernel._workspace(self.stream, device))
         self.held_counter = held
         if held is not None:
             held.zero_()

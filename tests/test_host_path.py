@@ -132,19 +132,44 @@ def _kernels_with_scratch(n):
 def test_each_stream_has_its_own_workspace(tmp_path, recorded):
     """Calls on two streams may run at once, so nothing one works in is the
     other's: not the scratch of a team stage, not a plane the stage writes for
-    it, not a launcher's.  Calls on one stream share."""
+    it, not a launcher's.  Runs on one stream share, and so do its launchers."""
     cases = _kernels_with_scratch(2000)
     for k, (_, planes) in zip(_load(tmp_path, *(c[0] for c in cases)), cases):
         used = {}
-        for turn, stream in enumerate((0, 7, 0, 7)):
+        for stream in (0, 7, 0, 7):
             for way, _ in enumerate(_both_ways(k, 2000, stream, **planes)):
                 here = _work_pointers(recorded, planes)
-                assert here, k.name
-                if turn > 1 or way:
-                    assert here == used[stream], (k.name, stream)
-                used[stream] = here
+                assert here and used.setdefault((stream, way), here) == here, (k.name, stream)
                 recorded.clear()
-        assert not used[0] & used[7], k.name
+        assert not (used[0, 0] | used[0, 1]) & (used[7, 0] | used[7, 1]), k.name
+
+
+def test_runs_of_many_sizes_hold_a_multiple_of_the_largest(tmp_path, recorded):
+    """hawk.run over ever new sample counts holds, for every scratch tensor, at
+    most half more than the largest needs and twice that outgrown; a size seen
+    before works where it did, and a launcher's addresses are its own."""
+    sizes = [2000 + 200 * i for i in range(40)]
+    kernels = [case[0] for case in _kernels_with_scratch(2000)]
+    calls = {n: [case[1] for case in _kernels_with_scratch(n)] for n in sizes}
+    for i, k in enumerate(_load(tmp_path, *kernels)):
+        launch = k.prepare(stream=0, **calls[sizes[0]][i])
+        recorded.clear()
+        launch()
+        mine = _work_pointers(recorded, calls[sizes[0]][i])
+        seen = {}
+        for n in sizes * 2:
+            recorded.clear()
+            k._run(dict(calls[n][i]), 0, n, n, 0, False)
+            here = _work_pointers(recorded, calls[n][i])
+            assert here and not here & mine and seen.setdefault(n, here) == here
+        work = k._workspace(0, calls[sizes[0]][i]["x"].device)
+        for key, buffer in work._buffers.items():
+            need = max(x.numel() * x.element_size() for held, x in work.items() if held[:2] == key)
+            assert buffer.numel() <= max(8, 1.5 * need)
+        assert sum(x.numel() for x in work._outgrown) <= 2 * sum(x.numel() for x in work._buffers.values())
+        recorded.clear()
+        launch()
+        assert _work_pointers(recorded, calls[sizes[0]][i]) == mine
 
 
 def test_each_stream_has_its_own_trip_count_and_finish_counter(tmp_path, recorded):
