@@ -110,6 +110,9 @@ def _on(stream: int):
     return cuda.stream(cuda.ExternalStream(stream) if stream else cuda.default_stream())
 
 
+_UNMADE = object()
+
+
 class _Workspace(dict):
     """What a kernel's launches on one stream of one GPU work in: its scratch
     tensors by ``(what, name, *sizes)``, each made when first asked for.  A
@@ -199,7 +202,7 @@ class DeviceKernel:
         self.steps_max = None     # a fast entry's largest trips a sample (one int32 cell)
         self.steps_sum = None     # a fast entry's trips over every sample (one int64 cell)
         self._major = (sidecar.get("sample_major") or {}).get("planes") or []
-        self._direct = self._direct_plan()
+        self._direct_held = _UNMADE
 
     # -- validation ----------------------------------------------------------
     def _real_dtype(self):
@@ -208,6 +211,18 @@ class DeviceKernel:
 
     def caller_planes(self) -> list:
         return [n for n, p in self.planes.items() if not p.get("scratch") and n != FUSED_STEPS_PLANE]
+
+    @property
+    def _direct(self):
+        """:meth:`_direct_plan`, made by the first run (it names torch's types,
+        which loading a kernel does not import)."""
+        if self._direct_held is _UNMADE:
+            self._direct_held = self._direct_plan()
+        return self._direct_held
+
+    @_direct.setter
+    def _direct(self, plan):
+        self._direct_held = plan
 
     def _direct_plan(self):
         """What :meth:`run_direct` checks per plane, in ``arg_spec`` order:

@@ -4,6 +4,8 @@ them the runtime's own."""
 
 from __future__ import annotations
 
+from pathlib import Path
+
 import pytest
 
 import hawk_amd as hawk
@@ -217,3 +219,29 @@ def test_a_cut_chain_crosses_in_planes_of_its_stream_one_call_at_a_time(tmp_path
         assert other.is_alive() and not recorded
     other.join(10)
     assert len(recorded) == len(k.segments) > 1
+
+
+def test_loading_a_kernel_imports_no_torch(tmp_path):
+    """hawk.load of a kernel with no code object of its own, and the load of
+    any other past its code object, leave torch alone."""
+    import subprocess
+    import sys
+    from hawk_amd import examples as E
+    hawk.build([E.mm16, E.energy], tmp_path)
+    text = """
+import sys
+import hawk_amd as hawk
+from hawk_amd import _core
+class Library:
+    def __init__(self, code): pass
+    def entry(self, name): return name
+class Block:
+    def __init__(self, descriptor): pass
+_core.DeviceLibrary, _core.ArgBlock = Library, Block
+for name in ("mm16", "energy"):
+    hawk.load(sys.argv[1], name)
+    assert "torch" not in sys.modules, name
+"""
+    done = subprocess.run([sys.executable, "-c", text, str(tmp_path)], capture_output=True, text=True,
+                          cwd=Path(__file__).resolve().parent.parent)
+    assert done.returncode == 0, done.stderr
