@@ -2104,6 +2104,11 @@ constexpr long long kFewKeys = 512;
 // groups a wave: 7.1 and 9.8).
 constexpr long long kOneLaunchRows = 16 * kFoldLanes;
 
+// Whether a keyed ordered sum goes group by group, its group values in scratch.
+constexpr bool keyed_by_groups(long long keys, long long group) {
+    return group > (keys < kFewKeys / 4 ? kOneLaunchRows : kVirtualLanes);
+}
+
 // The ordered sum in T (hk_ordered_sum_f64 / _f32): the lanes, then the fold;
 // up to kOneLaunchRows rows one launch of the keyed sum's kernel.
 // A float sum keeps the double layout's offsets, its data in the front of
@@ -2165,7 +2170,7 @@ int keyed_ordered_sum(const T* u, int64_t n, int64_t group, T* out, void* scratc
         else hipLaunchKernelGGL((hawk_keyed_wave<T, 16>), grid, dim3(256), 0, s, u, len, keys, out);
         return launch_error("hawk_keyed_wave launch");
     }
-    if (group <= (keys < kFewKeys / 4 ? kOneLaunchRows : kVirtualLanes)) {
+    if (!keyed_by_groups(keys, group)) {
         const dim3 grid(static_cast<unsigned>(keys));
         if (keys < kFewKeys && group <= kOneLaunchRows)
             hipLaunchKernelGGL((hawk_keyed_rows<T, 16>), grid, dim3(1024), 0, s, u, len, out);
@@ -2436,8 +2441,8 @@ int hk_ordered_sum_f64_noalloc(const double* u, int64_t n, double* out, void* st
 size_t hk_keyed_ordered_sum_scratch_bytes(int64_t n, int64_t group) {
     if (n <= 0 || group <= 0 || n % group != 0) return 0;
     if (n == group) return kSumScratch;
-    if (group <= kOneLaunchRows) return 256;                 // the keys read their rows directly
-    // group values (the entry's size for longer keys, a lane partial each, holds them too)
+    if (!keyed_by_groups(n / group, group)) return 256;      // the keys read their rows directly
+    // group values; for keys past 65536 rows the entry's size, a lane partial each, stays
     return sizeof(double) * static_cast<size_t>(n / group) *
                static_cast<size_t>(group > kVirtualLanes ? kVirtualLanes : kGroups) + 256;
 }

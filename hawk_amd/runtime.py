@@ -809,7 +809,7 @@ class DeviceKernel:
                                        stream)
             elif t["op"] == "keyed_sum":
                 scratch = work.bytes(("keyed", t["out"], n), _core.keyed_ordered_sum_scratch_bytes(n, t["group"]),
-                                     zero=True)
+                                     zero=t["group"] == n)
                 fn = _core.keyed_ordered_sum_f32 if self._is_f32(t["out"]) else _core.keyed_ordered_sum
                 fn(bound[t["u"]].data_ptr(), n, t["group"], bound[t["out"]].data_ptr(), scratch.data_ptr(), stream)
             elif t["op"] == "ordered_fold":
@@ -1173,7 +1173,8 @@ class Prepared:
                 self.steps.append((_core.band_ordered_sum, args))
             elif t["op"] == "keyed_sum":
                 scratch = work.bytes(("keyed", t["out"], self.n),
-                                     _core.keyed_ordered_sum_scratch_bytes(self.n, t["group"]), zero=True)
+                                     _core.keyed_ordered_sum_scratch_bytes(self.n, t["group"]),
+                                     zero=t["group"] == self.n)
                 args = (bound[t["u"]].data_ptr(), self.n, t["group"], bound[t["out"]].data_ptr(), scratch.data_ptr())
                 self.steps.append((_core.keyed_ordered_sum_f32 if kernel._is_f32(t["out"]) else _core.keyed_ordered_sum,
                                    args))

@@ -171,6 +171,17 @@ def test_team_stage_arguments_are_checked_before_any_launch():
     assert L.hk_mm16_f64(ins, 2, outs, 1, prods, 0, None) == 0     # no samples: nothing launched
 
 
+def test_keyed_ordered_sum_scratch_is_what_its_kernels_use():
+    """Group values (64 a key) only where few keys are long: keys a workgroup
+    sums whole read their rows directly."""
+    size = _core.lib().hk_keyed_ordered_sum_scratch_bytes
+    for group in (65, 1024, 1025, 16_384):
+        assert size(2 * group, group) == size(600 * group, group) == 256
+    for group in (16_385, 65_536):
+        assert [size(keys * group, group) for keys in (128, 400, 5000)] == [256] * 3
+        assert [size(keys * group, group) for keys in (2, 127)] == [8 * 64 * keys + 256 for keys in (2, 127)]
+
+
 def test_scatter_chunk_rule():
     """clamp(n // max(cells, 1), 1, 256), the reference's own vectors."""
     ga = golden("scatter_chunks")
