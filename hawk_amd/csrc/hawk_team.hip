@@ -2104,6 +2104,15 @@ constexpr long long kFewKeys = 512;
 // groups a wave: 7.1 and 9.8).
 constexpr long long kOneLaunchRows = 16 * kFoldLanes;
 
+// Waves a key of hawk_keyed_comp: sixteen for few or long keys (see there), four
+// otherwise and where sixteen would pass a launch's 2^32 - 1 threads.
+constexpr int keyed_comp_waves(long long keys, long long group) {
+    return (keys < kFewKeys || group > 8192) && keys * 1024 < (1LL << 32) ? 16 : 4;
+}
+static_assert(keyed_comp_waves(600, 8193) == 16 && keyed_comp_waves((1LL << 22) - 1, 8193) == 16 &&
+              keyed_comp_waves(1LL << 22, 8193) == 4 && keyed_comp_waves((1LL << 24) - 1, 8193) == 4,
+              "up to 2^24 - 1 keys of any length fit a launch");
+
 // Whether a keyed ordered sum goes group by group, its group values in scratch.
 constexpr bool keyed_by_groups(long long keys, long long group) {
     return group > (keys < kFewKeys / 4 ? kOneLaunchRows : kVirtualLanes);
@@ -2279,7 +2288,7 @@ int keyed_sample_sum(const T* u, int64_t n, int64_t group, T* out, void* stream,
         return launch_error("hawk_keyed_comp_wave launch");
     }
     const dim3 grid(static_cast<unsigned>(keys));
-    if (keys < kFewKeys || group > 8192)
+    if (keyed_comp_waves(keys, group) == 16)
         hipLaunchKernelGGL((hawk_keyed_comp<T, 16>), grid, dim3(1024), 0, s, u, len, out);
     else hipLaunchKernelGGL((hawk_keyed_comp<T, 4>), grid, dim3(256), 0, s, u, len, out);
     return launch_error("hawk_keyed_comp launch");

@@ -157,6 +157,29 @@ def test_keyed_default_sum_routes(tmp_path, gpu, mode, keys, group):
     assert (np.isnan(got) == nan).all() and got[~nan].tobytes() == want[~nan].tobytes()
 
 
+def test_default_sums_of_more_keys_than_sixteen_waves_each_launch(gpu):
+    """2^22 keys of 8193 float32 samples: sixteen waves a key would pass the
+    2^32 - 1 threads of a launch, four do not.  A 137 GB plane, its first and
+    last keys checked."""
+    import oracle_lib as O
+    import torch
+    from hawk_amd import _core
+    keys, group = 1 << 22, 8193
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < keys * group * 4 + (4 << 30):
+        pytest.skip("the plane does not fit the memory that is free")
+    u = torch.empty(keys * group, dtype=torch.float32, device=gpu)
+    ends = np.random.default_rng(22).normal(size=2 * group).astype(np.float32)
+    u[:group], u[-group:] = (torch.from_numpy(e).to(gpu) for e in (ends[:group], ends[group:]))
+    out = torch.zeros(keys, dtype=torch.float32, device=gpu)
+    _core.keyed_sample_sum_f32(u.data_ptr(), keys * group, group, out.data_ptr(),
+                               torch.cuda.current_stream().cuda_stream)
+    got = torch.stack((out[0], out[-1])).cpu().numpy()
+    del u
+    torch.cuda.empty_cache()
+    assert got.tobytes() == O.keyed_sample_sum(ends, group).tobytes()
+
+
 @pytest.mark.parametrize("mode", ["float64", "float32"])
 @pytest.mark.parametrize("keys, group", [
     (9, 1), (70, 3), (257, 16), (5, 17), (7, 33), (1025, 64), (5, 65), (9, 128), (5, 129), (6, 256), (5, 257),
