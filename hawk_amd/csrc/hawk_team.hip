@@ -1017,7 +1017,9 @@ __device__ __forceinline__ void walk_load(const int* __restrict__ key, const T* 
 // of kAhead chunks are in flight while a third is added: 64 loads a thread,
 // since a grid of one thread per cell (65536 at the split walk's largest)
 // holds only a wave or two per SIMD to cover HBM's latency.  A short block
-// reads only the groups of 8 chunks it holds.
+// reads only the groups of 8 chunks it holds; a whole one reads all its chunks
+// with no test among the loads (256 chunks, fp64, every block by groups / this:
+// 64 cells 13.6 / 7.5 us, 1000 cells 15.7 / 10.2, 65536 cells 28.5 / 24.6).
 template <class T>
 __global__ __launch_bounds__(256) void hawk_scatter_cells(const T* __restrict__ parts, long long cells,
                                                           int chunks, T* __restrict__ target) {
@@ -1025,6 +1027,11 @@ __global__ __launch_bounds__(256) void hawk_scatter_cells(const T* __restrict__ 
     if (c >= cells) return;
     constexpr int kAhead = 32;
     auto fetch = [&](int b, T (&x)[kAhead]) {
+        if (b + kAhead <= chunks) {
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q) x[q] = parts[static_cast<long long>(b + q) * cells + c];
+            return;
+        }
 #pragma unroll
         for (int q = 0; q < kAhead; ++q) x[q] = T(0);
 #pragma unroll

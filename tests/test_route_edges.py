@@ -121,6 +121,31 @@ def test_ordered_scatter_peers(gpu, mode, cells, n, each):
     assert not status[1:].any()
 
 
+@pytest.mark.parametrize("mode", ["float64", "float32"])
+def test_ordered_scatter_partials(gpu, mode):
+    """Every number of chunks around the fold's blocks of 32 and groups of 8:
+    the serial walk's bits."""
+    import oracle_lib as O
+    import torch
+    from hawk_amd import _core
+    dt = np.float32 if mode == "float32" else np.float64
+    fn = _core.ordered_scatter_f32 if mode == "float32" else _core.ordered_scatter
+    for chunks in (1, 2, 7, 8, 9, 31, 32, 33, 40, 41, 63, 64, 65, 95, 96, 97, 128, 255, 256):
+        for cells in (7, 300):
+            n = cells * chunks + cells // 2
+            assert _core.scatter_chunks(n, cells) == chunks
+            g = np.random.default_rng(n)
+            key, x = g.integers(-1, cells, n).astype(np.int32), g.normal(size=n).astype(dt)
+            acc0 = g.normal(size=cells).astype(dt)
+            want, _ = O.ordered_scatter(key, x, acc0)
+            kd, xd, acc = (torch.from_numpy(a).to(gpu) for a in (key, x, acc0))
+            scratch = torch.full((_core.ordered_scatter_scratch_bytes(n, cells),), 255, dtype=torch.uint8, device=gpu)
+            status = torch.zeros(257, dtype=torch.int32, device=gpu)
+            fn(kd.data_ptr(), xd.data_ptr(), n, acc.data_ptr(), cells, scratch.data_ptr(), status.data_ptr(),
+               torch.cuda.current_stream().cuda_stream)
+            assert acc.cpu().numpy().tobytes() == want.tobytes(), (chunks, cells)
+
+
 def _per_key(group, policy):
     import hawk_amd as hawk
     from hawk_amd import Grid, Kernel, Scalar
