@@ -26,11 +26,10 @@ constexpr int kVirtualLanes = 65536;   // reference hawk/emit/team.py:21-23
 constexpr int kFoldLanes = 1024;
 constexpr int kGroups = 64;            // reference hawk/ir/team.py:649 GROUPS
 constexpr int kLaneBlock = 256;
-// Rows a lane keeps in flight twice over: 32 in float64, 64 in float32 (with 32,
-// a float sum of 2^26 rows took 58 us, with 64 47, one batch at a time 88), 8
-// up to that many rows (testing 64 loads that read nothing costs 1.3 us).
-template <class T> constexpr int kSumBatch = 256 / static_cast<int>(sizeof(T));
-constexpr int kSumFew = 8;
+// Rows of a batch: 32, and 64 in float32 past 64 rows a lane (2^26 float rows:
+// 58 us in batches of 32, 47 of 64, 88 with one batch at a time).
+constexpr int kSumBatch = 32;
+constexpr int kSumLong = 64;
 
 // Scratch layout (bytes): lanes[65536] f64 | gp[64] f64 | ticket u32 (+pad).
 constexpr size_t kLanesBytes = sizeof(double) * kVirtualLanes;
@@ -40,11 +39,14 @@ constexpr size_t kSumScratch = kLanesBytes + kGpBytes + 256;
 // Virtual lane l = blockIdx.x*256 + threadIdx.x adds u[l], u[l+65536], ... in
 // order from +0.0.  A batch of rows is in flight while the one
 // before it is added (one wave a SIMD holds the lanes, so nothing else covers
-// the loads' latency); a row past the end adds +0.0, which leaves a sum that is
-// never -0.0 as it is.  The fold's ticket is cleared here, one launch ahead of
+// the loads' latency); Once: all rows are one batch.  A row past the end adds
+// +0.0, which leaves a sum that is never -0.0 as it is, and a group of eight
+// rows past every lane's end is neither tested row by row nor added (testing
+// 64 loads that read nothing cost 1.5 us of a float sum of 524 289 to
+// 5 000 000 rows).  The fold's ticket is cleared here, one launch ahead of
 // the fold that takes it, so a sum never depends on what an earlier call left
 // in its scratch.
-template <class T, int Batch>
+template <class T, int Batch, bool Once>
 __global__ __launch_bounds__(kLaneBlock) void hawk_sum_lanes(const T* __restrict__ u,
                                                               long long n,
                                                               T* __restrict__ lanes,
@@ -56,27 +58,41 @@ __global__ __launch_bounds__(kLaneBlock) void hawk_sum_lanes(const T* __restrict
     T s = T(0);
     auto load = [&](long long r, T (&a)[Batch]) {
         const T* p = u + r * kStep + l;
-        if ((r + Batch) * kStep <= n) {
+        if (!Once && (r + Batch) * kStep <= n) {
 #pragma unroll
             for (int k = 0; k < Batch; ++k) a[k] = __builtin_nontemporal_load(p + k * kStep);
         } else if (r < rows) {
             const int left = n - r * kStep - l <= 0 ? 0 : static_cast<int>((n - r * kStep - l + kStep - 1) / kStep);
+            const int held = static_cast<int>(rows - r);
 #pragma unroll
-            for (int k = 0; k < Batch; ++k) a[k] = k < left ? __builtin_nontemporal_load(p + k * kStep) : T(0);
+            for (int k8 = 0; k8 < Batch; k8 += 8) {
+                if (k8 >= held) break;                       // the whole grid
+#pragma unroll
+                for (int k = k8; k < k8 + 8; ++k) a[k] = k < left ? __builtin_nontemporal_load(p + k * kStep) : T(0);
+            }
         }
     };
     auto add = [&](long long r, const T (&a)[Batch]) {
-        if (r >= rows) return;
+        const long long held = rows - r;
 #pragma unroll
-        for (int k = 0; k < Batch; ++k) s += a[k];
+        for (int k8 = 0; k8 < Batch; k8 += 8) {
+            if (k8 >= held) break;                           // the whole grid
+#pragma unroll
+            for (int k = k8; k < k8 + 8; ++k) s += a[k];
+        }
     };
-    T a[Batch], b[Batch];
+    T a[Batch];
     load(0, a);
-    for (long long r = 0; r < rows; r += 2 * Batch) {
-        load(r + Batch, b);
-        add(r, a);
-        load(r + 2 * Batch, a);
-        add(r + Batch, b);
+    if constexpr (Once) {
+        add(0, a);
+    } else {
+        T b[Batch];
+        for (long long r = 0; r < rows; r += 2 * Batch) {
+            load(r + Batch, b);
+            add(r, a);
+            load(r + 2 * Batch, a);
+            add(r + Batch, b);
+        }
     }
     lanes[l] = s;
 }
@@ -2145,10 +2161,13 @@ int ordered_sum(const T* u, int64_t n, T* out, void* scratch, void* stream, cons
     }
     const dim3 grid(kVirtualLanes / kLaneBlock), block(kLaneBlock);
     const long long len = n;
-    if (n <= kSumFew * static_cast<long long>(kVirtualLanes))
-        hipLaunchKernelGGL((hawk_sum_lanes<T, kSumFew>), grid, block, 0, s, u, len, lanes, ticket);
+    auto rows_up_to = [n](int rows) { return n <= rows * static_cast<int64_t>(kVirtualLanes); };
+    if (rows_up_to(kSumBatch))
+        hipLaunchKernelGGL((hawk_sum_lanes<T, kSumBatch, true>), grid, block, 0, s, u, len, lanes, ticket);
+    else if (sizeof(T) == 8 || rows_up_to(2 * kSumBatch))
+        hipLaunchKernelGGL((hawk_sum_lanes<T, kSumBatch, false>), grid, block, 0, s, u, len, lanes, ticket);
     else
-        hipLaunchKernelGGL((hawk_sum_lanes<T, kSumBatch<T>>), grid, block, 0, s, u, len, lanes, ticket);
+        hipLaunchKernelGGL((hawk_sum_lanes<T, kSumLong, false>), grid, block, 0, s, u, len, lanes, ticket);
     int rc = launch_error("hawk_sum_lanes launch");
     if (rc != HK_OK) return rc;
     hipLaunchKernelGGL(hawk_sum_fold<T>, dim3(kGroups), dim3(256), 0, s, lanes, gp, ticket, out);

@@ -229,6 +229,27 @@ def test_ordered_sum_routes(tmp_path, gpu, mode, keys, group):
 
 
 @pytest.mark.parametrize("mode", ["float64", "float32"])
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 16, 31, 32, 33, 40, 63, 64, 65, 72, 95, 96, 127, 128, 129, 193])
+def test_ordered_sum_batches(gpu, mode, rows):
+    """Every kind of last batch a virtual lane can have, whole, one row short of
+    a group and one past: the fixed tree's bits."""
+    import oracle_lib as O
+    import torch
+    from hawk_amd import _core
+    dt = np.float32 if mode == "float32" else np.float64
+    g = np.random.default_rng(rows)
+    x = (g.normal(size=65_536 * rows) * 2.0 ** g.integers(-10, 10, 65_536 * rows)).astype(dt)
+    x[g.random(x.size) < 0.05] = -0.0
+    u, out = torch.from_numpy(x).to(gpu), torch.full((1,), 7.0, dtype=torch.float32 if mode == "float32" else
+                                                     torch.float64, device=gpu)
+    scratch = torch.zeros(_core.ordered_sum_scratch_bytes(), dtype=torch.uint8, device=gpu)
+    fn = _core.ordered_sum_f32 if mode == "float32" else _core.ordered_sum
+    for n in (65_536 * rows, 65_536 * rows - 1, 65_536 * (rows - 1) + 1, 65_536 * rows - 40_000):
+        fn(u.data_ptr(), n, out.data_ptr(), scratch.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        assert out.cpu().numpy().tobytes() == O.keyed_ordered_sum(x[:n], n).tobytes(), n
+
+
+@pytest.mark.parametrize("mode", ["float64", "float32"])
 @pytest.mark.parametrize("rows", [1, 255, 256, 257, 4095, 4096, 4097, 2 * 4096, 128 * 4096 + 1, 129 * 4096,
                                   1024 * 4096, 1025 * 4096 + 17])
 def test_rows_finish_together(gpu, mode, rows):
