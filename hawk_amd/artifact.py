@@ -123,9 +123,11 @@ def launch_shape(plan, mode: str) -> tuple:
     if mode == "float32" and nbytes <= STREAM_BYTES and fp_ops_per_sample(plan.source) <= LIGHT_OPS:
         shape = LIGHT_SHAPE
     else:
-        # five to eight 8-byte planes, or float32 ones
-        low, high = (16, 32) if mode == "float32" else (32, 64)
-        shape = (256, 1) if low < nbytes <= high else (128, 1)
+        # five to eight 8-byte planes, or five to sixteen float32 ones (over
+        # 10 000 019 samples, 128 x 1 and 256 x 1: six rows 44.8 and 42.9 us,
+        # eight 68 and 61, nine 71.1 and 63.6, sixteen 143 and 131)
+        low = 16 if mode == "float32" else 32
+        shape = (256, 1) if low < nbytes <= 64 else (128, 1)
     if stage.row_sums and not stage.fused_folds:
         # row reductions take two samples a lane (the paired layout)
         shape = (shape[0], 2)
