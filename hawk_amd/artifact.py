@@ -22,7 +22,7 @@ from . import policy as _policy
 from .emit_hip import fp_ops_per_sample
 from .resources import kernel_resources
 from .emit_hip import plan_kernel, sample_major_entry, sample_major_name, sample_major_planes
-from .ir import AUTO_K_MAX, FINISHED_PLANE, Finish, HawkError
+from .ir import AUTO_K_MAX, FINISHED_PLANE, Finish, HawkError, topo
 from .targets import TARGETS, row
 from .trace import Kernel
 
@@ -81,12 +81,35 @@ def _stage_bytes(plan, mode: str) -> int:
 #: 0.36 at 512 x 2, 0.28 at 1024 x 2, 0.41 at 1024 x 4).
 GATHER_SHAPE = (1024, 2)
 
-#: The launch shape of a stage whose tables are read by its lane axes alone (no
-#: index plane): a wave reads few cells, so nothing waits on a gather, and
-#: workgroups of 2048 samples leave a last round nearly empty.  The nets' losses
-#: at 1024 x 2 and 256 x 1: 16384 nets of 40 samples 21.2 and 14.4 us, 8192 of 96
-#: 23.7 and 16.1, 16384 of 64 22.8 and 21.4, 32768 of 16 12.3 and 12.2.
-LANE_TABLE_SHAPE = (256, 1)
+#: The launch shapes of a stage whose tables are read along its lanes
+#: (:func:`_along_lanes`): a wave's reads share lines or stride through them, so
+#: nothing waits on a gather, and workgroups of 2048 samples leave a last round
+#: nearly empty.  A heavy stage (past LANE_TABLE_OPS) runs one sample a thread:
+#: the nets' losses (287 ops) at 1024 x 2, 256 x 2 and 256 x 1, 16384 nets of 40
+#: samples 21 / 18 / 14 us, 131072 of 64 189 / 165 / 132.  A lighter one takes
+#: two, for its loads (10^7 samples, the same shapes, us).  float32: three cells
+#: a key of 64 samples (26 ops) 18.2 / 17.0 / 24.3, sixteen of 16 (130 ops) 31.4 /
+#: 30.7 / 32.4, twenty-four of 4 (194 ops) 44.8 / 44.9 / 44.0.  float64: 26 ops
+#: 32.6 / 29.6 / 35.2; eight of 1000 (66 ops) 41.0 / 38.8 / 38.4, over 3 * 10^7
+#: 122 / 118 / 112.
+LANE_TABLE_OPS = {"float32": 160, "float64": 32}
+LANE_TABLE_SHAPES = ((256, 2), (256, 1))
+
+#: What a table index along the lanes is made of.
+_LANE_KINDS = {"lane_axis", "loop_index", "iconst", "add", "sub", "mul"}
+
+
+def _along_lanes(stage) -> bool:
+    """Whether every table of ``stage`` is read at lane coordinates, loop
+    counters, constants, their sums and products: an index with a remainder or
+    a quotient of its own scatters a wave's reads as an index plane does (a
+    float64 table of 10^6 cells read at (7919 lane) mod its size, 10^7 samples:
+    107 us at GATHER_SHAPE, 164 at 256 x 2)."""
+    if any(info["role"] == "per_sample" and info["dtype"] in ("i32", "u32") for info in stage.planes.values()):
+        return False
+    reads = [n for n in topo([node for _, node in stage.writes]) if n.kind in ("gather", "table_index")]
+    return all(m.kind in _LANE_KINDS for n in reads for m in topo(n.operands[1:]))
+
 
 #: The launch shape of a light stream whose planes are all scalar float64
 #: planes: 64 threads of one pair of adjacent samples, read and written 16
@@ -115,8 +138,10 @@ def launch_shape(plan, mode: str) -> tuple:
     infos = stage.planes.values()
     if (any(info["role"] == "lookup" for info in infos) and not stage.row_sums
             and not stage.fused_folds and not stage.key_writes and stage.guard is None and stage.finish is None):
-        keyed = any(info["role"] == "per_sample" and info["dtype"] in ("i32", "u32") for info in infos)
-        return GATHER_SHAPE if keyed else LANE_TABLE_SHAPE
+        if not _along_lanes(stage):
+            return GATHER_SHAPE
+        line = LANE_TABLE_OPS["float32" if mode == "float32" else "float64"]
+        return LANE_TABLE_SHAPES[fp_ops_per_sample(plan.source) > line]
     nbytes = _stage_bytes(plan, mode)
     if nbytes <= STREAM_BYTES and fp_ops_per_sample(plan.source) <= STREAM_OPS:
         return PAIR_SHAPE if pair_candidate(stage, mode) else STREAM_SHAPE
