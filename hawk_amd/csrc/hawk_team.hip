@@ -1032,18 +1032,20 @@ __device__ __forceinline__ void walk_load(const int* __restrict__ key, const T* 
 // target: target[c] += sum (reference hawk/emit/team.py:437-460).  Two blocks
 // of kAhead chunks are in flight while a third is added: 64 loads a thread,
 // since a grid of one thread per cell (65536 at the split walk's largest)
-// holds only a wave or two per SIMD to cover HBM's latency.  A short block
-// reads only the groups of 8 chunks it holds; a whole one reads all its chunks
-// with no test among the loads (256 chunks, fp64, every block by groups / this:
-// 64 cells 13.6 / 7.5 us, 1000 cells 15.7 / 10.2, 65536 cells 28.5 / 24.6).
-template <class T>
+// holds only a wave or two per SIMD to cover HBM's latency.  Few: at most
+// kAhead chunks, one block, by the groups of 8 chunks it holds.  Otherwise a
+// whole block reads all its chunks with no test among the loads (256 chunks,
+// fp64, every block by groups / this: 64 cells 13.6 / 7.5 us, 1000 cells 15.7 /
+// 10.2, 65536 cells 28.5 / 24.6; with both forms in one kernel, 16 chunks of
+// 262144 cells took 9.5 us instead of 8.3).
+constexpr int kAhead = 32;
+template <class T, bool Few>
 __global__ __launch_bounds__(256) void hawk_scatter_cells(const T* __restrict__ parts, long long cells,
                                                           int chunks, T* __restrict__ target) {
     const long long c = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
     if (c >= cells) return;
-    constexpr int kAhead = 32;
     auto fetch = [&](int b, T (&x)[kAhead]) {
-        if (b + kAhead <= chunks) {
+        if (!Few && b + kAhead <= chunks) {
 #pragma unroll
             for (int q = 0; q < kAhead; ++q) x[q] = parts[static_cast<long long>(b + q) * cells + c];
             return;
@@ -1063,19 +1065,25 @@ __global__ __launch_bounds__(256) void hawk_scatter_cells(const T* __restrict__ 
             }
         }
     };
-    T x0[kAhead], x1[kAhead];
-    fetch(0, x0);
-    fetch(kAhead, x1);
+    T x0[kAhead];
     T s = T(0);
-    for (int b = 0; b < chunks; b += kAhead) {
-        T x2[kAhead];
-        fetch(b + 2 * kAhead, x2);
+    fetch(0, x0);
+    if constexpr (Few) {
 #pragma unroll
         for (int q = 0; q < kAhead; ++q) s = s + x0[q];
+    } else {
+        T x1[kAhead];
+        fetch(kAhead, x1);
+        for (int b = 0; b < chunks; b += kAhead) {
+            T x2[kAhead];
+            fetch(b + 2 * kAhead, x2);
 #pragma unroll
-        for (int q = 0; q < kAhead; ++q) {
-            x0[q] = x1[q];
-            x1[q] = x2[q];
+            for (int q = 0; q < kAhead; ++q) s = s + x0[q];
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q) {
+                x0[q] = x1[q];
+                x1[q] = x2[q];
+            }
         }
     }
     target[c] = target[c] + s;
@@ -2431,8 +2439,12 @@ int ordered_scatter(const int32_t* key, const T* v, int64_t n, T* target, int64_
         }
     }
     const long long grid = (cells + 255) / 256;
-    hipLaunchKernelGGL(hawk_scatter_cells<T>, dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, parts,
-                       static_cast<long long>(cells), chunks, target);
+    if (chunks <= kAhead)
+        hipLaunchKernelGGL((hawk_scatter_cells<T, true>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, parts,
+                           static_cast<long long>(cells), chunks, target);
+    else
+        hipLaunchKernelGGL((hawk_scatter_cells<T, false>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, parts,
+                           static_cast<long long>(cells), chunks, target);
     return launch_error("hawk_scatter_cells launch");
 }
 
