@@ -1372,8 +1372,10 @@ __device__ __forceinline__ void fold_heads(Sh& sh, int c) {
 // in the window's place (a scan over the keys' peer counts gives the runs'
 // starts), and the lowest lane adds its run from consecutive reads: finding
 // each peer in the match mask instead (count trailing zeros, clear the bit)
-// took most of a window's instructions.  A wave's LDS operations complete in
-// issue order, so a key's windows meet its accumulator one after another.
+// took most of a window's instructions.  In the widest tail window a window of
+// one key alone is a chain by rows (3*10^7 sorted lanes into 65537 cells 1586 ->
+// 816 us, five keys 1640 -> 634).  A wave's LDS operations complete in issue
+// order, so a key's windows meet its accumulator one after another.
 // With the head chains by rows, on MI355X in float64: 2^23 lanes into 64
 // uniform cells 120.5 -> 82.1 us, into 64 Zipf cells 99.0 -> 72.2, into 4096
 // uniform cells 84.6 -> 73.7, 2^26 Zipf lanes into 65536 cells 571 -> 524, and
@@ -1391,6 +1393,7 @@ __device__ void fold_class(Sh& sh, int c) {
     constexpr int kLow = Sh::kPeers == 64 ? 6 : 7;
     constexpr int kBits = kKeys > 512 ? 10 : kKeys > 256 ? 9 : kKeys > 128 ? 8 : 7;
     static_assert(Sh::kPeers == (1u << kLow) && kKeys <= (1 << kBits), "class matching covers every key");
+    constexpr bool kChains = !Hot && Sh::kWindow == kTailRange;      // the others have no registers to spare
     unsigned long long* peer = sh.f.peer[wave];
     unsigned k = sh.key[s + lane];
     T x = sh.val[s + lane];
@@ -1424,20 +1427,53 @@ __device__ void fold_class(Sh& sh, int c) {
         T a = a0 + x;
         const unsigned long long more = __ballot(rank > 1u);
         if (more != 0ull) {
-            // a key has several peers: each key's to a run of their own in the window's place
-            const int peers = valid && rank == 0u ? static_cast<int>(__popcll(pm)) - 1 : 0;
-            const int start = static_cast<int>(wave_inclusive_scan(static_cast<unsigned>(peers))) - peers;
-            const int low = pm != 0ull ? static_cast<int>(__builtin_ctzll(pm)) : 0;
-            const int run = __builtin_amdgcn_ds_bpermute(low << 2, start);
-            if (rank != 0u) sh.val[base + run + static_cast<int>(rank) - 1] = x;
-            __builtin_amdgcn_wave_barrier();
-            const T* y = sh.val + base + start;
-            for (int left = peers; left > 0; left -= kPeerBlock, y += kPeerBlock) {
-                T r[kPeerBlock];
+            if (kChains && __ballot(valid && rank == 0u) == 1ull) {
+                // one key: its chain by rows, no peer looked for, and on through
+                // the whole windows of the same key that follow (sorted keys)
+                a = lane_value(a0, 0);
+                T r[4];
+                auto rows = [&](int at) {
 #pragma unroll
-                for (int q = 0; q < kPeerBlock; ++q) r[q] = y[q];
+                    for (int q = 0; q < 4; ++q) {
+                        const int i = at + 16 * q + (lane & 15);
+                        const T v = sh.val[i];                   // up to 63 entries past the run (the padding)
+                        r[q] = i < e ? v : T(0);
+                    }
+                };
+                rows(base);
+                const unsigned one = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(kv)));
+                while (base + 128 <= e && __ballot(nk == one) == ~0ull) {
+                    T y[4];
 #pragma unroll
-                for (int q = 0; q < kPeerBlock; ++q) a = a + (q < left ? r[q] : T(0));
+                    for (int q = 0; q < 4; ++q) y[q] = r[q];
+                    base += 64;
+                    rows(base);
+                    if (base + 64 < e) {
+                        nk = sh.key[base + 64 + lane];
+                        nx = sh.val[base + 64 + lane];
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) a = row_chain(a, y[q]);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (base + 16 * q < e) a = row_chain(a, r[q]);
+            } else {
+                // a key has several peers: each key's to a run of their own in the window's place
+                const int peers = valid && rank == 0u ? static_cast<int>(__popcll(pm)) - 1 : 0;
+                const int start = static_cast<int>(wave_inclusive_scan(static_cast<unsigned>(peers))) - peers;
+                const int low = pm != 0ull ? static_cast<int>(__builtin_ctzll(pm)) : 0;
+                const int run = __builtin_amdgcn_ds_bpermute(low << 2, start);
+                if (rank != 0u) sh.val[base + run + static_cast<int>(rank) - 1] = x;
+                __builtin_amdgcn_wave_barrier();
+                const T* y = sh.val + base + start;
+                for (int left = peers; left > 0; left -= kPeerBlock, y += kPeerBlock) {
+                    T r[kPeerBlock];
+#pragma unroll
+                    for (int q = 0; q < kPeerBlock; ++q) r[q] = y[q];
+#pragma unroll
+                    for (int q = 0; q < kPeerBlock; ++q) a = a + (q < left ? r[q] : T(0));
+                }
             }
         }
         if (valid && rank == 0u) {

@@ -51,7 +51,7 @@ def test_mm16_streamed_and_cached(tmp_path, gpu, mode, n, shift):
     (8192, 60_000, "zipf"), (8193, 60_000, "zipf"), (9000, 9000 * 31, "one"), (9000, 9000 * 32, "one"),
     (12_289, 100, "uniform"), (20_000, 20_000 * 191, "zipf"), (20_000, 20_000 * 192, "sorted"),
     (65_537, 65_537, "uniform"), (65_537, 400_003, "sorted"), (65_600, 700_001, "zipf"), (65_600, 300_000, "one"),
-    (289_792, 600_001, "zipf"), (289_793, 600_001, "zipf"), (1 << 20, 5_000, "uniform"), (70_000, 0, "uniform")])
+    (289_792, 600_001, "zipf"), (289_793, 600_001, "zipf"), (1 << 20, 5_000, "uniform"), (70_000, 0, "uniform"), (5_000_001, 700, "uniform")])
 def test_ordered_scatter_walks(tmp_path, gpu, mode, cells, n, keys):
     """Few chunks, many cells and their neighbours on the other walk: the
     serial walk's bits, skip keys and infinities among the lanes, and the bad
@@ -119,6 +119,43 @@ def test_ordered_scatter_peers(gpu, mode, cells, n, each):
        torch.cuda.current_stream().cuda_stream)
     assert acc.cpu().numpy().tobytes() == want.tobytes()
     assert not status[1:].any()
+
+
+@pytest.mark.parametrize("mode", ["float64", "float32"])
+@pytest.mark.parametrize("cells, chunks", [(12_289, 95), (12_289, 96), (16_384, 95), (16_384, 96), (16_385, 96),
+                                           (20_000, 192), (65_600, 130)])
+def test_ordered_scatter_long_runs(gpu, mode, cells, chunks):
+    """Runs of one key of every length about a window, in the class of one wave
+    of the tail and sorted over all cells, on both sides of the walks' lines:
+    the serial walk's bits, negative zeros and an infinity among the values."""
+    import oracle_lib as O
+    import torch
+    from hawk_amd import _core
+    dt = np.float32 if mode == "float32" else np.float64
+    n = cells * chunks + 77
+    assert _core.scatter_chunks(n, cells) == chunks
+    g = np.random.default_rng(cells + chunks)
+    x = (g.normal(size=n) * np.exp(g.normal(size=n))).astype(dt)
+    x[::3] = -0.0
+    x[n // 2] = np.inf
+    acc0 = np.full(cells, -0.0, dt)
+    fn = _core.ordered_scatter_f32 if mode == "float32" else _core.ordered_scatter
+    xd = torch.from_numpy(x).to(gpu)
+    scratch = torch.empty(_core.ordered_scatter_scratch_bytes(n, cells), dtype=torch.uint8, device=gpu)
+    status = torch.zeros(257, dtype=torch.int32, device=gpu)
+    lengths = np.array([1, 2, 63, 64, 65, 127, 128, 129, 192, 200, 1000])
+    run = np.repeat(np.arange(n // 100), np.resize(lengths, n // 100))[:n]
+    run = np.concatenate([run, np.zeros(n - run.size, run.dtype)])
+    high = 12_288 if cells > 12_296 else 0
+    for key in (high + run * 8 % max(8, cells - high), np.arange(n) * cells // n, np.full(n, cells - 1)):
+        key = np.minimum(key, cells - 1).astype(np.int32)
+        want, _ = O.ordered_scatter(key, x, acc0)
+        kd, acc = torch.from_numpy(key).to(gpu), torch.from_numpy(acc0).to(gpu)
+        print(f"scatter runs cells={cells} chunks={chunks} {mode}", flush=True)
+        fn(kd.data_ptr(), xd.data_ptr(), n, acc.data_ptr(), cells, scratch.data_ptr(), status.data_ptr(),
+           torch.cuda.current_stream().cuda_stream)
+        assert acc.cpu().numpy().tobytes() == want.tobytes()
+        assert not status[1:].any()
 
 
 @pytest.mark.parametrize("mode", ["float64", "float32"])
