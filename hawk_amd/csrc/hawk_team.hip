@@ -1874,17 +1874,22 @@ constexpr int kWideGroups = 2048;                // workgroups hawk_split_tail g
 
 // Which walk: the wide one where the split walk cannot go (more than 65536
 // cells) and where its workgroup a chunk leaves the chip idle for longer than
-// a second pass over the lanes takes.  Measured (fp64, split / wide, us, at
-// uniform keys; the same lines hold at Zipf keys): 65536 cells in 16 chunks
-// 113 / 31, in 64 135 / 72, in 128 164 / 129, in 183 195 / 175, in 256
-// 225 / 238; 20000 cells in 104 chunks 73 / 51, in 209 83 / 87.  Up to 12288
-// cells (no tail ranges) a chunk is at most three tiles: 10000 cells in 20
-// chunks 29 / 23, in 50 31 / 34; 4000 cells in 16 chunks 16 / 18.  Past 65536
-// cells, against a sorted walk of each chunk: 2^18 cells, 2^22 lanes 1470 us uniform
-// and 1395 us Zipf -> 74 and 166 us (uniform 68 since the folds gather peers
-// into runs, which both walks share).
+// a second pass over the lanes takes.  Measured (fp64, uniform keys, split /
+// wide, us; Zipf keys and float32 cross at about the same chunks): 65536 cells
+// in 16 chunks 105 / 32, in 64 124 / 67, in 128 149 / 121, in 191 178 / 172; 20000
+// in 96 62 / 43, in 191 66 / 67.  Few lanes in the tail make the split walk's
+// second pass short: 14000 cells in 96 chunks 42 / 40, in 128 45 / 45; 12289 in
+// 64 36 / 34, in 96 38 / 41, and with sorted keys (a chunk's lanes all in one
+// range's workgroup) in 64 83 / 128, in 160 90 / 182.  Up to 12288 cells (no
+// tail ranges) a chunk is at most three tiles: 10500 cells in 20 chunks 24 / 21,
+// in 31 25 / 26; 4000 cells in 16 chunks 16 / 18.  Past 65536 cells, against a
+// sorted walk of each chunk (a serial one past 2^19 cells): 2^18 cells, 2^22
+// lanes 1470 us -> 68 uniform, 1395 -> 166 Zipf; 10^3 lanes into 10^8 cells, 346
+// passes, 5.2 ms -> 4.9; 65537 cells, 3*10^7 sorted lanes 885 -> 816, 8*10^6
+// 499 -> 554.
 bool wide_walk(int64_t cells, int chunks) {
-    return cells > kSplitCells || chunks < (cells > kSplitHot ? 192 : cells > 2 * kTile ? 32 : 0);
+    return cells > kSplitCells ||
+           chunks < (cells > kSplitHot + kTile ? 192 : cells > kSplitHot ? 96 : cells > 2 * kTile ? 32 : 0);
 }
 
 template <class T>
