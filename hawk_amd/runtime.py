@@ -254,7 +254,9 @@ class DeviceKernel:
         launched.  ``False``, with nothing done, where any test fails or the
         call is not plain: :func:`run`'s general path then runs it or says what
         is wrong."""
-        plan = self._direct
+        plan = self._direct_held
+        if plan is _UNMADE:
+            plan = self._direct
         if plan is None or len(arrays) != len(plan) or type(base) is not int:
             return False
         if layout is not None and layout not in LAYOUTS:
@@ -998,8 +1000,9 @@ def run(kernel: DeviceKernel, *, base: int = 0, count: int | None = None, n_samp
     ``layout`` (``"samples_first"`` / ``"samples_last"``) and the markers
     :func:`hawk_amd.samples_first` / :func:`~hawk_amd.samples_last` say which
     axis of a per-sample plane holds the samples (:mod:`hawk_amd.layout`)."""
-    if steps is None and entry == "plain" and type(kernel) is DeviceKernel and kernel._direct is not None:
-        if kernel.run_direct(arrays, base, count, n_samples, layout, _stream_of(stream)):
+    if steps is None and entry == "plain" and type(kernel) is DeviceKernel and kernel._direct_held is not None:
+        if kernel.run_direct(arrays, base, count, n_samples, layout,
+                             _current_stream() if stream is None else _stream_of(stream)):
             return
     from . import layout as _layout
     torch = _torch()
