@@ -399,18 +399,59 @@ def test_sample_major_stage(tmp_path, gpu, mode, n):
                 assert torch.equal(part[name][..., n - 55:], ins[name][..., n - 55:])
 
 
+def test_sample_major_banded_and_tables(tmp_path, gpu):
+    """The stage over (N, w) planes in the banded mode, with its band rows, and
+    beside tables: the component-major run's bits."""
+    import hawk_amd as hawk
+    import torch
+    from hawk_amd import Grid, Mutable, Scalar, Table, Vector
+
+    @hawk.kernel
+    def banded_vec(v: Vector[3], w: Mutable[Vector[2]], s: Mutable[Scalar]):
+        w = hawk.math.vec(v[0] * v[1], v[2])
+        s = hawk.sum(v[0] * v[2])
+
+    @hawk.kernel
+    def by_key(lane: Grid["key", "sample":5], t: Table["key", "w":3], v: Vector[3], w: Mutable[Vector[2]]):
+        w = hawk.math.vec(v[0] * t.at(key=lane.key, w=0), v[1] + v[2] * t.at(key=lane.key, w=2))
+    n = 10_005
+    g = torch.Generator(device=gpu).manual_seed(5)
+    v = torch.randn(3, n, dtype=torch.float64, device=gpu, generator=g)
+    table = torch.randn(n // 5 * 3, dtype=torch.float64, device=gpu, generator=g)
+    for kernel, mode, more in ((banded_vec, "banded", dict(s=torch.zeros(1, dtype=torch.float64, device=gpu))),
+                               (by_key, "float64", dict(t=table)), (by_key, "banded", dict(t=table))):
+        (k,) = _unit(tmp_path, [kernel], mode)
+        last, first = (dict(more, v=p, w=torch.full(shape, 7.0, dtype=torch.float64, device=gpu))
+                       for p, shape in ((v, (2, n)), (v.t().contiguous(), (n, 2))))
+        hawk.run(k, layout="samples_last", **last)
+        cell = more["s"].clone() if "s" in more else None
+        assert k.takes_rows(first, ["v", "w"], "plain")
+        hawk.run(k, layout="samples_first", **first)
+        assert torch.equal(first["w"].t(), last["w"]) and not (last["w"] == 7.0).any()
+        assert cell is None or (torch.equal(more["s"], cell) and float(cell) != 0.0)
+
+
 def test_plain_calls_direct_and_general(tmp_path, gpu):
     """hawk.run's direct path for plain calls and its general path: the same
-    planes or the same refusal, call by call."""
+    planes or the same refusal, call by call, and each call on the path that
+    its planes say (True: the direct one)."""
     import hawk_amd as hawk
     import torch
     from hawk_amd import examples as E
     n = 1001
     direct, general = (_unit(tmp_path, [E.scale, E.energy_vjp, E.spd_solve]) for _ in range(2))
+    taken = []
+
+    def watched(run_direct):
+        def run(*args):
+            taken.append(run_direct(*args))
+            return taken[-1]
+        return run
     for k in general:
         k._direct = None
     for k in direct:
         assert k._direct is not None
+        k.run_direct = watched(k.run_direct)
 
     def t(*shape, dtype=torch.float64, device=gpu):
         return torch.randn(*shape, dtype=torch.float64, generator=torch.Generator().manual_seed(3)).to(dtype).to(device)
@@ -419,31 +460,35 @@ def test_plain_calls_direct_and_general(tmp_path, gpu):
     vjp = dict(v=v, bar_out=bar, bar_v=t(3, n))
     rows = dict(v=v.t().contiguous(), bar_out=bar, bar_v=t(n, 3))
     a = t(6, 6, 6) + 20.0 * torch.eye(6, dtype=torch.float64, device=gpu)[:, :, None]
-    calls = [(0, dict(scale, out=t(n))), (0, dict(scale, out=t(n), base=7, count=500)),
-             (0, dict(scale, out=t(n), base=7)), (0, dict(scale, out=t(n), count=0)), (0, dict(scale, a=3, out=t(n))),
-             (0, dict(scale, out=t(n), n_samples=n)), (0, dict(scale, out=t(n), n_samples=n - 1)),
-             (0, dict(scale, out=t(n), base=-1)), (0, dict(scale, out=t(n), count=n + 1)),
-             (0, dict(scale, out=t(n), base=True)), (0, dict(scale, a=True, out=t(n))),
-             (0, dict(scale, a=np.float64(2.0), out=t(n))), (0, dict(scale, a=x, out=t(n))),
-             (0, dict(scale)), (0, dict(scale, out=t(n), other=x)), (0, dict(scale, out=t(n - 1))),
-             (0, dict(scale, out=t(n, 1))), (0, dict(scale, out=t(n, dtype=torch.float32))),
-             (0, dict(scale, out=t(n, device="cpu"))), (0, dict(scale, out=t(2 * n)[::2])),
-             (0, dict(scale, out=torch.nn.Parameter(t(n)))), (0, dict(x=t(0), a=1.0, b=1.0, out=t(0))),
-             (0, dict(scale, out=t(n), layout="rows")), (0, dict(scale, out=t(n), steps=1)),
-             (0, dict(scale, out=t(n), entry="range")), (0, dict(scale, out=t(n), stream=torch.cuda.Stream())),
-             (1, vjp), (1, rows), (1, dict(vjp, layout="samples_last")), (1, dict(rows, layout="samples_first")),
-             (1, dict(rows, layout="samples_last")), (1, dict(vjp, layout="samples_first")),
-             (1, dict(vjp, v=rows["v"])), (1, dict(rows, v=hawk.samples_first(rows["v"]))),
-             (1, dict(v=t(3, 3), bar_out=t(3), bar_v=t(3, 3))),
-             (1, dict(v=t(3, 3), bar_out=t(3), bar_v=t(3, 3), layout="samples_first")),
-             (1, dict(v=t(3, 3), bar_out=t(3), bar_v=t(3, 3), layout="samples_last")),
-             (2, dict(A=a, b=t(6, 6), x=t(6, 6))), (2, dict(A=a, b=t(6, 6), x=t(6, 6), layout="samples_last")),
-             (2, dict(A=a.movedim(-1, 0).contiguous(), b=t(6, 6), x=t(6, 6), layout="samples_first"))]
-    for which, call in calls * 2:                    # twice: fresh and held bindings
+    small = dict(v=t(3, 3), bar_out=t(3), bar_v=t(3, 3))
+    calls = [(0, True, dict(scale, out=t(n))), (0, True, dict(scale, out=t(n), base=7, count=500)),
+             (0, True, dict(scale, out=t(n), base=7)), (0, True, dict(scale, out=t(n), count=0)),
+             (0, True, dict(scale, a=3, out=t(n))), (0, True, dict(scale, out=t(n), n_samples=n)),
+             (0, False, dict(scale, out=t(n), n_samples=n - 1)), (0, False, dict(scale, out=t(n), base=-1)),
+             (0, False, dict(scale, out=t(n), count=n + 1)), (0, False, dict(scale, out=t(n), base=True)),
+             (0, False, dict(scale, a=True, out=t(n))), (0, False, dict(scale, a=np.float64(2.0), out=t(n))),
+             (0, False, dict(scale, a=x, out=t(n))), (0, False, dict(scale)),
+             (0, False, dict(scale, out=t(n), other=x)), (0, False, dict(scale, out=t(n - 1))),
+             (0, False, dict(scale, out=t(n, 1))), (0, False, dict(scale, out=t(n, dtype=torch.float32))),
+             (0, False, dict(scale, out=t(n, device="cpu"))), (0, False, dict(scale, out=t(2 * n)[::2])),
+             (0, False, dict(scale, out=torch.nn.Parameter(t(n)))), (0, True, dict(x=t(0), a=1.0, b=1.0, out=t(0))),
+             (0, False, dict(scale, out=t(n), layout="rows")), (0, False, dict(scale, out=t(n), steps=1)),
+             (0, False, dict(scale, out=t(n), entry="range")),
+             (0, True, dict(scale, out=t(n), stream=torch.cuda.Stream())),
+             (1, True, vjp), (1, True, rows), (1, True, dict(vjp, layout="samples_last")),
+             (1, True, dict(rows, layout="samples_first")), (1, False, dict(rows, layout="samples_last")),
+             (1, False, dict(vjp, layout="samples_first")), (1, False, dict(vjp, v=rows["v"])),
+             (1, False, dict(rows, v=hawk.samples_first(rows["v"]))), (1, False, small),
+             (1, True, dict(small, layout="samples_first")), (1, True, dict(small, layout="samples_last")),
+             (2, False, dict(A=a, b=t(6, 6), x=t(6, 6))),
+             (2, True, dict(A=a, b=t(6, 6), x=t(6, 6), layout="samples_last")),
+             (2, True, dict(A=a.movedim(-1, 0).contiguous(), b=t(6, 6), x=t(6, 6), layout="samples_first"))]
+    for which, plain, call in calls * 2:             # twice: fresh and held bindings
         done = []
+        taken.clear()
         for k in (direct[which], general[which]):
             # fresh output planes a side, the same values in both
-            planes = {name: p.clone() if isinstance(p, torch.Tensor) and p.is_contiguous()
+            planes = {name: p.clone() if type(p) is torch.Tensor and p.is_contiguous()
                       and name in ("out", "bar_v", "x") and which + (name == "out") else p for name, p in call.items()}
             torch.cuda.synchronize()
             try:
@@ -453,7 +498,9 @@ def test_plain_calls_direct_and_general(tmp_path, gpu):
                              if isinstance(p, torch.Tensor)})
             except Exception as e:
                 done.append((type(e), str(e)))
-        assert done[0] == done[1], (which, {name: getattr(p, "shape", p) for name, p in call.items()}, done)
+        said = (which, {name: getattr(p, "shape", p) for name, p in call.items()}, done)
+        assert done[0] == done[1], said
+        assert any(taken) == plain, said
 
 
 def test_refused_param_leaves_bindings(tmp_path, gpu):
