@@ -1954,9 +1954,10 @@ __global__ __launch_bounds__(kWalkThreads) void hawk_wide_bin(
 }
 
 // The ordered scatter's scratch, in this order (each part 256-byte aligned):
-// parts[chunks][cells] f64; and for the split walk with tail ranges, the bin
-// offsets [chunks][tiles][ranges+1] u32, the bin keys [chunks][tiles][4096]
-// u16 and the bin values [chunks][tiles][4096] f64.
+// parts[chunks][cells] f64; and for the split walk with tail ranges and the
+// wide walk, the bin offsets [chunks][tiles][row] u32 (a range's and one more;
+// the wide walk's row ends in a bad-key flag), the bin keys
+// [chunks][tiles][4096] u16 and the bin values [chunks][tiles][4096] f64.
 struct ScatterLayout {
     int chunks = 1;
     long long span = 0;

@@ -282,8 +282,8 @@ int hk_rows_finish_many_f32(const hk_rows_job* jobs, int32_t count, int64_t rows
  * levels), every add a band add.  Scratch: hk_band_rows_finish_scratch_bytes(rows).
  *
  * hk_band_ordered_sum_f64: the fixed-tree ordered sum with band
- * accumulators (65536 virtual lanes add their rows as terms, the group and
- * final trees add bands).  Scratch: hk_band_ordered_sum_scratch_bytes(), no
+ * accumulators (8192 virtual lanes, 128 a group, add their rows as terms, the
+ * group and final trees add bands).  Scratch: hk_band_ordered_sum_scratch_bytes(), no
  * initial contents needed. */
 size_t hk_band_rows_finish_scratch_bytes(int64_t rows);
 int hk_band_rows_finish_f64(const double* hi, const double* lo, int64_t rows,
@@ -305,7 +305,7 @@ int hk_band_ordered_sum_f64(const double* u, int64_t n, double* out, void* scrat
  * contents needed: the per-(chunk, cell) partials, then the bins that carry
  * each tile's lanes from the first walk to the second (for 12288 < cells <=
  * 65536 in many chunks, the lanes of keys past the first 12288; for few chunks
- * or more cells, all of them; otherwise none). */
+ * or more cells, all of them, a pass of 289792 cells at a time; otherwise none). */
 int hk_scatter_chunks(int64_t n, int64_t cells);
 size_t hk_ordered_scatter_scratch_bytes(int64_t n, int64_t cells);
 int hk_ordered_scatter_f64(const int32_t* key, const double* v, int64_t n,
