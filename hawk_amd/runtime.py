@@ -836,6 +836,8 @@ class DeviceKernel:
         stages) over every sample with no per-call validation: the stable-binding
         path of reference ``tests/cards/CARD_LAUNCH_CROSSINGS.md`` (one crossing
         per launch).  The planes must stay alive and unmoved while it is used.
+        Launchers of one stream share scratch per sample count: graphs that
+        captured them are replayed one after another.
         ``steps`` / ``entry`` / ``chunk`` are :func:`run`'s; a prepared
         automatic kernel holds its own trip-count word, and its reports and
         finish count add up over calls."""

@@ -611,6 +611,62 @@ def test_two_streams_of_one_kernel(tmp_path, gpu):
                 assert torch.equal(p[name], w[name]), (way, name)
 
 
+def test_captured_calls_keep_their_scratch(tmp_path, gpu):
+    """A graph of a launcher and one of hawk.run on the same stream, replayed
+    with other inputs between eager runs of larger and smaller sizes there: the
+    eager results, every time."""
+    import hawk_amd as hawk
+    import torch
+    from hawk_amd import Index, Mutable, Scalar
+
+    @hawk.kernel
+    def all_of(x: Scalar, key: Index, a: Mutable[Scalar], b: Mutable[Scalar], o: Mutable[Scalar],
+               bins: Mutable[Scalar]):
+        a = hawk.sum(x * x)
+        b = hawk.max(x)
+        o = hawk.sum(x * 2.0, policy="ordered")
+        hawk.scatter(bins, policy="ordered")[key] += x * 3.0
+    (k,) = _unit(tmp_path, [all_of])
+
+    def planes(n, seed):
+        g = torch.Generator(device=gpu).manual_seed(seed)
+        return dict(x=torch.randn(n, dtype=torch.float64, device=gpu, generator=g),
+                    key=torch.randint(0, 20_000, (n,), dtype=torch.int32, device=gpu, generator=g),
+                    bins=torch.zeros(20_000, dtype=torch.float64, device=gpu),
+                    **{c: torch.zeros(1, dtype=torch.float64, device=gpu) for c in "abo"})
+    n = 50_001
+    inputs = [planes(n, seed) for seed in range(3)]
+    want = []
+    for p in inputs:
+        hawk.run(k, **p)
+        want.append({name: x.clone() for name, x in p.items()})
+    p = planes(n, 9)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    launch = k.prepare(stream=side, **p)
+    graphs = []
+    for call in (launch, lambda: hawk.run(k, check=False, **p)):
+        with torch.cuda.stream(side):
+            call()
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            call()
+        graphs.append(graph)
+    for turn, other in enumerate((1_000, 400_003, 100, 900_001)):
+        for graph in graphs:
+            source, result = inputs[turn % 3], want[turn % 3]
+            with torch.cuda.stream(side):
+                hawk.run(k, check=False, **planes(other, turn))
+                for name in ("x", "key"):
+                    p[name].copy_(source[name])
+                p["bins"].zero_()
+                graph.replay()
+            side.synchronize()
+            for name in p:
+                assert torch.equal(p[name], result[name]), (turn, name)
+
+
 def test_work_beside_a_launch_is_on_its_stream(gpu):
     """Resets, fills and allocations go to the launch's stream, the default
     stream inside another one's context included."""
