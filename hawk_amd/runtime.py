@@ -629,6 +629,13 @@ class DeviceKernel:
                              _core.rows_finish_many_scratch_bytes(rows, len(jobs)))
         return jobs, rows, self.planes[ops[0]["hi"]]["dtype"] == "f32", scratch.data_ptr()
 
+    def _keyed_scratch(self, t: dict, n: int, work: _Workspace):
+        """A keyed ordered sum's scratch: of one key the plain sum's (zero before
+        its first call), of more no contents needed."""
+        one = t["group"] == n
+        return work.bytes(("sum" if one else "keyed", t["out"], n),
+                          _core.keyed_ordered_sum_scratch_bytes(n, t["group"]), zero=one)
+
     def _row_identities(self, ops: list, bound: dict, stream: int) -> None:
         """A run of no samples leaves each reduction's identity: 0, -inf (max),
         +inf (min)."""
@@ -810,8 +817,7 @@ class DeviceKernel:
                 _core.band_ordered_sum(u.data_ptr(), n, self._cell_ptr(t, bound[t["out"]]), scratch.data_ptr(),
                                        stream)
             elif t["op"] == "keyed_sum":
-                scratch = work.bytes(("keyed", t["out"], n), _core.keyed_ordered_sum_scratch_bytes(n, t["group"]),
-                                     zero=t["group"] == n)
+                scratch = self._keyed_scratch(t, n, work)
                 fn = _core.keyed_ordered_sum_f32 if self._is_f32(t["out"]) else _core.keyed_ordered_sum
                 fn(bound[t["u"]].data_ptr(), n, t["group"], bound[t["out"]].data_ptr(), scratch.data_ptr(), stream)
             elif t["op"] == "ordered_fold":
@@ -1177,9 +1183,7 @@ class Prepared:
                 args = (bound[t["u"]].data_ptr(), self.n, kernel._cell_ptr(t, bound[t["out"]]), scratch.data_ptr())
                 self.steps.append((_core.band_ordered_sum, args))
             elif t["op"] == "keyed_sum":
-                scratch = work.bytes(("keyed", t["out"], self.n),
-                                     _core.keyed_ordered_sum_scratch_bytes(self.n, t["group"]),
-                                     zero=t["group"] == self.n)
+                scratch = kernel._keyed_scratch(t, self.n, work)
                 args = (bound[t["u"]].data_ptr(), self.n, t["group"], bound[t["out"]].data_ptr(), scratch.data_ptr())
                 self.steps.append((_core.keyed_ordered_sum_f32 if kernel._is_f32(t["out"]) else _core.keyed_ordered_sum,
                                    args))
